@@ -18,7 +18,7 @@
 // adjoint, the walker sums and the mean adjoints, and the weight-gradient
 // contraction X^T dY over walker rows (FP32 MFMA, deterministic slices).
 
-#include "kernels.h"
+#include "grad.h"
 
 namespace {
 
@@ -257,77 +257,155 @@ __global__ void pair_dx_kernel(long npairs, int fin, int fout, const float* __re
 
 // Weight-gradient contraction over rows on FP32 MFMA (v_mfma_f32_16x16x4f32):
 //   P[s][k][n] = sum_{r in slice s} X[r][k] dY[r][n]   (k < Kx, n < Ny)
-// X null: a column of ones (k = 0 only: column sums, the bias gradients).
+//   P[s][Kx][n] = sum_{r in slice s} dY[r][n]          (BIAS)
 // The A operand of a 16x16x4 step is X^T (row m = feature k, inner = row r),
 // the B operand dY: lane l reads X[r0 + l/16][k0 + l%16] and dY[r0 + l/16][n0 +
 // l%16], 64-byte row segments per lane group, no LDS staging.  A workgroup
 // (4 waves) owns a 64 x 64 output tile of one slice; the waves take every
-// fourth group of 4 rows and their partial tiles are summed through LDS.
+// fourth group of 4 rows, the next group's operands in flight while one is
+// multiplied, and their partial tiles are summed through LDS.  The column sums
+// are the operands of the first row of tiles, added in registers.
+// One launch serves a dense layer: its kernel (Q, K and V side by side), its
+// bias and, in FermiNet, both parts of its input; the slices are summed for
+// many layers at once (grad.h).  MFMA-bound in the large ones: 10752 rows x 256
+// x 768 in 68 us against 27 at the FP32 rate.  42 electrons, 256 walkers: 69
+// launches of 21.9 us and as many slice sums of 29.7 became 36 of 29 and 6 of
+// 16 us (the whole gradient 7.76 -> 5.26 ms; 14 electrons, 1024 walkers 4.08 ->
+// 2.99 ms).
 constexpr int WG_T = 4;  // 16x16 blocks per wave tile side
 
-__global__ __launch_bounds__(256) void wgrad_kernel(long rows, long rows_per_slice, const float* __restrict__ X,
-                                                    long ldx, int Kx, const float* __restrict__ dY, long ldy, int Ny,
-                                                    float* __restrict__ P) {
-  __shared__ float red[64 * 65];
+template <bool HASX>
+__global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a, long rows_per_slice, float* __restrict__ P) {
+  __shared__ float red[HASX ? 64 * 65 : 1];
+  __shared__ float csum[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lg = lane >> 4;
   const int k0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
   const long r_beg = (long)blockIdx.z * rows_per_slice;
-  const long r_end = r_beg + rows_per_slice < rows ? r_beg + rows_per_slice : rows;
+  const long r_end = r_beg + rows_per_slice < a.rows ? r_beg + rows_per_slice : a.rows;
+  const float* const __restrict__ X = a.X;
+  const float* const __restrict__ dY = a.dY;
   f32x4 acc[WG_T][WG_T];
+  float cs[WG_T];
 #pragma unroll
-  for (int a = 0; a < WG_T; ++a)
+  for (int i = 0; i < WG_T; ++i) {
+    cs[i] = 0.f;
 #pragma unroll
-    for (int b = 0; b < WG_T; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long r0 = r_beg + 4 * wave; r0 < r_end; r0 += 16) {
-    const long r = r0 + lg;
+    for (int j = 0; j < WG_T; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  bool kin[WG_T], nin[WG_T];
+#pragma unroll
+  for (int i = 0; i < WG_T; ++i) {
+    kin[i] = HASX && k0 + i * 16 + lr < a.Kx;
+    nin[i] = n0 + i * 16 + lr < a.Ny;
+  }
+  // the lane's row: number r of the contraction, row `row` of the operands
+  long r = r_beg + 4 * wave + lg;
+  long row = r;
+  int in_group = 0;
+  if (a.rgrp > 0) {
+    in_group = (int)(r % a.rgrp);
+    row = r / a.rgrp * a.rstride + in_group;
+  }
+  auto load = [&](float (&av)[WG_T], float (&bv)[WG_T]) __attribute__((always_inline)) {
     const bool rok = r < r_end;
-    float av[WG_T], bv[WG_T];
 #pragma unroll
-    for (int a = 0; a < WG_T; ++a) {
-      const int k = k0 + a * 16 + lr;
-      av[a] = (rok && k < Kx) ? (X ? X[r * ldx + k] : (k == 0 ? 1.f : 0.f)) : 0.f;
-      const int n = n0 + a * 16 + lr;
-      bv[a] = (rok && n < Ny) ? dY[r * ldy + n] : 0.f;
+    for (int i = 0; i < WG_T; ++i) {
+      if (HASX) av[i] = rok && kin[i] ? X[row * a.ldx + k0 + i * 16 + lr] : 0.f;
+      bv[i] = rok && nin[i] ? dY[row * a.ldy + n0 + i * 16 + lr] : 0.f;
+    }
+    r += 16;
+    if (a.rgrp > 0) {
+      in_group += 16;
+      row += 16;
+      while (in_group >= a.rgrp) {
+        in_group -= a.rgrp;
+        row += a.rstride - a.rgrp;
+      }
+    } else {
+      row += 16;
+    }
+  };
+  float av[WG_T], bv[WG_T];
+  load(av, bv);
+  for (long r0 = r_beg + 4 * wave; r0 < r_end; r0 += 16) {
+    float an[WG_T], bn[WG_T];
+    load(an, bn);
+#pragma unroll
+    for (int j = 0; j < WG_T; ++j) cs[j] += bv[j];
+    if constexpr (HASX) {
+#pragma unroll
+      for (int i = 0; i < WG_T; ++i)
+#pragma unroll
+        for (int j = 0; j < WG_T; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
     }
 #pragma unroll
-    for (int a = 0; a < WG_T; ++a)
-#pragma unroll
-      for (int b = 0; b < WG_T; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+    for (int i = 0; i < WG_T; ++i) {
+      av[i] = an[i];
+      bv[i] = bn[i];
+    }
   }
-  // acc[a][b][v]: output row k0 + a*16 + 4*lg + v, column n0 + b*16 + lr
-  for (int src = 0; src < 4; ++src) {
-    if (wave == src) {
+  const int nrow = a.Kx + (a.bias ? 1 : 0);
+  float* Ps = P + (long)blockIdx.z * nrow * a.Ny;
+  if (a.bias && blockIdx.x == 0) {
 #pragma unroll
-      for (int a = 0; a < WG_T; ++a)
-#pragma unroll
-        for (int b = 0; b < WG_T; ++b)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            float* t = &red[(a * 16 + 4 * lg + v) * 65 + b * 16 + lr];
-            *t = (src == 0 ? 0.f : *t) + acc[a][b][v];
-          }
+    for (int j = 0; j < WG_T; ++j) {
+      float t = cs[j] + __shfl_xor(cs[j], 16);
+      t += __shfl_xor(t, 32);
+      if (lg == 0) csum[wave][j * 16 + lr] = t;
     }
     __syncthreads();
+    const int n = threadIdx.x;
+    if (n < 64 && n0 + n < a.Ny)
+      Ps[(long)a.Kx * a.Ny + n0 + n] = (csum[0][n] + csum[1][n]) + (csum[2][n] + csum[3][n]);
   }
-  float* Ps = P + (long)blockIdx.z * Kx * Ny;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int kk = e / 64, nn = e % 64;
-    if (k0 + kk < Kx && n0 + nn < Ny) Ps[(long)(k0 + kk) * Ny + n0 + nn] = red[kk * 65 + nn];
+  if constexpr (HASX) {
+    // acc[i][j][v]: output row k0 + i*16 + 4*lg + v, column n0 + j*16 + lr
+    for (int src = 0; src < 4; ++src) {
+      if (wave == src) {
+#pragma unroll
+        for (int i = 0; i < WG_T; ++i)
+#pragma unroll
+          for (int j = 0; j < WG_T; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              float* t = &red[(i * 16 + 4 * lg + v) * 65 + j * 16 + lr];
+              *t = (src == 0 ? 0.f : *t) + acc[i][j][v];
+            }
+      }
+      __syncthreads();
+    }
+    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
+      const int kk = e / 64, nn = e % 64;
+      if (k0 + kk < a.Kx && n0 + nn < a.Ny) Ps[(long)(k0 + kk) * a.Ny + n0 + nn] = red[kk * 65 + nn];
+    }
   }
 }
 
-// acc[off + (row0 + k) * ld + n] += sum_s P[s][k][n]   (FP64, fixed slice order)
-__global__ void slice_sum_kernel(const float* __restrict__ P, int ns, int Kx, int Ny, double* __restrict__ acc,
-                                 long off, int row0, int ld) {
-  const long tot = (long)Kx * Ny;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int z = 0; z < ns; ++z) s += P[(long)z * tot + e];
-    const int k = (int)(e / Ny), n = (int)(e % Ny);
-    acc[off + (long)(row0 + k) * ld + n] += s;
+// acc[place of (k, n)] += sum_s P[s][k][n] of every waiting contraction (FP64,
+// fixed slice order), one thread per entry.
+__global__ __launch_bounds__(256) void slice_sum_kernel(SliceJobs jobs, double* __restrict__ acc) {
+  int q = 0;
+  while (q + 1 < jobs.n && (int)blockIdx.x >= jobs.first[q + 1]) ++q;
+  const SliceJob& j = jobs.j[q];
+  const int tot = j.nrow * j.Ny;
+  const int e = ((int)blockIdx.x - jobs.first[q]) * 256 + threadIdx.x;
+  if (e >= tot) return;
+  const float* __restrict__ P = j.P + e;
+  double s = 0.0;
+  int z = 0;
+  for (; z + 8 <= j.ns; z += 8) {  // eight slices in flight, added in order
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = P[(long)(z + u) * tot];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += t[u];
   }
+  for (; z < j.ns; ++z) s += P[(long)z * tot];
+  const int k = e / j.Ny, n = e % j.Ny;
+  const long col = (long)(n / j.seg) * j.segstride + n % j.seg;
+  acc[k == j.Kx ? j.boff + col : j.off + (long)(k < j.ksplit ? k : k + j.kskip) * j.ld + col] += s;
 }
 
 __global__ void fill_f64_kernel(double* p, long n, double v) {
@@ -398,29 +476,48 @@ int launch_pair_dx(long npairs, int fin, int fout, const float* dz2, const float
   return 0;
 }
 
-// P needs nslices * Kx * Ny floats; returns the slice count used.
-int wgrad_slices(long rows, int Kx, int Ny, long pcap) {
-  const long tiles = (long)((Kx + 63) / 64) * ((Ny + 63) / 64);
-  long ns = 1024 / (tiles > 0 ? tiles : 1);
+// Slices of a contraction: about 1024 workgroups (four per CU, what the 64 x 64
+// tiles' registers allow) of at least 64 rows each.
+static int wgrad_slices(const WgradArgs& a, long cap) {
+  const long tiles = (long)(a.Kx > 0 ? (a.Kx + 63) / 64 : 1) * ((a.Ny + 63) / 64);
+  long ns = 1024 / tiles;
   ns = ns < 1 ? 1 : (ns > 256 ? 256 : ns);
-  const long by_rows = (rows + 63) / 64;
+  const long by_rows = (a.rows + 63) / 64;
   if (ns > by_rows) ns = by_rows > 0 ? by_rows : 1;
-  while (ns > 1 && ns * Kx * Ny > pcap) ns >>= 1;
+  while (ns > 1 && ns * (a.Kx + 1) * a.Ny > cap) ns >>= 1;
   return (int)ns;
 }
 
-int launch_wgrad(long rows, const float* X, long ldx, int Kx, const float* dY, long ldy, int Ny, float* P, long pcap,
-                 double* acc, long off, int row0, int ld, hipStream_t s) {
-  if (rows <= 0 || Kx <= 0 || Ny <= 0) return 0;
-  const int ns = wgrad_slices(rows, Kx, Ny, pcap);
-  if ((long)ns * Kx * Ny > pcap) return -1;
-  long rps = (rows + ns - 1) / ns;
+int WgradQueue::add(const WgradArgs& a) {
+  if (a.rows <= 0 || a.Ny <= 0 || (a.Kx <= 0 && !a.bias)) return 0;
+  const int ns = wgrad_slices(a, cap_);
+  const int nrow = a.Kx + (a.bias ? 1 : 0);
+  const long need = (long)ns * nrow * a.Ny;
+  if (need > cap_ || (long)nrow * a.Ny > 0x7FFFFFFFL) return -1;
+  bool wait = jobs_.n == kSliceJobs || used_ + need > cap_;
+  for (int i = 0; i < jobs_.n; ++i) wait = wait || jobs_.j[i].off == a.off || (a.bias && jobs_.j[i].boff == a.boff);
+  if (wait) flush();
+  long rps = (a.rows + ns - 1) / ns;
   rps = (rps + 3) / 4 * 4;
-  const dim3 grid((Kx + 63) / 64, (Ny + 63) / 64, ns);
-  hipLaunchKernelGGL(wgrad_kernel, grid, dim3(256), 0, s, rows, rps, X, ldx, Kx, dY, ldy, Ny, P);
-  hipLaunchKernelGGL(slice_sum_kernel, dim3(grid_of((long)Kx * Ny)), dim3(256), 0, s, P, ns, Kx, Ny, acc, off, row0,
-                     ld);
+  float* P = P_ + used_;
+  const dim3 grid(a.Kx > 0 ? (a.Kx + 63) / 64 : 1, (a.Ny + 63) / 64, ns);
+  if (a.Kx > 0)
+    hipLaunchKernelGGL(wgrad_kernel<true>, grid, dim3(256), 0, s_, a, rps, P);
+  else
+    hipLaunchKernelGGL(wgrad_kernel<false>, grid, dim3(256), 0, s_, a, rps, P);
+  used_ += need;
+  if (jobs_.n == 0) jobs_.first[0] = 0;
+  jobs_.j[jobs_.n] = SliceJob{P, ns, nrow, a.Ny, a.ld, a.ksplit, a.kskip, a.seg, a.Kx, a.off, a.boff, a.segstride};
+  jobs_.first[jobs_.n + 1] = jobs_.first[jobs_.n] + ceil_div((long)nrow * a.Ny, 256);
+  ++jobs_.n;
   return 0;
+}
+
+void WgradQueue::flush() {
+  if (jobs_.n > 0)
+    hipLaunchKernelGGL(slice_sum_kernel, dim3(jobs_.first[jobs_.n]), dim3(256), 0, s_, jobs_, acc_);
+  jobs_.n = 0;
+  used_ = 0;
 }
 
 int launch_fill_f64(double* p, long n, double v, hipStream_t s) {

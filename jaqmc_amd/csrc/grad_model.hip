@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "grad.h"
 #include "model.h"
 #include "prof.h"
 
@@ -21,8 +22,6 @@ int launch_one_adj(const FermiDims& d, int f1, const float* dX, long lddx, const
 int launch_pair_adj(const FermiDims& d, int f2, const float* dX, long lddx, int col0, float* dh2, hipStream_t s);
 int launch_pair_dx(long npairs, int fin, int fout, const float* dz2, const float* W2, int res, const float* dh2new,
                    float* dh2old, hipStream_t s);
-int launch_wgrad(long rows, const float* X, long ldx, int Kx, const float* dY, long ldy, int Ny, float* P, long pcap,
-                 double* acc, long off, int row0, int ld, hipStream_t s);
 int launch_fill_f64(double* p, long n, double v, hipStream_t s);
 int launch_fill_f32(float* p, long n, float v, hipStream_t s);
 int launch_f64_to_f32(const double* a, long n, float* out, hipStream_t s);
@@ -168,6 +167,7 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
     return 0;
   }
   const long KN = (long)K * N;
+  WgradQueue wq(Pw, pw_cap, gacc, s);
   for (int b0 = 0; b0 < B; b0 += gchunk) {
     const int Bc = std::min(gchunk, B - b0);
     const float* ec = elec + (long)b0 * T;
@@ -187,8 +187,8 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
       const long u0 = (nch == 1 || c == 0) ? 0 : (long)Bc * n_up;
       const long nu = nch == 1 ? (long)Bc * N : (c == 0 ? (long)Bc * n_up : (long)Bc * n_dn);
       const int set = norb == 2 ? c : 0;
-      rc = launch_wgrad(nu, (const float*)Xt[L] + u0 * korb, korb, dL, dPhi + u0 * ldko, ldko, (int)KN, Pw, pw_cap,
-                        gacc, off_orb[set], 0, (int)KN, s);
+      rc = wq.add(wgrad_args(nu, (const float*)Xt[L] + u0 * korb, korb, dL, dPhi + u0 * ldko, ldko, (int)KN,
+                             off_orb[set], false, -1));
       rc |= gemm_nt(dPhi + u0 * ldko, ldko, Worb_o[set], (int)ldko, dL, dh + u0 * ldd, ldd, nu, s);
       if (rc) return jq_fail(JQ_EINVAL, "orbital adjoint launch rejected");
     }
@@ -203,8 +203,7 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
       if (ly.has_pair) {
         launch_tanh_bwd(npairs, ly.d2, H2t[l + 1], ly.d2, H2t[l], ly.f2, dh2n, ly.d2, ly.res2, dZ2, ly.d2, nullptr, 0,
                         s);
-        rc = launch_wgrad(npairs, H2t[l], ly.f2, ly.f2, dZ2, ly.d2, ly.d2, Pw, pw_cap, gacc, ly.off_w2, 0, ly.d2, s);
-        rc |= launch_wgrad(npairs, nullptr, 0, 1, dZ2, ly.d2, ly.d2, Pw, pw_cap, gacc, ly.off_b2, 0, ly.d2, s);
+        rc = wq.add(wgrad_args(npairs, H2t[l], ly.f2, ly.f2, dZ2, ly.d2, ly.d2, ly.off_w2, true, ly.off_b2));
         if (rc) return jq_fail(JQ_EINVAL, "pair-stream adjoint launch rejected");
         if (l > 0) launch_pair_dx(npairs, ly.f2, ly.d2, dZ2, ly.W2, ly.res2, dh2n, dh2o, s);
       } else if (l > 0) {
@@ -215,15 +214,16 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
       if (l > 0 && !ly.res1) launch_fill_f32(dho, units * ldd, 0.f, s);
       launch_tanh_bwd(units, ly.d1, (const float*)Xt[l + 1], ldn, (const float*)Xt[l], ly.kmain, dh, ldd, ly.res1,
                       dZ, ldd, (l > 0 && ly.res1) ? dho : nullptr, ldd, s);
-      const int in_rows_h = ly.f1, g_row0 = ly.f1, p_row0 = ly.f1 * (1 + nch);
-      rc = launch_wgrad(units, (const float*)Xt[l], ly.kmain, in_rows_h, dZ, ldd, ly.d1, Pw, pw_cap, gacc, ly.off_w, 0,
-                        ly.d1, s);
-      rc |= launch_wgrad(units, (const float*)Xt[l] + ly.f1, ly.kmain, nch * ly.f2, dZ, ldd, ly.d1, Pw, pw_cap, gacc,
-                         ly.off_w, p_row0, ly.d1, s);
-      rc |= launch_wgrad(units, nullptr, 0, 1, dZ, ldd, ly.d1, Pw, pw_cap, gacc, ly.off_b, 0, ly.d1, s);
+      // kernel rows [h (f1) | spin means (nch f1) | pair means (nch f2)]: the
+      // layer input [h | pair means] leaves the rows of the means out
+      WgradArgs wm = wgrad_args(units, (const float*)Xt[l], ly.kmain, ly.f1 + nch * ly.f2, dZ, ldd, ly.d1, ly.off_w,
+                                true, ly.off_b);
+      wm.ksplit = ly.f1;
+      wm.kskip = nch * ly.f1;
+      rc = wq.add(wm);
       launch_walker_sum(fd, dZ, ldd, ly.d1, dG, ly.d1, s);
-      rc |= launch_wgrad(Bc, (const float*)gt[l], ly.kg, nch * ly.f1, dG, ly.d1, ly.d1, Pw, pw_cap, gacc, ly.off_w,
-                         g_row0, ly.d1, s);
+      rc |= wq.add(wgrad_args(Bc, (const float*)gt[l], ly.kg, nch * ly.f1, dG, ly.d1, ly.d1,
+                              ly.off_w + (long)ly.f1 * ly.d1, false, -1));
       if (rc) return jq_fail(JQ_EINVAL, "layer adjoint launch rejected");
       if (l > 0) {
         // adjoints of h_l (spin means and the layer input) and of h2_l (pair means)
@@ -237,6 +237,7 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
       }
     }
   }
+  wq.flush();
   launch_f64_to_f32(gacc, n_params, grad, s);
   return 0;
 }
@@ -260,8 +261,6 @@ int launch_attn_bwd(const float* QKV, const float* dO, long lddo, float* dQKV, l
                     hipStream_t st);
 int launch_jastrow_grad(const float* elec, int Bc, int N, int n_up, float ap, float aa, const double* cot, int b0,
                         float* out, hipStream_t st);
-int launch_mask_rows(long units, int N, int i0, int i1, int ncols, const float* src, long lds, float* dst, long ldd,
-                     hipStream_t st);
 int launch_add_rows(long rows, int n, const float* a, long lda, const float* b, long ldb, float* out, long ldo,
                     hipStream_t st);
 int launch_scale_f64(double* p, long n, double v, hipStream_t st);
@@ -277,7 +276,7 @@ int jq_model::alloc_grad_workspace_psi(size_t budget) {
       wmax = std::max(wmax, (long)round_up(ly.mdims[j], 32));
     }
   }
-  const long back = 2L * D + 2L * wmax + wmax + D + 3L * D + D + D + 2L * ldko + KN;
+  const long back = 2L * D + 2L * wmax + wmax + D + 3L * D + D + D + ldko + KN;
   const size_t per_walker = 4 * (size_t)N * (tape + back) + 64;
   gchunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)chunk_fwd, budget / per_walker));
   const size_t U = (size_t)gchunk * N;
@@ -320,13 +319,12 @@ int jq_model::alloc_grad_workspace_psi(size_t budget) {
   dXin = fa(U * D);
   Pln = fa(U * D);
   dPhi = fa(U * ldko);
-  dPhiM = fa(U * ldko);
   dEnv = fa(U * KN);
   jtmp = fa(2 * (size_t)gchunk);
   pw_cap = 16l << 20;
   Pw = fa(pw_cap);
   gacc = (double*)alloc((size_t)n_params * 8);
-  if (!ok || !dH[0] || !dH1 || !dM[0] || !dM[1] || !dZ || !dO || !dQKV || !dXin || !Pln || !dPhi || !dPhiM ||
+  if (!ok || !dH[0] || !dH1 || !dM[0] || !dM[1] || !dZ || !dO || !dQKV || !dXin || !Pln || !dPhi ||
       !dEnv || !jtmp || !Pw || !gacc)
     return jq_fail(JQ_ENOMEM, "gradient workspace allocation failed");
   // padding columns of dPhi (KN .. ldko) are read by the orbital adjoint GEMM
@@ -451,8 +449,13 @@ static int gemm_nt_groups(const float* Xp, long ldx, const float* W, int K_, int
 int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStream_t s) {
   const long KN = (long)K * N;
   const bool pre = ln_mode == JQ_LN_PRE, post = ln_mode == JQ_LN_POST;
-  auto wg = [&](long rows, const float* X, long ldx, int Kx, const float* dY, long ldy, int Ny, long off) {
-    return launch_wgrad(rows, X, ldx, Kx, dY, ldy, Ny, Pw, pw_cap, gacc, off, 0, Ny, s);
+  WgradQueue wq(Pw, pw_cap, gacc, s);
+  // a dense layer's kernel and bias gradients; column sums only
+  auto wg = [&](long rows, const float* X, long ldx, int Kx, const float* dY, long ldy, int Ny, long off, long boff) {
+    return wq.add(wgrad_args(rows, X, ldx, Kx, dY, ldy, Ny, off, true, boff));
+  };
+  auto colsum = [&](long rows, const float* dY, long ldy, int Ny, long off) {
+    return wq.add(wgrad_args(rows, nullptr, 0, 0, dY, ldy, Ny, -1 - off, true, off));
   };
   for (int b0 = 0; b0 < B; b0 += gchunk) {
     const int Bc = std::min(gchunk, B - b0);
@@ -472,13 +475,11 @@ int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStre
     for (int c = 0; c < nch; ++c) {
       const int set = norb == 2 ? c : 0;
       const int i0 = (nch == 1 || c == 0) ? 0 : n_up, ns = nch == 1 ? N : (c == 0 ? n_up : n_dn);
-      const float* dP = dPhi;
-      if (nch == 2) {
-        launch_mask_rows(units, N, i0, i0 + ns, (int)ldko, dPhi, ldko, dPhiM, ldko, s);
-        dP = dPhiM;
-      }
-      rc = wg(units, Ht[L], D, D, dP, ldko, (int)KN, off_orb[set]);
-      if (borb[c]) rc |= wg(units, nullptr, 0, 1, dP, ldko, (int)KN, off_borb[set]);
+      WgradArgs wo = wgrad_args((long)Bc * ns, Ht[L] + (long)i0 * D, D, D, dPhi + (long)i0 * ldko, ldko, (int)KN,
+                                off_orb[set], borb[c] != nullptr, off_borb[set]);
+      wo.rgrp = ns;
+      wo.rstride = N;
+      rc = wq.add(wo);
       rc |= gemm_nt_groups(dPhi + (long)i0 * ldko, ldko, Worb_o[set], (int)ldko, D, gH + (long)i0 * D, D,
                            (long)Bc * ns, ns, (long)N * ldko, (long)N * D, s);
       if (rc) return jq_fail(JQ_EINVAL, "orbital adjoint launch rejected");
@@ -488,8 +489,8 @@ int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStre
       if (post) {  // H' = LN2(U2): the adjoint of U2 (= that of m) into dH1
         if (launch_ln_bwd(units, D, U2t[l], D, ly.ln2_s, gH, D, 1e-5f, nullptr, 0, dH1, D, Pln, D, s))
           return jq_fail(JQ_EINVAL, "LayerNorm adjoint supports D <= 512");
-        rc = wg(units, nullptr, 0, 1, Pln, D, D, ly.off_ln2s);
-        rc |= wg(units, nullptr, 0, 1, gH, D, D, ly.off_ln2b);
+        rc = colsum(units, Pln, D, D, ly.off_ln2s);
+        rc |= colsum(units, gH, D, D, ly.off_ln2b);
       }
       // MLP: dm starts as the adjoint of the MLP output (H' = H1 + m, or U2)
       const int nm = (int)ly.Wm.size();
@@ -502,8 +503,7 @@ int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStre
         launch_tanh_bwd(units, outw, MHt[l][j], outp, nullptr, 0, dm, lddm, 0, dZ, outp, nullptr, 0, s);
         const float* xin = j == 0 ? M0t[l] : MHt[l][j - 1];
         const long ldxin = j == 0 ? D : round_up(inw, 32);
-        rc = wg(units, xin, ldxin, inw, dZ, outp, outw, ly.off_mw[j]);
-        rc |= wg(units, nullptr, 0, 1, dZ, outp, outw, ly.off_mb[j]);
+        rc = wg(units, xin, ldxin, inw, dZ, outp, outw, ly.off_mw[j], ly.off_mb[j]);
         const long ldn = round_up(inw, 32);
         rc |= gemm_nt(dZ, outp, ly.Wm_o[j], outp, inw, dM[mi], ldn, units, s);
         dm = dM[mi];
@@ -516,49 +516,48 @@ int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStre
       if (post) {
         launch_add_rows(units, D, dH1, D, dm, lddm, gH, D, s);
         launch_ln_bwd(units, D, U1t[l], D, ly.ln1_s, gH, D, 1e-5f, nullptr, 0, dH1, D, Pln, D, s);
-        rc = wg(units, nullptr, 0, 1, Pln, D, D, ly.off_ln1s);
-        rc |= wg(units, nullptr, 0, 1, gH, D, D, ly.off_ln1b);
+        rc = colsum(units, Pln, D, D, ly.off_ln1s);
+        rc |= colsum(units, gH, D, D, ly.off_ln1b);
       } else if (pre) {
         if (launch_ln_bwd(units, D, H1t[l], D, ly.ln2_s, dm, lddm, 1e-5f, gH, D, dH1, D, Pln, D, s))
           return jq_fail(JQ_EINVAL, "LayerNorm adjoint supports D <= 512");
-        rc = wg(units, nullptr, 0, 1, Pln, D, D, ly.off_ln2s);
-        rc |= wg(units, nullptr, 0, 1, dm, lddm, D, ly.off_ln2b);
+        rc = colsum(units, Pln, D, D, ly.off_ln2s);
+        rc |= colsum(units, dm, lddm, D, ly.off_ln2b);
       } else {
         launch_add_rows(units, D, gH, D, dm, lddm, dH1, D, s);
       }
       // attention output projection and the attention itself
-      rc |= wg(units, Ot[l], D, D, dH1, D, D, ly.off_wo);
-      rc |= wg(units, nullptr, 0, 1, dH1, D, D, ly.off_bo);
+      rc |= wg(units, Ot[l], D, D, dH1, D, D, ly.off_wo, ly.off_bo);
       rc |= gemm_nt(dH1, D, ly.Wo_o, D, D, dO, D, units, s);
       if (rc) return jq_fail(JQ_EINVAL, "attention projection adjoint launch rejected");
       if (launch_attn_bwd(QKVt[l], dO, D, dQKV, 3L * D, Bc, N, H, dh, s))
         return jq_fail(JQ_EINVAL, "attention adjoint supports N <= 64 and heads_dim <= 64");
-      const long offw[3] = {ly.off_wq, ly.off_wk, ly.off_wv}, offb[3] = {ly.off_bq, ly.off_bk, ly.off_bv};
-      for (int p = 0; p < 3; ++p) {
-        rc |= wg(units, XINt[l], D, D, dQKV + (long)p * D, 3L * D, D, offw[p]);
-        rc |= wg(units, nullptr, 0, 1, dQKV + (long)p * D, 3L * D, D, offb[p]);
-      }
+      // q, k, v kernels and biases are D (D + 1) entries apart in the pack
+      WgradArgs wa = wgrad_args(units, XINt[l], D, D, dQKV, 3L * D, 3 * D, ly.off_wq, true, ly.off_bq);
+      wa.ld = wa.seg = D;
+      wa.segstride = ly.off_wk - ly.off_wq;
+      rc |= wq.add(wa);
       rc |= gemm_nt(dQKV, 3L * D, ly.Wqkv_o, 3 * D, D, dXin, D, units, s);
       if (rc) return jq_fail(JQ_EINVAL, "attention input adjoint launch rejected");
       // LN1 (pre-LN): dH = dH1 + LN1'(dXin); otherwise (U1 = H + ..., XIN = H) dH = dH1 + dXin
       if (pre) {
         launch_ln_bwd(units, D, Ht[l], D, ly.ln1_s, dXin, D, 1e-5f, dH1, D, gH, D, Pln, D, s);
-        rc = wg(units, nullptr, 0, 1, Pln, D, D, ly.off_ln1s);
-        rc |= wg(units, nullptr, 0, 1, dXin, D, D, ly.off_ln1b);
+        rc = colsum(units, Pln, D, D, ly.off_ln1s);
+        rc |= colsum(units, dXin, D, D, ly.off_ln1b);
       } else {
         launch_add_rows(units, D, dH1, D, dXin, D, gH, D, s);
       }
     }
     if (rc) return jq_fail(JQ_EINVAL, "layer adjoint launch rejected");
     // input projection
-    rc = wg(units, F0t, kin, 4 * M + 1, gH, D, D, off_win);
-    rc |= wg(units, nullptr, 0, 1, gH, D, D, off_bin);
+    rc = wg(units, F0t, kin, 4 * M + 1, gH, D, D, off_win, off_bin);
     if (d.jastrow) {
       launch_jastrow_grad(ec, Bc, N, n_up, jas[0], jas[1], cot, b0, jtmp, s);
-      rc |= wg(Bc, nullptr, 0, 1, jtmp, 2, 2, off_jas);
+      rc |= colsum(Bc, jtmp, 2, 2, off_jas);
     }
     if (rc) return jq_fail(JQ_EINVAL, "input adjoint launch rejected");
   }
+  wq.flush();
   // the pack's q kernel and bias enter as 1/sqrt(dh) times the device's
   const double qs = 1.0 / std::sqrt((double)dh);
   for (const PsiLayer& ly : pl) {

@@ -161,18 +161,6 @@ __global__ void jastrow_grad_kernel(const float* __restrict__ elec, int Bc, int 
   out[2 * w + 1] = (float)(c * ga);
 }
 
-// dst[unit][n] = src[unit][n] for the electrons i0 <= i < i1 of every walker
-// (walker-major units), 0 for the others
-__global__ void mask_rows_kernel(long units, int N, int i0, int i1, int ncols, const float* __restrict__ src, long lds,
-                                 float* __restrict__ dst, long ldd) {
-  const long tot = units * ncols;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-    const long u = e / ncols;
-    const int n = (int)(e % ncols), i = (int)(u % N);
-    dst[u * ldd + n] = (i >= i0 && i < i1) ? src[u * lds + n] : 0.f;
-  }
-}
-
 // out[r][c] = a[r][c] + b[r][c]
 __global__ void add_rows_kernel(long rows, int n, const float* a, long lda, const float* b, long ldb, float* out,
                                 long ldo) {
@@ -226,13 +214,6 @@ int launch_jastrow_grad(const float* elec, int Bc, int N, int n_up, float ap, fl
   if (Bc <= 0) return 0;
   hipLaunchKernelGGL(jastrow_grad_kernel, dim3((unsigned)((Bc + 63) / 64)), dim3(64), 0, st, elec, Bc, N, n_up, ap, aa,
                      cot, b0, out);
-  return 0;
-}
-
-int launch_mask_rows(long units, int N, int i0, int i1, int ncols, const float* src, long lds, float* dst, long ldd,
-                     hipStream_t st) {
-  hipLaunchKernelGGL(mask_rows_kernel, dim3(grid_for(units * ncols)), dim3(256), 0, st, units, N, i0, i1, ncols, src,
-                     lds, dst, ldd);
   return 0;
 }
 

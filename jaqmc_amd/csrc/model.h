@@ -139,7 +139,7 @@ struct jq_model {
   std::vector<float*> Ht, XINt, QKVt, Ot, H1t, M0t, U1t, U2t;
   std::vector<std::vector<float*>> MHt;
   float *dH1 = nullptr, *dM[2] = {nullptr, nullptr}, *dO = nullptr, *dQKV = nullptr, *dXin = nullptr;
-  float *Pln = nullptr, *dPhiM = nullptr, *jtmp = nullptr;
+  float *Pln = nullptr, *jtmp = nullptr;
   int alloc_grad_workspace_psi(size_t tape_budget);
   int forward_psiformer_tape(const float* elec_chunk, int Bc, hipStream_t s);
   int vjp_psiformer(const float* elec, int B, const double* cot, hipStream_t s);

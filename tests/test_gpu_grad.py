@@ -271,3 +271,25 @@ def test_psiformer_vjp_at_the_ring42_shape(cuda):
           f"violations {int(bad.sum())} of {g.size}", flush=True)
     assert not bad.any()
     dm.close()
+
+
+# a batch whose rows (97 x 14, 97 x 4, 97 x 3) leave remainders in every slice,
+# group of rows and channel of the weight-gradient contractions
+@pytest.mark.parametrize("case", ["n2_small", "psi_pre", "psi_null_shared", "psi_polarized"])
+def test_vjp_ragged_batch(cuda, case):
+    """Six walkers repeated to a batch of 97 with positive weights: the float64
+    gradient of the six with their weights added up, to this file's tolerance."""
+    import torch
+
+    from jaqmc_amd.device import DeviceModel
+
+    print(f"[grad] ragged batch {case}", flush=True)
+    B = 97
+    sysm, spec, p, x = (_setup if case in CASES else _psi_setup)(case, 6)
+    dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, with_gradients=True)
+    cot = 0.5 + np.random.default_rng(B).random(B)
+    who = np.arange(B) % 6
+    g = dm.logpsi_vjp(torch.from_numpy(x[who]).to(cuda), torch.from_numpy(cot).to(cuda)).cpu().numpy()
+    ref = _torch_grad_unused(spec, p, x, sysm.atoms, np.bincount(who, cot))
+    dm.close()
+    assert np.all(np.abs(g - ref) <= 1e-4 * np.abs(ref).max() + 1e-3 * np.abs(ref))

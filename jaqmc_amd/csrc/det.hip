@@ -17,26 +17,10 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "gauss_jordan.h"
 #include "kernels.h"
 
 namespace {
-
-// log|prod_p v_p| over the pivots without one log per factor: the running
-// product is kept as a mantissa in [0.5, 1) and a binary exponent (both
-// factors split with frexp, so it neither overflows nor underflows), and one
-// log is taken at the end.  A zero pivot gives -inf, a NaN or inf pivot
-// propagates, as the sum of logs would.
-struct LogAbsProduct {
-  double m = 1.0;
-  int e = 0;
-  __device__ void mul(double v) {
-    int ev, em;
-    const double mv = frexp(fabs(v), &ev);
-    m = frexp(m * mv, &em);
-    e += ev + em;
-  }
-  __device__ double log_abs() const { return log(m) + (double)e * 0.69314718055994530942; }
-};
 
 // Orbital-matrix element (value, and optionally Jacobian row c or Laplacian).
 __device__ inline const float* env_ptr(const FermiDims& d, const float* env, int w, int i, int k, int o) {
@@ -114,15 +98,7 @@ __global__ __launch_bounds__(256, (NP <= 48 ? 2 : 1)) void det_mfma_kernel(Fermi
   }
   __syncthreads();
 
-  // ---- Gauss-Jordan on [A | I] with the matrix in registers ----
-  // Thread (ti, tj) = (tid % 16, tid / 16) owns rows i = ti + 16a and columns
-  // j = tj + 16b of the NP x 2NP augmented matrix.  No rows are exchanged:
-  // the pivot for column p is the unused row q with the largest |A[q][p]|
-  // (smallest q on ties), and at the end row p of A^-1 is row q of the right
-  // half.  Per pivot: the owners of column p (16 lanes of one DPP row) have
-  // already reduced their candidates to (q, A[q][p]); barrier; the owners of
-  // row q and of column p publish them; barrier; every thread updates its
-  // elements and the owners of column p + 1 reduce the next candidates.
+  // ---- Gauss-Jordan on [A | I] with the matrix in registers (gauss_jordan.h) ----
   constexpr int RA = NP / 16, CB = NP / 8;
   const int ti = tid & 15, tj = tid >> 4;
   double x[RA][CB];
@@ -134,99 +110,11 @@ __global__ __launch_bounds__(256, (NP <= 48 ? 2 : 1)) void det_mfma_kernel(Fermi
       x[a][b] = j < NP ? A[i * NP + j] : (i == j - NP ? 1.0 : 0.0);
     }
   __syncthreads();  // A is scratch from here on
-  double* prow = A;             // pivot row, 2NP
-  double* pcol = A + 2 * NP;    // pivot column, NP
-  double* cval = A + 3 * NP;    // signed pivot value
-  int* cidx = (int*)(A + 3 * NP + 1);
-  int* perm = (int*)(A + 3 * NP + 2);  // perm[p] = pivot row of column p
-  unsigned used = 0;
+  int* const perm = gj_wg_perm<NP>(A);
   int pos[RA];  // pivot index of the thread's rows
-  // candidates of a column held in x[.][b] by the 16 lanes of this DPP row
-  auto candidates = [&](int b) __attribute__((always_inline)) {
-    double v = -1.0, sv = 0.0;
-    int bi = NP;
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      const double y = fabs(x[a][b]);
-      if (!((used >> a) & 1u) && (bi == NP || y > v)) {  // any unused row, even a non-finite one
-        v = y;
-        sv = x[a][b];
-        bi = ti + 16 * a;
-      }
-    }
-    // lanes without an unused row (bi == NP) take any offered candidate, so
-    // the result is a valid unused row whenever one exists
-    auto pick = [&](double ov, double osv, int oi) __attribute__((always_inline)) {
-      if (oi != NP && (bi == NP || ov > v || (ov == v && oi < bi))) {
-        v = ov;
-        sv = osv;
-        bi = oi;
-      }
-    };
-    pick(dpp_d<0xB1>(v), dpp_d<0xB1>(sv), __builtin_amdgcn_mov_dpp(bi, 0xB1, 0xF, 0xF, false));
-    pick(dpp_d<0x4E>(v), dpp_d<0x4E>(sv), __builtin_amdgcn_mov_dpp(bi, 0x4E, 0xF, 0xF, false));
-    pick(dpp_d<0x141>(v), dpp_d<0x141>(sv), __builtin_amdgcn_mov_dpp(bi, 0x141, 0xF, 0xF, false));
-    pick(dpp_d<0x140>(v), dpp_d<0x140>(sv), __builtin_amdgcn_mov_dpp(bi, 0x140, 0xF, 0xF, false));
-    if (ti == 0) {
-      *cval = sv;
-      *cidx = bi;
-    }
-  };
-  if (tj == 0) candidates(0);
   LogAbsProduct logdet;
   int sgn = 1;
-#pragma unroll
-  for (int pb = 0; pb < RA; ++pb) {
-    for (int pr = 0; pr < 16; ++pr) {
-      const int p = 16 * pb + pr;
-      __syncthreads();
-      const int q = *cidx;
-      const double piv = *cval;
-      const double rp = 1.0 / piv;
-      if (tid == 0) {
-        logdet.mul(piv);
-        if (piv < 0) sgn = -sgn;
-        perm[p] = q;
-      }
-      if (ti == (q & 15)) {
-#pragma unroll
-        for (int a = 0; a < RA; ++a)
-          if (a == (q >> 4)) {
-#pragma unroll
-            for (int b = 0; b < CB; ++b) prow[tj + 16 * b] = x[a][b];
-          }
-      }
-      if (tj == pr) {
-#pragma unroll
-        for (int a = 0; a < RA; ++a) pcol[ti + 16 * a] = x[a][pb];
-      }
-      __syncthreads();
-      double r[CB];
-#pragma unroll
-      for (int b = 0; b < CB; ++b) r[b] = prow[tj + 16 * b] * rp;
-#pragma unroll
-      for (int a = 0; a < RA; ++a) {
-        const int i = ti + 16 * a;
-        if (i == q) {
-#pragma unroll
-          for (int b = 0; b < CB; ++b) x[a][b] = r[b];
-          used |= 1u << a;
-          pos[a] = p;
-        } else {
-          const double f = pcol[i];
-#pragma unroll
-          for (int b = 0; b < CB; ++b) x[a][b] -= f * r[b];
-        }
-      }
-      if (p + 1 < NP && tj == ((p + 1) & 15)) {
-        if (pr == 15) {
-          candidates(pb + 1 < RA ? pb + 1 : pb);  // p + 1 < NP implies pb + 1 < RA here
-        } else {
-          candidates(pb);
-        }
-      }
-    }
-  }
+  gj_wg<NP>(x, pos, A, logdet, sgn);
   // row p of A^-1 = right half of row perm[p]
 #pragma unroll
   for (int a = 0; a < RA; ++a)
@@ -237,18 +125,7 @@ __global__ __launch_bounds__(256, (NP <= 48 ? 2 : 1)) void det_mfma_kernel(Fermi
     }
   __syncthreads();
   if (tid == 0) {
-    // sign of the row permutation: parity from its cycles
-    unsigned long long seen = 0ull;
-    for (int p = 0; p < NP; ++p) {
-      if ((seen >> p) & 1ull) continue;
-      int len = 0, c = p;
-      while (len < NP && c < NP && !((seen >> c) & 1ull)) {
-        seen |= 1ull << c;
-        c = perm[c];
-        ++len;
-      }
-      if ((len & 1) == 0) sgn = -sgn;
-    }
+    sgn *= perm_sign(perm, NP);
   }
   double* o_ = out + det_id * (3 + T);
 
@@ -486,7 +363,7 @@ __global__ __launch_bounds__(256) void det_fwd_reg_kernel(FermiDims d, const flo
 // tile in the wave's LDS slice.
 // ---------------------------------------------------------------------------
 
-constexpr int SM_NP = 16;
+constexpr int SM_NP = kGjWave;
 // coordinates in flight in the small kernel (even).  Two, with the kernel
 // bounded to 128 VGPRs (four waves per SIMD, 16 per CU), beat four at three
 // waves per SIMD: more waves hide the LDS transposes and wave barriers.
@@ -549,14 +426,6 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
 
   LogAbsProduct logdet;
   int sgn = 1;
-  // pivot search over rows p..15 in lanes 0..15: DPP butterfly within the
-  // first 16-lane row (largest |value|, smallest row on ties)
-  auto pick = [&](double& v, int& bi, double ov, int oi) __attribute__((always_inline)) {
-    if (oi != SM_NP && (bi == SM_NP || ov > v || (ov == v && oi < bi))) {
-      v = ov;
-      bi = oi;
-    }
-  };
   if constexpr (!lapmode) {
     // forward mode needs only log|det| and the sign: LU without row
     // exchanges with the 16x16 block in registers.  Lane (ti, tj) =
@@ -581,10 +450,7 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
         if (b == pb) xp = x[b];
       double v = used ? -1.0 : fabs(xp);
       int bi = used ? SM_NP : ti;
-      pick(v, bi, dpp_d<0xB1>(v), __builtin_amdgcn_mov_dpp(bi, 0xB1, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x4E>(v), __builtin_amdgcn_mov_dpp(bi, 0x4E, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x141>(v), __builtin_amdgcn_mov_dpp(bi, 0x141, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x140>(v), __builtin_amdgcn_mov_dpp(bi, 0x140, 0xF, 0xF, false));
+      gj_pick16(v, bi);
       int q = __builtin_amdgcn_readlane(bi, 16 * pr);
       if (q >= SM_NP) q = 0;  // unreachable: an unused row always remains
       const double piv = readlane_d(xp, 16 * pr + q);
@@ -609,17 +475,7 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
       wave_sync();
     }
     if (lane == 0) {
-      int seen = 0;
-      for (int p0 = 0; p0 < SM_NP; ++p0) {
-        if ((seen >> p0) & 1) continue;
-        int len = 0, c = p0;
-        while (len < SM_NP && c < SM_NP && !((seen >> c) & 1)) {
-          seen |= 1 << c;
-          c = perm[c];
-          ++len;
-        }
-        if ((len & 1) == 0) sgn = -sgn;
-      }
+      sgn *= perm_sign(perm, SM_NP);
       double* o_ = out + det_id * 3;
       o_[0] = logdet.log_abs();
       o_[1] = (double)sgn;
@@ -627,75 +483,20 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
     }
     return;
   }
-  // Gauss-Jordan on [A | I] with the matrix in registers and no row
-  // exchanges: lane (ti, tj) = (lane % 16, lane / 16) owns row ti, columns
-  // tj + 4b (b = 0..7).  The pivot of column p is the unused row with the
-  // largest |entry| (smallest row on ties), reduced with DPP inside the
-  // 16-lane row that holds column p; the pivot row and column are published
-  // through LDS; at the end row p of A^-1 is the right half of the pivot row
-  // of column p, and the parity of that row permutation enters the sign.
+  // Gauss-Jordan on [A | I] with the matrix in registers (gauss_jordan.h)
   {
     const int ti = lane & 15, tj = lane >> 4;
     double x[8];
 #pragma unroll
     for (int b = 0; b < 8; ++b) x[b] = S.M[ti * 32 + tj + 4 * b];
-    bool used = false;
     int pos = 0;
-    double* prow = S.Tt;       // 32 doubles
-    double* pcol = S.Tt + 32;  // 16 doubles
-    int* perm = (int*)(S.Tt + 48);
-    for (int p = 0; p < SM_NP; ++p) {
-      const int pb = p >> 2, pr = p & 3;
-      double xp = 0.0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if (b == pb) xp = x[b];
-      double v = used ? -1.0 : fabs(xp);
-      int bi = used ? SM_NP : ti;
-      pick(v, bi, dpp_d<0xB1>(v), __builtin_amdgcn_mov_dpp(bi, 0xB1, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x4E>(v), __builtin_amdgcn_mov_dpp(bi, 0x4E, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x141>(v), __builtin_amdgcn_mov_dpp(bi, 0x141, 0xF, 0xF, false));
-      pick(v, bi, dpp_d<0x140>(v), __builtin_amdgcn_mov_dpp(bi, 0x140, 0xF, 0xF, false));
-      int q = __builtin_amdgcn_readlane(bi, 16 * pr);
-      if (q >= SM_NP) q = 0;  // unreachable: an unused row always remains
-      const double piv = readlane_d(xp, 16 * pr + q);
-      logdet.mul(piv);
-      if (piv < 0) sgn = -sgn;
-      if (lane == 0) perm[p] = q;
-      if (ti == q) {
-#pragma unroll
-        for (int b = 0; b < 8; ++b) prow[tj + 4 * b] = x[b];
-      }
-      if (tj == pr) pcol[ti] = xp;
-      wave_sync();
-      const double rp = 1.0 / piv;
-      const double f = ti == q ? 0.0 : pcol[ti];
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const double r = prow[tj + 4 * b] * rp;
-        x[b] = ti == q ? r : x[b] - f * r;
-      }
-      if (ti == q) {
-        used = true;
-        pos = p;
-      }
-      wave_sync();
-    }
+    int* const perm = gj_wave_perm(S.Tt);
+    gj_wave16(x, pos, S.Tt, logdet, sgn);
     // row pos of A^-1 = right half of this lane's row
 #pragma unroll
     for (int b = 4; b < 8; ++b) S.M[pos * 32 + tj + 4 * b] = x[b];
     if (lane == 0) {
-      int seen = 0;
-      for (int p0 = 0; p0 < SM_NP; ++p0) {
-        if ((seen >> p0) & 1) continue;
-        int len = 0, c = p0;
-        while (len < SM_NP && c < SM_NP && !((seen >> c) & 1)) {
-          seen |= 1 << c;
-          c = perm[c];
-          ++len;
-        }
-        if ((len & 1) == 0) sgn = -sgn;
-      }
+      sgn *= perm_sign(perm, SM_NP);
     }
     wave_sync();
   }

@@ -18,111 +18,156 @@
 // adjoint, the walker sums and the mean adjoints, and the weight-gradient
 // contraction X^T dY over walker rows (FP32 MFMA, deterministic slices).
 
+#include "gauss_jordan.h"
 #include "grad.h"
 
 namespace {
 
-constexpr int GJ_NP = 64;
+// w_k of determinant k of a walker (stride-3 determinant records), formed
+// by one wavefront; uniform result.
+__device__ inline double det_weight(const double* __restrict__ dw, int K, int k) {
+  const int lane = threadIdx.x & 63;
+  double m = -INFINITY;
+  for (int j = lane; j < K; j += 64) m = fmax(m, dw[j * 3]);
+  m = wave_max_d(m);
+  double S = 0.0;
+  for (int j = lane; j < K; j += 64) S += dw[j * 3 + 1] * exp(dw[j * 3] - m);
+  S = wave_sum_d(S);
+  return dw[k * 3 + 1] * exp(dw[k * 3] - m) / S;
+}
 
-// dA_k = c_w w_k A_k^-T for one (walker, det) per workgroup, by FP64
-// Gauss-Jordan with partial pivoting on [A | I] in LDS.  Writes
+// dA_k = c_w w_k A_k^-T for one (walker, det), by FP64 Gauss-Jordan in
+// registers (gauss_jordan.h): one workgroup each for 16 < N <= 64, one
+// wavefront for N <= 16.  Writes
 //   dPhi[unit(w,i)][k N + o] = dA[i][o] env[i][o]
 //   denv[w][i][k N + o]      = dA[i][o] Phi[i][o]
 // A walker with c_w = 0 writes zeros without touching its matrices (a zero
-// weight stays exact even for a singular walker).
-__global__ __launch_bounds__(256) void det_vjp_kernel(FermiDims d, const float* __restrict__ Phi, long ldphi,
-                                                      const float* __restrict__ env, const double* __restrict__ det,
-                                                      const double* __restrict__ cot, int b0,
-                                                      float* __restrict__ dPhi, long lddphi,
-                                                      float* __restrict__ denv) {
-  __shared__ double M[GJ_NP][2 * GJ_NP + 1];
-  __shared__ double red_v[256];
-  __shared__ int red_i[256];
-  __shared__ double mult[GJ_NP];  // column p of the rows, read before the update
-  __shared__ double wk_s;
-  const int w = blockIdx.x / d.K, k = blockIdx.x % d.K;
-  const int N = d.N, KN = d.K * d.N;
-  const int tid = threadIdx.x;
-  const double c = cot[b0 + w];
-  if (c == 0.0) {
-    for (int e = tid; e < N * N; e += 256) {
-      const int i = e / N, o = e % N;
-      dPhi[(long)unit_idx(d, w, i) * lddphi + k * N + o] = 0.f;
-      denv[((long)w * N + i) * KN + k * N + o] = 0.f;
+// weight stays exact even for a singular walker).  Bound by the latency of the
+// pivot steps (two barriers each; wavefronts have none): 4096 matrices of 42 in
+// 270 us (1184 with the matrix in LDS and a barrier tree for each pivot), 16384
+// of 14 in 73 us (800).  A workgroup inverts a matrix of up to 16 in the same
+// steps as one wavefront, at four times the waves: hence the line at 16.
+struct DetVjp {
+  FermiDims d;
+  const float* Phi;
+  long ldphi;
+  const float* env;
+  const double* det;
+  const double* cot;
+  int b0;
+  float* dPhi;
+  long lddphi;
+  float* denv;
+};
+// thread t of nt writes its share of (walker w, det k); Inv row o, column i at Inv[o * is + i]
+__device__ inline void det_vjp_out(const DetVjp& a, int w, int k, double scale, const double* Inv, int is, int t,
+                                   int nt) {
+  const int N = a.d.N, KN = a.d.K * N;
+  for (int e = t; e < N * N; e += nt) {
+    const int i = e / N, o = e % N;
+    const long u = unit_idx(a.d, w, i), ie = ((long)w * N + i) * KN + k * N + o;
+    float gp = 0.f, ge = 0.f;
+    if (Inv) {
+      const double da = scale * Inv[o * is + i];
+      gp = (float)(da * a.env[ie * env_stride(a.d)]);
+      ge = (float)(da * a.Phi[u * a.ldphi + k * N + o]);
     }
+    a.dPhi[u * a.lddphi + k * N + o] = gp;
+    a.denv[ie] = ge;
+  }
+}
+
+template <int NP>
+__global__ __launch_bounds__(256) void det_vjp_wg_kernel(DetVjp a) {
+  constexpr int IS = NP + 1;  // odd row stride: transposed reads hit distinct banks
+  __shared__ double M[NP * IS];
+  __shared__ double wk_s;
+  static_assert(NP * IS >= gj_wg_scratch<NP>(), "the scratch takes the matrix's place");
+  const int w = blockIdx.x / a.d.K, k = blockIdx.x % a.d.K, N = a.d.N, tid = threadIdx.x;
+  const double c = a.cot[a.b0 + w];
+  if (c == 0.0) {
+    det_vjp_out(a, w, k, 0.0, nullptr, 0, tid, 256);
     return;
   }
-  if (tid == 0) {
-    const double* dw = det + (long)w * d.K * 3;
-    double m = -INFINITY;
-    for (int j = 0; j < d.K; ++j) m = fmax(m, dw[j * 3]);
-    double S = 0.0;
-    for (int j = 0; j < d.K; ++j) S += dw[j * 3 + 1] * exp(dw[j * 3] - m);
-    wk_s = dw[k * 3 + 1] * exp(dw[k * 3] - m) / S;
+  if (tid < 64) {
+    const double wk = det_weight(a.det + (long)w * a.d.K * 3, a.d.K, k);
+    if (tid == 0) wk_s = wk;
   }
-  for (int e = tid; e < N * 2 * N; e += 256) {
-    const int i = e / (2 * N), j = e % (2 * N);
-    double v;
-    if (j < N)
-      v = (double)Phi[(long)unit_idx(d, w, i) * ldphi + k * N + j] *
-          (double)env[(((long)w * N + i) * KN + k * N + j) * env_stride(d)];
-    else
-      v = (j - N == i) ? 1.0 : 0.0;
-    M[i][j] = v;
+  for (int e = tid; e < NP * NP; e += 256) {
+    const int i = e / NP, o = e % NP;
+    double v = i == o ? 1.0 : 0.0;
+    if (i < N && o < N)
+      v = (double)a.Phi[(long)unit_idx(a.d, w, i) * a.ldphi + k * N + o] *
+          (double)a.env[(((long)w * N + i) * a.d.K * N + k * N + o) * env_stride(a.d)];
+    M[i * IS + o] = v;
   }
   __syncthreads();
-  for (int p = 0; p < N; ++p) {
-    // pivot: largest |M[r][p]| over r >= p
-    double best = -1.0;
-    int bi = p;
-    for (int r = p + tid; r < N; r += 256) {
-      const double a = fabs(M[r][p]);
-      if (a > best) {
-        best = a;
-        bi = r;
-      }
+  constexpr int RA = NP / 16, CB = NP / 8;
+  const int ti = tid & 15, tj = tid >> 4;
+  double x[RA][CB];
+#pragma unroll
+  for (int r = 0; r < RA; ++r)
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int i = ti + 16 * r, j = tj + 16 * b;
+      x[r][b] = j < NP ? M[i * IS + j] : (i == j - NP ? 1.0 : 0.0);
     }
-    red_v[tid] = best;
-    red_i[tid] = bi;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (tid < s && red_v[tid + s] > red_v[tid]) {
-        red_v[tid] = red_v[tid + s];
-        red_i[tid] = red_i[tid + s];
-      }
-      __syncthreads();
+  __syncthreads();  // M is scratch from here on
+  int pos[RA];
+  LogAbsProduct logdet;
+  int sgn = 1;
+  gj_wg<NP>(x, pos, M, logdet, sgn);
+  __syncthreads();  // the scratch is read; M takes the inverse
+#pragma unroll
+  for (int r = 0; r < RA; ++r)
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int j = tj + 16 * b;
+      if (j >= NP) M[pos[r] * IS + (j - NP)] = x[r][b];
     }
-    const int pr = red_i[0];
-    if (pr != p)
-      for (int j = tid; j < 2 * N; j += 256) {
-        const double t = M[p][j];
-        M[p][j] = M[pr][j];
-        M[pr][j] = t;
-      }
-    __syncthreads();
-    const double inv = 1.0 / M[p][p];
-    __syncthreads();
-    for (int j = tid; j < 2 * N; j += 256) M[p][j] *= inv;
-    for (int r = tid; r < N; r += 256)
-      if (r != p) mult[r] = M[r][p];
-    __syncthreads();
-    for (int e = tid; e < N * 2 * N; e += 256) {
-      const int r = e / (2 * N), j = e % (2 * N);
-      if (r != p) M[r][j] -= mult[r] * M[p][j];
-    }
-    __syncthreads();
+  __syncthreads();
+  det_vjp_out(a, w, k, c * wk_s, M, IS, tid, 256);
+}
+
+__global__ __launch_bounds__(256) void det_vjp_wave_kernel(DetVjp a) {
+  constexpr int NP = kGjWave, IS = NP + 1;
+  __shared__ double Ms[4][NP * IS];
+  __shared__ double scratch[4][kGjWaveScratch];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, N = a.d.N, K = a.d.K;
+  const int kb = (K + 3) / 4, w = blockIdx.x / kb, k = 4 * (blockIdx.x % kb) + wave;
+  if (k >= K) return;  // the whole wave; no workgroup barriers below
+  const double c = a.cot[a.b0 + w];
+  if (c == 0.0) {
+    det_vjp_out(a, w, k, 0.0, nullptr, 0, lane, 64);
+    return;
   }
-  // inverse in columns N..2N-1: Ainv[o][i] = M[o][N + i]; dA[i][o] = c w_k Ainv[o][i]
-  const double scale = c * wk_s;
-  for (int e = tid; e < N * N; e += 256) {
-    const int i = e / N, o = e % N;
-    const double da = scale * M[o][N + i];
-    const long u = unit_idx(d, w, i);
-    const float ph = Phi[u * ldphi + k * N + o];
-    const float ev = env[(((long)w * N + i) * KN + k * N + o) * env_stride(d)];
-    dPhi[u * lddphi + k * N + o] = (float)(da * ev);
-    denv[((long)w * N + i) * KN + k * N + o] = (float)(da * ph);
+  const double wk = det_weight(a.det + (long)w * K * 3, K, k);
+  double* M = Ms[wave];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int e = lane + 64 * t, i = e >> 4, o = e & 15;
+    double v = i == o ? 1.0 : 0.0;
+    if (i < N && o < N)
+      v = (double)a.Phi[(long)unit_idx(a.d, w, i) * a.ldphi + k * N + o] *
+          (double)a.env[(((long)w * N + i) * K * N + k * N + o) * env_stride(a.d)];
+    M[i * IS + o] = v;
   }
+  wave_sync();
+  const int ti = lane & 15, tj = lane >> 4;
+  double x[8];
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int j = tj + 4 * b;
+    x[b] = j < NP ? M[ti * IS + j] : (ti == j - NP ? 1.0 : 0.0);
+  }
+  int pos = 0;
+  LogAbsProduct logdet;
+  int sgn = 1;
+  gj_wave16(x, pos, scratch[wave], logdet, sgn);
+#pragma unroll
+  for (int b = 4; b < 8; ++b) M[pos * IS + tj + 4 * b - NP] = x[b];
+  wave_sync();
+  det_vjp_out(a, w, k, c * wk, M, IS, lane, 64);
 }
 
 // Envelope parameter gradients, one wavefront per (orbital set, o, I, k),
@@ -429,9 +474,17 @@ inline int grid_of(long total) {
 
 int launch_det_vjp(const FermiDims& d, const float* Phi, long ldphi, const float* env, const double* det,
                    const double* cot, int b0, float* dPhi, long lddphi, float* denv, hipStream_t s) {
-  if (d.N > GJ_NP) return -1;
-  hipLaunchKernelGGL(det_vjp_kernel, dim3(d.Bc * d.K), dim3(256), 0, s, d, Phi, ldphi, env, det, cot, b0, dPhi,
-                     lddphi, denv);
+  const DetVjp a{d, Phi, ldphi, env, det, cot, b0, dPhi, lddphi, denv};
+  if (d.N <= kGjWave)
+    hipLaunchKernelGGL(det_vjp_wave_kernel, dim3(d.Bc * ((d.K + 3) / 4)), dim3(256), 0, s, a);
+  else if (d.N <= 32)
+    hipLaunchKernelGGL(det_vjp_wg_kernel<32>, dim3(d.Bc * d.K), dim3(256), 0, s, a);
+  else if (d.N <= 48)
+    hipLaunchKernelGGL(det_vjp_wg_kernel<48>, dim3(d.Bc * d.K), dim3(256), 0, s, a);
+  else if (d.N <= 64)
+    hipLaunchKernelGGL(det_vjp_wg_kernel<64>, dim3(d.Bc * d.K), dim3(256), 0, s, a);
+  else
+    return -1;
   return 0;
 }
 

@@ -293,3 +293,25 @@ def test_vjp_ragged_batch(cuda, case):
     ref = _torch_grad_unused(spec, p, x, sysm.atoms, np.bincount(who, cot))
     dm.close()
     assert np.all(np.abs(g - ref) <= 1e-4 * np.abs(ref).max() + 1e-3 * np.abs(ref))
+
+
+# the adjoint's workgroup inversions of 32 and 64 rows (padding rows in both)
+@pytest.mark.parametrize("n", [20, 50])
+def test_vjp_larger_determinants(cuda, n):
+    """Hydrogen chains with spread envelopes, whose orbital matrices an FP32
+    evaluation inverts to better than a sixth of this file's tolerance."""
+    import torch
+
+    from jaqmc_amd.device import DeviceModel
+
+    print(f"[grad] chain of {n}", flush=True)
+    sysm = S.h_chain(n)
+    spec = P.ModelSpec("ferminet", sysm.nspins, n, ndets=2, hidden_single=[32, 32], hidden_double=[8, 8])
+    p = P.init_params(spec, seed=51, bias_scale=0.1, env_jitter=1.0)
+    x = S.init_walkers(sysm, 4, seed=52)
+    cot = np.array([0.5, 1.25, 0.0, 2.0])
+    dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, with_gradients=True)
+    g = dm.logpsi_vjp(torch.from_numpy(x).to(cuda), torch.from_numpy(cot).to(cuda)).cpu().numpy()
+    dm.close()
+    ref = _torch_grad(spec, p, x, sysm.atoms, cot)
+    assert np.all(np.abs(g - ref) <= 1e-4 * np.abs(ref).max() + 1e-3 * np.abs(ref))

@@ -170,56 +170,110 @@ __global__ __launch_bounds__(256) void det_vjp_wave_kernel(DetVjp a) {
   det_vjp_out(a, w, k, c * wk, M, IS, lane, 64);
 }
 
-// Envelope parameter gradients, one wavefront per (orbital set, o, I, k),
-// its lanes splitting the (walker, electron) terms and summing in FP64 in a
-// fixed order:
+// Envelope parameter gradients:
 //   d pi[o,I,k]    += sum_{w, i in set} denv[w][i][k N + o] e_iI
 //   d sigma[o,I,k] += sum denv pi e_iI (-r_iI) (sign(sigma) for abs_isotropic)
 // accumulated in FP64 into acc (pack layout (N, M, K) per set: pi then sigma,
 // at off0 / off1).  The device keeps pi, sigma as [I][k][o].
-__global__ void env_grad_kernel(FermiDims d, const float* __restrict__ elec, const float* __restrict__ atoms,
-                                const float* __restrict__ pi0, const float* __restrict__ pi1,
-                                const float* __restrict__ sg0, const float* __restrict__ sg1, int kind, int nsets,
-                                const float* __restrict__ denv, double* __restrict__ acc, long off0, long off1) {
-  const int N = d.N, M = d.M, K = d.K, KN = K * N;
-  const long per = (long)N * M * K;
-  const long tot = per * nsets;
-  const int lane = threadIdx.x & 63;
-  const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
-  for (long t = blockIdx.x * (long)(blockDim.x >> 6) + (threadIdx.x >> 6); t < tot; t += nwaves) {
-    const int set = (int)(t / per);
-    const long q = t % per;  // (o, I, k) in pack order
-    const int o = (int)(q / ((long)M * K)), I = (int)((q / K) % M), k = (int)(q % K);
-    const long qd = ((long)I * K + k) * N + o;  // device layout
-    const float pi = (set ? pi1 : pi0)[qd];
-    const float sg = (set ? sg1 : sg0)[qd];
-    const float a = kind == 1 ? fabsf(sg) : sg;
-    const float sgn = kind == 1 ? (sg > 0.f ? 1.f : (sg < 0.f ? -1.f : 0.f)) : 1.f;
-    int i0 = 0, i1 = N;
-    if (nsets == 2) {
-      i0 = set == 0 ? 0 : d.n_up;
-      i1 = set == 0 ? d.n_up : N;
-    }
-    double gp = 0.0, gs = 0.0;
-    const int ni = i1 - i0;
-    for (long wi = lane; wi < (long)d.Bc * ni; wi += 64) {
-      const int w = (int)(wi / ni), i = i0 + (int)(wi % ni);
-      const float* x = elec + ((long)w * N + i) * 3;
-      const float dx = x[0] - atoms[3 * I], dy = x[1] - atoms[3 * I + 1], dz = x[2] - atoms[3 * I + 2];
-      const float r = sqrtf(dx * dx + dy * dy + dz * dz);
-      const float e = expf(-a * r);
-      const double de = denv[((long)w * N + i) * KN + k * N + o];
-      gp += de * e;
-      gs += de * (double)(pi * e * (-r) * sgn);
-    }
-    gp = wave_sum_d(gp);
-    gs = wave_sum_d(gs);
-    if (lane == 0) {
-      const long off = set ? off1 : off0;
-      acc[off + q] += gp;
-      acc[off + per + q] += gs;
+// A workgroup owns 64 consecutive (k, o) of one set, one per lane, so that a
+// row of denv is read coalesced, EG_I nuclei, for which the row is used, and a
+// slice of the (walker, electron) rows, which its waves take in turn, EG_R rows
+// in flight.  Its FP64 sums go to the workspace, P[slice][set][pi | sigma][I][k
+// N + o], and env_sum_kernel adds the slices in order.  Bound by latency and the
+// exponentials (42 electrons, 12 nuclei, 16 determinants, 256 walkers: 408 ->
+// 85 us; 14, 2, 16, 1024: 60 -> 18 us): a wavefront per parameter gathered denv
+// at a row stride and read it once per nucleus.
+constexpr int EG_WAVES = 4, EG_I = 4, EG_R = 4;
+struct EnvGrad {
+  FermiDims d;
+  const float *elec, *atoms;
+  const float *pi[2], *sg[2];
+  int kind, nsets;
+  const float* denv;
+};
+__global__ __launch_bounds__(64 * EG_WAVES) void env_grad_kernel(EnvGrad a, int slices, double* __restrict__ P) {
+  __shared__ double red[EG_WAVES][64];
+  const FermiDims& d = a.d;
+  const int N = d.N, M = d.M, KN = d.K * N;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ko = blockIdx.x * 64 + lane, I0 = blockIdx.y * EG_I, set = blockIdx.z % a.nsets, sl = blockIdx.z / a.nsets;
+  const bool in = ko < KN;
+  float pi[EG_I], sa[EG_I], sgn[EG_I];
+  double gp[EG_I], gs[EG_I];
+  // distances are the same for all lanes: lane EG_I u + q forms that of row u
+  // to nucleus q
+  const int lu = lane / EG_I % EG_R, lI = I0 + lane % EG_I < M ? I0 + lane % EG_I : M - 1;
+  const float Rx = a.atoms[3 * lI], Ry = a.atoms[3 * lI + 1], Rz = a.atoms[3 * lI + 2];
+#pragma unroll
+  for (int q = 0; q < EG_I; ++q) {
+    const int I = I0 + q < M ? I0 + q : M - 1;
+    const long qd = (long)I * KN + (in ? ko : 0);  // device layout [I][k][o]
+    pi[q] = a.pi[set][qd];
+    const float sg = a.sg[set][qd];
+    sa[q] = a.kind == 1 ? fabsf(sg) : sg;
+    sgn[q] = a.kind == 1 ? (sg > 0.f ? 1.f : (sg < 0.f ? -1.f : 0.f)) : 1.f;
+    gp[q] = gs[q] = 0.0;
+  }
+  int i0 = 0, i1 = N;
+  if (a.nsets == 2) {
+    i0 = set == 0 ? 0 : d.n_up;
+    i1 = set == 0 ? d.n_up : N;
+  }
+  const int ni = i1 - i0, rows = d.Bc * ni;
+  for (int r0 = sl * EG_WAVES + wave; r0 < rows; r0 += EG_R * EG_WAVES * slices) {
+    auto walker_row = [&](int u) __attribute__((always_inline)) {
+      const int r = r0 + u * EG_WAVES * slices, rc = r < rows ? r : r0;
+      return (long)(rc / ni) * N + i0 + rc % ni;
+    };
+    float de[EG_R];
+#pragma unroll
+    for (int u = 0; u < EG_R; ++u)
+      de[u] = in && r0 + u * EG_WAVES * slices < rows ? a.denv[walker_row(u) * KN + ko] : 0.f;
+    const float* x = a.elec + walker_row(lu) * 3;
+    const float dx = x[0] - Rx, dy = x[1] - Ry, dz = x[2] - Rz;
+    const int rl = __float_as_int(sqrtf(dx * dx + dy * dy + dz * dz));
+#pragma unroll
+    for (int u = 0; u < EG_R; ++u)
+#pragma unroll
+      for (int q = 0; q < EG_I; ++q) {
+        const float rr = __int_as_float(__builtin_amdgcn_readlane(rl, EG_I * u + q));
+        const float e = expf(-sa[q] * rr);
+        gp[q] += (double)de[u] * e;
+        gs[q] += (double)de[u] * (double)(pi[q] * e * (-rr) * sgn[q]);
+      }
+  }
+  double* Ps = P + ((long)sl * a.nsets + set) * 2 * M * KN;
+#pragma unroll
+  for (int q = 0; q < 2 * EG_I; ++q) {
+    __syncthreads();
+    red[wave][lane] = q < EG_I ? gp[q % EG_I] : gs[q % EG_I];
+    __syncthreads();
+    const int I = I0 + q % EG_I;
+    if (wave == 0 && in && I < M) {
+      double t = 0.0;
+#pragma unroll
+      for (int v = 0; v < EG_WAVES; ++v) t += red[v][lane];
+      Ps[((long)(q < EG_I ? 0 : M) + I) * KN + ko] = t;
     }
   }
+}
+__global__ void env_sum_kernel(int N, int M, int K, int nsets, int slices, const double* __restrict__ P,
+                               double* __restrict__ acc, long off0, long off1) {
+  const int KN = K * N, per = M * KN;
+  const int e = blockIdx.x * 256 + threadIdx.x;  // [set][pi | sigma][I][k N + o]
+  if (e >= 2 * per * nsets) return;
+  double s = 0.0;
+  int z = 0;
+  for (; z + 8 <= slices; z += 8) {  // eight slices in flight, added in order
+    double t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = P[(long)(z + u) * 2 * per * nsets + e];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += t[u];
+  }
+  for (; z < slices; ++z) s += P[(long)z * 2 * per * nsets + e];
+  const int set = e / (2 * per), part = e / per % 2, I = e / KN % M, k = e % KN / N, o = e % N;
+  acc[(set ? off1 : off0) + (long)part * per + ((long)o * M + I) * K + k] += s;
 }
 
 // tanh and residual adjoint of h_new = tanh(z) (+ h_old) / sqrt 2:
@@ -270,33 +324,81 @@ __global__ void one_adj_kernel(FermiDims d, int f1, const float* __restrict__ dX
   }
 }
 
-// dh2[w][j][i][f] += dX[unit(w,i)][col0 + ch(j) f2 + f] / n_ch(j)  (pair means
-// over the first index j within its spin channel)
-__global__ void pair_adj_kernel(FermiDims d, int f2, const float* __restrict__ dX, long lddx, int col0,
-                                float* __restrict__ dh2) {
-  const long tot = (long)d.Bc * d.N * d.N * f2;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-    const int f = (int)(e % f2);
-    const long p = e / f2;
-    const int i = (int)(p % d.N), j = (int)((p / d.N) % d.N), w = (int)(p / ((long)d.N * d.N));
-    const int ch = (d.nch == 2 && j >= d.n_up) ? 1 : 0;
-    const int nc = d.nch == 2 ? (ch ? d.n_dn : d.n_up) : d.N;
-    dh2[e] += dX[(long)unit_idx(d, w, i) * lddx + col0 + ch * f2 + f] / (float)nc;
+// Adjoint of the pair stream's input of one layer, for pair (w, j, i):
+//   dh2[f] = sum_n dz2[n] W2[f][n] (+ dh2_new[f] / sqrt 2 with the residual)   (dz2 set)
+//          + dX[unit(w,i)][col0 + ch(j) f2 + f] / n_ch(j)
+// (the layer's own pair product, then the pair means over the first index j
+// within its spin channel).  A workgroup stages W2 and the dz2 rows of PD_P
+// pairs in LDS; a thread owns one f and several pairs, so a weight is read once
+// for PD_V of them.  Memory-bound: 200704 pairs of 32 in 36 us, where the
+// product alone took 379 us with W2 gathered from global memory and the means
+// another 25.
+constexpr int PD_P = 64, PD_V = 8;
+__global__ __launch_bounds__(256) void pair_bwd_kernel(FermiDims d, long npairs, int f2, int fout,
+                                                       const float* __restrict__ dz2, const float* __restrict__ W2,
+                                                       int res, const float* __restrict__ dh2new,
+                                                       const float* __restrict__ dX, long lddx, int col0,
+                                                       float* __restrict__ dh2) {
+  extern __shared__ float sm[];
+  const int tid = threadIdx.x, SW = fout + 1;
+  float* Ws = sm;              // [f2][fout + 1]
+  float* Zs = Ws + f2 * SW;    // [PD_P][fout]
+  const long p0 = (long)blockIdx.x * PD_P;
+  if (dz2) {
+    for (int e = tid; e < f2 * fout; e += 256) Ws[(e / fout) * SW + e % fout] = W2[e];
+    const long lim = (npairs - p0) * fout;
+    for (int e = tid; e < PD_P * fout; e += 256) Zs[e] = e < lim ? dz2[p0 * fout + e] : 0.f;
+    __syncthreads();
+  }
+  const int groups = 256 / f2 > 0 ? 256 / f2 : 1;  // pairs side by side
+  const int NN = d.N * d.N;
+  for (int f = f2 <= 256 ? tid % f2 : tid; f < f2; f += f2 <= 256 ? f2 : 256) {
+    const int g = f2 <= 256 ? tid / f2 : 0;
+    if (g >= groups) break;
+    for (int pb = g; pb < PD_P; pb += groups * PD_V) {
+      float s[PD_V];
+#pragma unroll
+      for (int v = 0; v < PD_V; ++v) s[v] = 0.f;
+      if (dz2)
+        for (int n = 0; n < fout; ++n) {
+          const float wv = Ws[f * SW + n];
+#pragma unroll
+          for (int v = 0; v < PD_V; ++v) {
+            const int q = pb + v * groups;
+            s[v] += Zs[(q < PD_P ? q : 0) * fout + n] * wv;
+          }
+        }
+#pragma unroll
+      for (int v = 0; v < PD_V; ++v) {
+        const int q = pb + v * groups;
+        const long p = p0 + q;
+        if (q >= PD_P || p >= npairs) continue;
+        const int w = (int)(p / NN), rem = (int)(p % NN), j = rem / d.N, i = rem % d.N;
+        const int ch = (d.nch == 2 && j >= d.n_up) ? 1 : 0;
+        const int nc = d.nch == 2 ? (ch ? d.n_dn : d.n_up) : d.N;
+        float t = s[v];
+        if (dz2 && res) t += dh2new[p * fout + f] * 0.70710678118654752f;
+        dh2[p * f2 + f] = t + dX[(long)unit_idx(d, w, i) * lddx + col0 + ch * f2 + f] / (float)nc;
+      }
+    }
   }
 }
 
-// dh2_old[p][f] = sum_n dz2[p][n] W2[f][n] (+ dh2_new[p][f] / sqrt 2 with the residual)
-__global__ void pair_dx_kernel(long npairs, int fin, int fout, const float* __restrict__ dz2,
-                               const float* __restrict__ W2, int res, const float* __restrict__ dh2new,
-                               float* __restrict__ dh2old) {
-  const long tot = npairs * fin;
+// Wider pair streams than the staged weights' LDS: one thread per entry.
+__global__ void pair_bwd_wide_kernel(FermiDims d, long npairs, int f2, int fout, const float* __restrict__ dz2,
+                                     const float* __restrict__ W2, int res, const float* __restrict__ dh2new,
+                                     const float* __restrict__ dX, long lddx, int col0, float* __restrict__ dh2) {
+  const long tot = npairs * f2;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-    const long p = e / fin;
-    const int f = (int)(e % fin);
+    const long p = e / f2;
+    const int f = (int)(e % f2);
     float s = 0.f;
     for (int n = 0; n < fout; ++n) s += dz2[p * fout + n] * W2[f * fout + n];
     if (res) s += dh2new[p * fout + f] * 0.70710678118654752f;
-    dh2old[e] = s;
+    const int i = (int)(p % d.N), j = (int)((p / d.N) % d.N), w = (int)(p / ((long)d.N * d.N));
+    const int ch = (d.nch == 2 && j >= d.n_up) ? 1 : 0;
+    const int nc = d.nch == 2 ? (ch ? d.n_dn : d.n_up) : d.N;
+    dh2[e] = s + dX[(long)unit_idx(d, w, i) * lddx + col0 + ch * f2 + f] / (float)nc;
   }
 }
 
@@ -488,12 +590,23 @@ int launch_det_vjp(const FermiDims& d, const float* Phi, long ldphi, const float
   return 0;
 }
 
-int launch_env_grad(const FermiDims& d, const float* elec, const float* atoms, const float* pi0, const float* pi1,
-                    const float* sg0, const float* sg1, int kind, int nsets, const float* denv, double* acc,
+// P: workspace of cap doubles
+int launch_env_grad(const FermiDims& d, const float* elec, const float* atoms, const float* const* pi,
+                    const float* const* sg, int kind, int nsets, const float* denv, double* P, long cap, double* acc,
                     long off0, long off1, hipStream_t s) {
-  const long tot = (long)d.N * d.M * d.K * nsets;  // one wavefront each
-  hipLaunchKernelGGL(env_grad_kernel, dim3(grid_of(tot * 64)), dim3(256), 0, s, d, elec, atoms, pi0, pi1, sg0, sg1,
-                     kind, nsets, denv, acc, off0, off1);
+  const EnvGrad a{d, elec, atoms, {pi[0], pi[1]}, {sg[0], sg[1]}, kind, nsets, denv};
+  const int bx = ceil_div((long)d.K * d.N, 64), by = ceil_div(d.M, EG_I);
+  // about 1024 workgroups, but at least two turns of its rows for each wave
+  const long entries = 2L * d.M * d.K * d.N * nsets, turns = ceil_div((long)d.Bc * d.N, 2 * EG_R * EG_WAVES);
+  long slices = 1024 / ((long)bx * by * nsets);
+  slices = slices > turns ? turns : slices;
+  while (slices > 1 && slices * entries > cap) slices >>= 1;
+  slices = slices < 1 ? 1 : slices;
+  if (entries > cap) return -1;
+  hipLaunchKernelGGL(env_grad_kernel, dim3(bx, by, (unsigned)(nsets * slices)), dim3(64 * EG_WAVES), 0, s, a,
+                     (int)slices, P);
+  hipLaunchKernelGGL(env_sum_kernel, dim3(ceil_div(entries, 256)), dim3(256), 0, s, d.N, d.M, d.K, nsets, (int)slices,
+                     P, acc, off0, off1);
   return 0;
 }
 
@@ -516,16 +629,18 @@ int launch_one_adj(const FermiDims& d, int f1, const float* dX, long lddx, const
   return 0;
 }
 
-int launch_pair_adj(const FermiDims& d, int f2, const float* dX, long lddx, int col0, float* dh2, hipStream_t s) {
-  hipLaunchKernelGGL(pair_adj_kernel, dim3(grid_of((long)d.Bc * d.N * d.N * f2)), dim3(256), 0, s, d, f2, dX, lddx,
-                     col0, dh2);
-  return 0;
-}
-
-int launch_pair_dx(long npairs, int fin, int fout, const float* dz2, const float* W2, int res, const float* dh2new,
-                   float* dh2old, hipStream_t s) {
-  hipLaunchKernelGGL(pair_dx_kernel, dim3(grid_of(npairs * fin)), dim3(256), 0, s, npairs, fin, fout, dz2, W2, res,
-                     dh2new, dh2old);
+// dz2 null: the means' part alone (fout, W2, res, dh2new unused)
+int launch_pair_bwd(const FermiDims& d, int f2, int fout, const float* dz2, const float* W2, int res,
+                    const float* dh2new, const float* dX, long lddx, int col0, float* dh2, hipStream_t s) {
+  const long npairs = (long)d.Bc * d.N * d.N;
+  if (!dz2) fout = 0;
+  const size_t smem = dz2 ? ((size_t)f2 * (fout + 1) + (size_t)PD_P * fout) * 4 : 0;
+  if (smem <= 64 * 1024)
+    hipLaunchKernelGGL(pair_bwd_kernel, dim3(ceil_div(npairs, PD_P)), dim3(256), smem, s, d, npairs, f2, fout, dz2, W2,
+                       res, dh2new, dX, lddx, col0, dh2);
+  else
+    hipLaunchKernelGGL(pair_bwd_wide_kernel, dim3(grid_of(npairs * f2)), dim3(256), 0, s, d, npairs, f2, fout, dz2, W2,
+                       res, dh2new, dX, lddx, col0, dh2);
   return 0;
 }
 

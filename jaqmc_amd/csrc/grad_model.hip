@@ -11,17 +11,16 @@
 
 int launch_det_vjp(const FermiDims& d, const float* Phi, long ldphi, const float* env, const double* det,
                    const double* cot, int b0, float* dPhi, long lddphi, float* denv, hipStream_t s);
-int launch_env_grad(const FermiDims& d, const float* elec, const float* atoms, const float* pi0, const float* pi1,
-                    const float* sg0, const float* sg1, int kind, int nsets, const float* denv, double* acc,
+int launch_env_grad(const FermiDims& d, const float* elec, const float* atoms, const float* const* pi,
+                    const float* const* sg, int kind, int nsets, const float* denv, double* P, long cap, double* acc,
                     long off0, long off1, hipStream_t s);
 int launch_tanh_bwd(long rows, int n, const float* hnew, long ldn, const float* hold, long ldo, const float* dhnew,
                     long lddn, int res, float* dz, long lddz, float* dhold, long lddo, hipStream_t s);
 int launch_walker_sum(const FermiDims& d, const float* dz, long lddz, int n, float* dG, long lddg, hipStream_t s);
 int launch_one_adj(const FermiDims& d, int f1, const float* dX, long lddx, const float* dg, long lddg, float* dh,
                    long lddh, hipStream_t s);
-int launch_pair_adj(const FermiDims& d, int f2, const float* dX, long lddx, int col0, float* dh2, hipStream_t s);
-int launch_pair_dx(long npairs, int fin, int fout, const float* dz2, const float* W2, int res, const float* dh2new,
-                   float* dh2old, hipStream_t s);
+int launch_pair_bwd(const FermiDims& d, int f2, int fout, const float* dz2, const float* W2, int res,
+                    const float* dh2new, const float* dX, long lddx, int col0, float* dh2, hipStream_t s);
 int launch_fill_f64(double* p, long n, double v, hipStream_t s);
 int launch_fill_f32(float* p, long n, float v, hipStream_t s);
 int launch_f64_to_f32(const double* a, long n, float* out, hipStream_t s);
@@ -70,7 +69,8 @@ int jq_model::alloc_grad_workspace(size_t budget) {
   dZ2 = (float*)alloc((size_t)G * N * N * d2m * 4);
   dPhi = (float*)alloc((size_t)G * N * ldko * 4);
   dEnv = (float*)alloc((size_t)G * N * KN * 4);
-  pw_cap = 16l << 20;
+  // weight-gradient slices; also one slice of the envelope's FP64 sums
+  pw_cap = std::max(16l << 20, 4l * norb * M * KN);
   Pw = (float*)alloc((size_t)pw_cap * 4);
   gacc = (double*)alloc((size_t)n_params * 8);
   if (!dH[0] || !dH[1] || !dH2[0] || !dH2[1] || !dZ || !dX || !dG || !dg || !dZ2 || !dPhi || !dEnv || !Pw || !gacc)
@@ -176,9 +176,12 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
     if (rc) return rc;
     if (launch_det_vjp(fd, Phi, ldphi, env, det, cot, b0, dPhi, ldko, dEnv, s))
       return jq_fail(JQ_EINVAL, "determinant adjoint supports N <= 64");
-    if (d.envelope != JQ_ENV_NULL)
-      launch_env_grad(fd, ec, atoms, pi[0], pi[1], sigma[0], sigma[1], d.envelope, norb, dEnv, gacc, off_env[0],
-                      off_env[1], s);
+    if (d.envelope != JQ_ENV_NULL) {
+      wq.flush();  // its workspace holds the envelope's partial sums
+      if (launch_env_grad(fd, ec, atoms, pi, sigma, d.envelope, norb, dEnv, (double*)Pw, pw_cap / 2, gacc, off_env[0],
+                          off_env[1], s))
+        return jq_fail(JQ_EINVAL, "envelope adjoint exceeds the workspace");
+    }
     // orbital projection: dW_orb (channel rows, spin-blocked units), dh_L = dPhi W_orb^T
     const int dL = fl[L - 1].d1;
     float* dh = dH[0];
@@ -205,9 +208,6 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
                         s);
         rc = wq.add(wgrad_args(npairs, H2t[l], ly.f2, ly.f2, dZ2, ly.d2, ly.d2, ly.off_w2, true, ly.off_b2));
         if (rc) return jq_fail(JQ_EINVAL, "pair-stream adjoint launch rejected");
-        if (l > 0) launch_pair_dx(npairs, ly.f2, ly.d2, dZ2, ly.W2, ly.res2, dh2n, dh2o, s);
-      } else if (l > 0) {
-        launch_fill_f32(dh2o, npairs * ly.f2, 0.f, s);
       }
       // one-electron stream: dz, weight and bias gradients; the adjoint of h_l
       // starts from the residual branch (or zero, with its own width f1)
@@ -231,7 +231,8 @@ int jq_model::vjp(const float* elec, int B, const double* cot, float* grad, hipS
         rc |= gemm_nt(dZ, ldd, ly.Wm_o, ly.d1, ly.f1 + nch * ly.f2, dX, ly.kmain, units, s);
         if (rc) return jq_fail(JQ_EINVAL, "input adjoint GEMM launch rejected");
         launch_one_adj(fd, ly.f1, dX, ly.kmain, dg, ly.kg, dho, ldd, s);
-        launch_pair_adj(fd, ly.f2, dX, ly.kmain, ly.f1, dh2o, s);
+        launch_pair_bwd(fd, ly.f2, ly.d2, ly.has_pair ? dZ2 : nullptr, ly.W2, ly.res2, dh2n, dX, ly.kmain, ly.f1, dh2o,
+                        s);
         std::swap(dh, dho);
         std::swap(dh2n, dh2o);
       }
@@ -321,7 +322,8 @@ int jq_model::alloc_grad_workspace_psi(size_t budget) {
   dPhi = fa(U * ldko);
   dEnv = fa(U * KN);
   jtmp = fa(2 * (size_t)gchunk);
-  pw_cap = 16l << 20;
+  // weight-gradient slices; also one slice of the envelope's FP64 sums
+  pw_cap = std::max(16l << 20, 4l * norb * M * KN);
   Pw = fa(pw_cap);
   gacc = (double*)alloc((size_t)n_params * 8);
   if (!ok || !dH[0] || !dH1 || !dM[0] || !dM[1] || !dZ || !dO || !dQKV || !dXin || !Pln || !dPhi ||
@@ -466,9 +468,12 @@ int jq_model::vjp_psiformer(const float* elec, int B, const double* cot, hipStre
     if (rc) return rc;
     if (launch_det_vjp(fd, Phi, ldphi, env, det, cot, b0, dPhi, ldko, dEnv, s))
       return jq_fail(JQ_EINVAL, "determinant adjoint supports N <= 64");
-    if (d.envelope != JQ_ENV_NULL)
-      launch_env_grad(fd, ec, atoms, pi[0], pi[1], sigma[0], sigma[1], d.envelope, norb, dEnv, gacc, off_env[0],
-                      off_env[1], s);
+    if (d.envelope != JQ_ENV_NULL) {
+      wq.flush();  // its workspace holds the envelope's partial sums
+      if (launch_env_grad(fd, ec, atoms, pi, sigma, d.envelope, norb, dEnv, (double*)Pw, pw_cap / 2, gacc, off_env[0],
+                          off_env[1], s))
+        return jq_fail(JQ_EINVAL, "envelope adjoint exceeds the workspace");
+    }
     // orbital projection: weight (and bias) gradients from the channel's rows,
     // dH_L = dPhi W_orb^T per channel
     float* gH = dH[0];  // adjoint of the residual stream

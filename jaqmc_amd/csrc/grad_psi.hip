@@ -68,97 +68,147 @@ __global__ __launch_bounds__(256) void ln_bwd_kernel(long rows, int D, const flo
 // One workgroup per (walker, head).  Q, K, V come head-split
 // ([w][part][h][i][dh], one row per electron), dO row-major with the head's
 // features at columns h*dh; dq, dk, dv go to row-major [unit][part*D + h*dh + d].
+// Bound by LDS reads: threads work on register blocks, 2 x 4 scores with
+// 16-byte reads along d, then 4 rows x 4 features of dq, dk, dv (two thirds of
+// the reads of one output per thread go); softmax and its adjoint take a
+// wavefront per row.  42 electrons, 64-wide heads, 1024 walker-heads: 116 -> 87
+// us at two workgroups per CU.  Rows N .. N4 of the arrays are zeros.
+constexpr int AB_PAD = 4;  // row strides dh + 4, N4 + 4: 16-byte aligned, rows on shifted banks
 __global__ __launch_bounds__(256) void attn_bwd_kernel(const float* __restrict__ QKV, const float* __restrict__ dO,
                                                        long lddo, float* __restrict__ dQKV, long ldq, int N, int H,
                                                        int dh) {
-  extern __shared__ float sm[];
-  const int SR = dh + 1, SN = N + 1;
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int N4 = (N + 3) & ~3, SR = dh + AB_PAD, SN = N4 + AB_PAD;
   float* Qs = sm;
-  float* Ks = Qs + N * SR;
-  float* Vs = Ks + N * SR;
-  float* Gs = Vs + N * SR;  // dO
-  float* As = Gs + N * SR;  // scores, then a
-  float* Ds = As + N * SN;  // da, then ds
-  const int w = blockIdx.x / H, h = blockIdx.x % H, tid = threadIdx.x;
+  float* Ks = Qs + N4 * SR;
+  float* Vs = Ks + N4 * SR;
+  float* Gs = Vs + N4 * SR;  // dO
+  float* As = Gs + N4 * SR;  // scores, then a
+  float* Ds = As + N4 * SN;  // da, then ds
+  const int w = blockIdx.x / H, h = blockIdx.x % H, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long blk = (long)N * dh;
   const float* q = QKV + ((long)w * 3 * H + h) * blk;
-  for (int e = tid; e < N * dh; e += 256) {
+  for (int e = tid; e < N4 * dh; e += 256) {
     const int i = e / dh, d = e % dh;
-    Qs[i * SR + d] = q[e];
-    Ks[i * SR + d] = q[(long)H * blk + e];
-    Vs[i * SR + d] = q[2L * H * blk + e];
-    Gs[i * SR + d] = dO[((long)w * N + i) * lddo + h * dh + d];
+    const bool in = i < N;
+    Qs[i * SR + d] = in ? q[e] : 0.f;
+    Ks[i * SR + d] = in ? q[(long)H * blk + e] : 0.f;
+    Vs[i * SR + d] = in ? q[2L * H * blk + e] : 0.f;
+    Gs[i * SR + d] = in ? dO[((long)w * N + i) * lddo + h * dh + d] : 0.f;
   }
   __syncthreads();
-  for (int e = tid; e < N * N; e += 256) {
-    const int i = e / N, j = e % N;
-    float sa = 0.f, da = 0.f;
-    for (int d = 0; d < dh; ++d) {
-      sa += Qs[i * SR + d] * Ks[j * SR + d];
-      da += Gs[i * SR + d] * Vs[j * SR + d];
+  auto dot4 = [](float s, const float4& a, const float4& b) __attribute__((always_inline)) {
+    s += a.x * b.x;
+    s += a.y * b.y;
+    s += a.z * b.z;
+    return s + a.w * b.w;
+  };
+  const int nj = N4 / 4;
+  for (int e = tid; e < (N4 / 2) * nj; e += 256) {
+    const int i = 2 * (e / nj), j = 4 * (e % nj);
+    float sa[2][4] = {}, da[2][4] = {};
+    for (int d = 0; d < dh; d += 4) {
+      float4 x[2], g[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        x[u] = *(const float4*)&Qs[(i + u) * SR + d];
+        g[u] = *(const float4*)&Gs[(i + u) * SR + d];
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float4 k4 = *(const float4*)&Ks[(j + v) * SR + d], v4 = *(const float4*)&Vs[(j + v) * SR + d];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          sa[u][v] = dot4(sa[u][v], x[u], k4);
+          da[u][v] = dot4(da[u][v], g[u], v4);
+        }
+      }
     }
-    As[i * SN + j] = sa;
-    Ds[i * SN + j] = da;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        As[(i + u) * SN + j + v] = sa[u][v];
+        Ds[(i + u) * SN + j + v] = da[u][v];
+      }
   }
   __syncthreads();
-  for (int i = tid; i < N; i += 256) {
-    float m = -INFINITY;
-    for (int j = 0; j < N; ++j) m = fmaxf(m, As[i * SN + j]);
-    float z = 0.f;
-    for (int j = 0; j < N; ++j) {
-      const float e = expf(As[i * SN + j] - m);
-      As[i * SN + j] = e;
-      z += e;
+  for (int i = wave; i < N4; i += 4) {  // N <= 64: one column per lane
+    const bool in = lane < N && i < N;
+    const float s = in ? As[i * SN + lane] : -INFINITY;
+    const float m = wave_max(s);
+    const float e = in ? expf(s - m) : 0.f;
+    const float a = i < N ? e * (1.f / wave_sum(e)) : 0.f;
+    const float da = in ? Ds[i * SN + lane] : 0.f;
+    const float rsum = wave_sum(a * da);
+    if (lane < N4) {
+      As[i * SN + lane] = a;
+      Ds[i * SN + lane] = a * (da - rsum);
     }
-    const float iz = 1.f / z;
-    float rsum = 0.f;
-    for (int j = 0; j < N; ++j) {
-      const float a = As[i * SN + j] * iz;
-      As[i * SN + j] = a;
-      rsum += a * Ds[i * SN + j];
-    }
-    for (int j = 0; j < N; ++j) Ds[i * SN + j] = As[i * SN + j] * (Ds[i * SN + j] - rsum);
   }
   __syncthreads();
-  const int D = H * dh;
+  const int D = H * dh, nd = dh / 4;
   float* out = dQKV + (long)w * N * ldq + h * dh;
-  for (int e = tid; e < N * dh; e += 256) {
-    const int i = e / dh, d = e % dh;
-    float gq = 0.f, gk = 0.f, gv = 0.f;
+  auto fma4 = [](float4& s, float a, const float4& b) __attribute__((always_inline)) {
+    s.x += a * b.x;
+    s.y += a * b.y;
+    s.z += a * b.z;
+    s.w += a * b.w;
+  };
+  for (int e = tid; e < (N4 / 4) * nd; e += 256) {
+    const int i = 4 * (e / nd), d = 4 * (e % nd);
+    float4 gq[4] = {}, gk[4] = {}, gv[4] = {};
     for (int j = 0; j < N; ++j) {
-      gq += Ds[i * SN + j] * Ks[j * SR + d];
-      gk += Ds[j * SN + i] * Qs[j * SR + d];
-      gv += As[j * SN + i] * Gs[j * SR + d];
+      const float4 k4 = *(const float4*)&Ks[j * SR + d], q4 = *(const float4*)&Qs[j * SR + d],
+                   g4 = *(const float4*)&Gs[j * SR + d];
+      const float4 ds = *(const float4*)&Ds[j * SN + i], aj = *(const float4*)&As[j * SN + i];
+      const float dsj[4] = {ds.x, ds.y, ds.z, ds.w}, ajj[4] = {aj.x, aj.y, aj.z, aj.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        fma4(gq[u], Ds[(i + u) * SN + j], k4);
+        fma4(gk[u], dsj[u], q4);
+        fma4(gv[u], ajj[u], g4);
+      }
     }
-    out[(long)i * ldq + d] = gq;
-    out[(long)i * ldq + D + d] = gk;
-    out[(long)i * ldq + 2 * D + d] = gv;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i + u < N) {
+        float* o = out + (long)(i + u) * ldq + d;
+        *(float4*)o = gq[u];
+        *(float4*)(o + D) = gk[u];
+        *(float4*)(o + 2 * D) = gv[u];
+      }
   }
 }
 
-// out[w][0..1] = c_w dJ_w / d(alpha_par, alpha_anti), one thread per walker
-// of the chunk (walker b0 + w of the weights)
-__global__ void jastrow_grad_kernel(const float* __restrict__ elec, int Bc, int N, int n_up, float ap, float aa,
-                                    const double* __restrict__ cot, int b0, float* __restrict__ out) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= Bc) return;
+// out[w][0..1] = c_w dJ_w / d(alpha_par, alpha_anti), one wavefront per walker
+// of the chunk (walker b0 + w of the weights), its lanes taking the pairs in turn
+__global__ __launch_bounds__(64) void jastrow_grad_kernel(const float* __restrict__ elec, int Bc, int N, int n_up,
+                                                          float ap, float aa, const double* __restrict__ cot, int b0,
+                                                          float* __restrict__ out) {
+  const int w = blockIdx.x, lane = threadIdx.x;
   const float* x = elec + (long)w * N * 3;
   double gp = 0.0, ga = 0.0;
-  for (int i = 0; i < N; ++i)
-    for (int j = i + 1; j < N; ++j) {
-      const double dx = x[3 * i] - x[3 * j], dy = x[3 * i + 1] - x[3 * j + 1], dz = x[3 * i + 2] - x[3 * j + 2];
-      const double r = sqrt(dx * dx + dy * dy + dz * dz);
-      if ((i < n_up) == (j < n_up)) {
-        const double q = ap + r;
-        gp += -0.25 * ap * (ap + 2.0 * r) / (q * q);
-      } else {
-        const double q = aa + r;
-        ga += -0.5 * aa * (aa + 2.0 * r) / (q * q);
-      }
+  for (int e = lane; e < N * N; e += 64) {
+    const int i = e / N, j = e % N;
+    if (j <= i) continue;
+    const double dx = x[3 * i] - x[3 * j], dy = x[3 * i + 1] - x[3 * j + 1], dz = x[3 * i + 2] - x[3 * j + 2];
+    const double r = sqrt(dx * dx + dy * dy + dz * dz);
+    if ((i < n_up) == (j < n_up)) {
+      const double q = ap + r;
+      gp += -0.25 * ap * (ap + 2.0 * r) / (q * q);
+    } else {
+      const double q = aa + r;
+      ga += -0.5 * aa * (aa + 2.0 * r) / (q * q);
     }
-  const double c = cot[b0 + w];
-  out[2 * w] = (float)(c * gp);
-  out[2 * w + 1] = (float)(c * ga);
+  }
+  gp = wave_sum_d(gp);
+  ga = wave_sum_d(ga);
+  if (lane == 0) {
+    const double c = cot[b0 + w];
+    out[2 * w] = (float)(c * gp);
+    out[2 * w + 1] = (float)(c * ga);
+  }
 }
 
 // out[r][c] = a[r][c] + b[r][c]
@@ -192,12 +242,15 @@ int launch_ln_bwd(long rows, int D, const float* x, long ldx, const float* s, co
   return 0;
 }
 
-size_t attn_bwd_smem(int N, int dh) { return (size_t)(4 * N * (dh + 1) + 2 * N * (N + 1)) * 4; }
+size_t attn_bwd_smem(int N, int dh) {
+  const int N4 = round_up(N, 4);
+  return (size_t)(4 * N4 * (dh + AB_PAD) + 2 * N4 * (N4 + AB_PAD)) * 4;
+}
 
 int launch_attn_bwd(const float* QKV, const float* dO, long lddo, float* dQKV, long ldq, int Bc, int N, int H, int dh,
                     hipStream_t st) {
   const size_t smem = attn_bwd_smem(N, dh);
-  if (N > 64 || dh > 64 || Bc <= 0) return Bc <= 0 ? 0 : -1;
+  if (N > 64 || dh > 64 || dh % 4 || ldq % 4 || Bc <= 0) return Bc <= 0 ? 0 : -1;
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)attn_bwd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -212,7 +265,7 @@ int launch_attn_bwd(const float* QKV, const float* dO, long lddo, float* dQKV, l
 int launch_jastrow_grad(const float* elec, int Bc, int N, int n_up, float ap, float aa, const double* cot, int b0,
                         float* out, hipStream_t st) {
   if (Bc <= 0) return 0;
-  hipLaunchKernelGGL(jastrow_grad_kernel, dim3((unsigned)((Bc + 63) / 64)), dim3(64), 0, st, elec, Bc, N, n_up, ap, aa,
+  hipLaunchKernelGGL(jastrow_grad_kernel, dim3((unsigned)Bc), dim3(64), 0, st, elec, Bc, N, n_up, ap, aa,
                      cot, b0, out);
   return 0;
 }

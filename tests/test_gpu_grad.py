@@ -315,3 +315,24 @@ def test_vjp_larger_determinants(cuda, n):
     dm.close()
     ref = _torch_grad(spec, p, x, sysm.atoms, cot)
     assert np.all(np.abs(g - ref) <= 1e-4 * np.abs(ref).max() + 1e-3 * np.abs(ref))
+
+
+# pair-stream widths that do not divide a workgroup (24) and that exceed the
+# staged weights' memory (128)
+@pytest.mark.parametrize("width", [24, 128])
+def test_vjp_pair_widths(cuda, width):
+    import torch
+
+    from jaqmc_amd.device import DeviceModel
+
+    print(f"[grad] pair width {width}", flush=True)
+    sysm, spec, *_ = S.workload("li")
+    spec.hidden_single, spec.hidden_double = [32, 32, 32], [width] * 3
+    p = P.init_params(spec, seed=61, bias_scale=0.1, env_jitter=0.2)
+    x = S.init_walkers(sysm, 5, seed=62)
+    cot = np.array([0.5, 1.25, 0.75, 2.0, 1.0])
+    dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, with_gradients=True)
+    g = dm.logpsi_vjp(torch.from_numpy(x).to(cuda), torch.from_numpy(cot).to(cuda)).cpu().numpy()
+    dm.close()
+    ref = _torch_grad(spec, p, x, sysm.atoms, cot)
+    assert np.all(np.abs(g - ref) <= 1e-4 * np.abs(ref).max() + 1e-3 * np.abs(ref))

@@ -45,7 +45,7 @@
 
 #include "kernels.h"
 
-// 0: default tile table; else UPT*10 + NBW (benchmark override)
+// 0: default tile table; else UPT*10 + NBW, plain rows MB*10 + NBW (benchmark override)
 extern int g_gemm_variant;
 // 4: no eight-wave tiles (benchmark override); 0: default
 extern int g_gemm_nw;
@@ -975,28 +975,57 @@ void default_cfg(int R, int prec, bool wide, int* upt, int* nbw) {
   }
 }
 
+// Tile of a plain (value-row) launch: 16 mb rows x 64 nbw columns, from sweeps
+// on MI355X (jq_bench_gemm; every tile gives the same bits).  A CU works its
+// tiles off at the matrix rate, so the time follows the most tiles a CU gets:
+// the largest tile only where it leaves every CU enough of them.
+//   FP32: 64 x 64 from two tiles per CU on (10752 rows, K = N = 256: 20.4 us,
+//     21.3 at 32 x 64, 26.1 at 64 x 128, 32.1 at 128 x 128; 86016 rows: 109,
+//     119, 117, 126), then 32 x 64 down to one per CU (1024 x 512, K = 256: 7.6
+//     us, 8.1 at 16 x 64, 11.0 at 64 x 64), then 16 x 64 (768 x 64, K = 96: 4.5
+//     us, 10.6 at 64 x 128).
+//   16-bit modes (more per chunk to stage, so larger tiles pay): 128 x 128 from
+//     400 tiles on (57344 rows, K = 320, N = 256: 72 us, 75 at 64 x 128; 28672 x
+//     224: 33, 38), then 64 x 64 from 160 (4096, K = 512: 16 us, 41 at 128 x 128,
+//     17.5 at 32 x 64), then 32 x 64 from 200 and 16 x 64 below (500 rows, K =
+//     512: 9.6, 10.3 at 32 x 64, 40.7 at 128 x 128).
+template <int PREC>
+void plain_cfg(const GemmArgs& a, int* mb, int* nbw) {
+  const long nb = a.nbatch > 1 ? a.nbatch : 1;
+  auto tiles = [&](int r, int c) { return (long)ceil_div(a.rows, r) * ceil_div(a.ncols, c) * nb; };
+  constexpr bool f32 = PREC == PREC_F32;
+  *nbw = 1;
+  if (!f32 && tiles(128, 128) >= 400) {
+    *mb = 8;
+    *nbw = 2;
+  } else if (tiles(64, 64) >= (f32 ? 512 : 160)) {
+    *mb = 4;
+  } else {
+    *mb = tiles(32, 64) >= (f32 ? 256 : 200) ? 2 : 1;
+  }
+}
+
 template <int PREC>
 int dispatch(const GemmArgs& a, hipStream_t s) {
   const bool wide = a.ncols > 128;
   if (a.R <= 1) {
     if (a.Yln) return -1;
-    // two 128-column blocks share their X panel through the XCD's L2, which
-    // beats one 256-column block at a third of the occupancy.  Launches of
-    // fewer than two rounds of 128-row tiles over the CUs (the Metropolis
-    // forward pass, the per-walker broadcast GEMMs there) take 64-row tiles,
-    // so the last round is not a mostly idle tail.
-    const bool wide_tile = g_gemm_variant > 0 ? (g_gemm_variant % 10) == 4 : false;
-    const long tiles128 = (long)ceil_div(a.rows, 128) * ceil_div(a.ncols, 128) * (a.nbatch > 1 ? a.nbatch : 1);
-    if constexpr (PREC != PREC_F32) {  // no 256-column FP32 tiles (they spill)
-      if (wide_tile) {
-        launch_one<8, 1, 4, PREC, false>(a, s);
-        return 0;
-      }
+    int mb, nbw;
+    plain_cfg<PREC>(a, &mb, &nbw);
+    if (g_gemm_variant > 0) {
+      mb = g_gemm_variant / 10;
+      nbw = g_gemm_variant % 10;
     }
-    if (tiles128 < 2L * 3 * 256)
-      launch_one<4, 1, 2, PREC, false>(a, s);
-    else
-      launch_one<8, 1, 2, PREC, false>(a, s);
+    switch (10 * mb + nbw) {
+      case 82:
+        if constexpr (PREC == PREC_F32) return -1;
+        else launch_one<8, 1, 2, PREC, false>(a, s);
+        break;
+      case 41: launch_one<4, 1, 1, PREC, false>(a, s); break;
+      case 21: launch_one<2, 1, 1, PREC, false>(a, s); break;
+      case 11: launch_one<1, 1, 1, PREC, false>(a, s); break;
+      default: return -1;
+    }
     return 0;
   }
   int upt, nbw;

@@ -462,3 +462,28 @@ def test_psiformer_chunking_and_bf16x6(cuda):
     rel, bnd = el_report("psi_small B=8", oc["e_loc"].cpu().numpy(), ref["e_loc"], ref["kappa"], "bf16x6",
                          ref["cancel"])
     assert np.median(rel) < 2e-5 and np.all(rel <= bnd)
+
+
+# batches on every tile of the plain GEMM's table (16 to 128 rows, 64 and 128
+# columns; value rows of 14 electrons, 256-wide layers and 12 x 14 orbitals)
+@pytest.mark.parametrize("prec", ["fp32", "fp16x3"])
+def test_value_batches_are_bit_identical(cuda, prec):
+    """A walker's log|psi| does not depend on the batch it is evaluated in, so
+    neither on the tile that the batch's size selects."""
+    import torch
+
+    from jaqmc_amd import params as P
+    from jaqmc_amd import systems as S
+    from jaqmc_amd.device import DeviceModel
+
+    sysm, spec, *_ = S.workload("n2")
+    spec.ndets = 12
+    p = P.init_params(spec, seed=71, bias_scale=0.1, env_jitter=0.3)
+    x = torch.from_numpy(S.init_walkers(sysm, 4100, seed=72)).to(cuda)
+    dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, precision=prec)
+    lp, sign = dm.logpsi(x)
+    for n in (1, 7, 60, 333, 1201):
+        for at in (0, 4100 - n):
+            a, b = dm.logpsi(x[at:at + n].contiguous())
+            assert torch.equal(a, lp[at:at + n]) and torch.equal(b, sign[at:at + n]), (n, at)
+    dm.close()

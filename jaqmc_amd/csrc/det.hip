@@ -8,11 +8,12 @@
 // Laplacian mode restates laplacian/primitives/slogdet.py:44-59:
 //   d logdet / dx_c = tr(A^-1 J_c)
 //   lap logdet      = tr(A^-1 L) - sum_c tr((A^-1 J_c)^2)
-// with B_c = A^-1 J_c on FP64 MFMA.  Three kernels: det_small_kernel
-// (N <= 16, one wavefront per determinant), det_mfma_kernel (16 < N <= 64,
-// Laplacian mode, one workgroup per determinant) and det_fwd_reg_kernel
-// (16 < N <= 64, log|det| and sign only, one wavefront per determinant with
-// the matrix in registers).
+// with B_c = A^-1 J_c on FP64 MFMA.  Laplacian mode: det_small_kernel (N <= 16,
+// one wavefront per determinant) and det_mfma_kernel (16 < N <= 64, one
+// workgroup per determinant).  log|det| and sign only: det_fwd_col_kernel (N <=
+// 16, four determinants per wavefront, a column per lane) and
+// det_fwd_reg_kernel (16 < N <= 64, one wavefront per determinant, a row per
+// lane).
 
 #include <algorithm>
 #include <type_traits>
@@ -354,9 +355,78 @@ __global__ __launch_bounds__(256) void det_fwd_reg_kernel(FermiDims d, const flo
 }
 
 // ---------------------------------------------------------------------------
-// Small systems (N <= 16): one wavefront per determinant, four per workgroup,
-// no workgroup barriers.  The augmented [A | I] (16 x 32 FP64) is reduced by
-// Gauss-Jordan with partial pivoting in the wave's LDS slice; then, for each
+// Forward mode, N <= 16: log|det| and sign, four determinants per wavefront,
+// one in each 16-lane DPP row: lane j holds column j (NP >= N rows in
+// registers, padded with the identity).  Step p broadcasts column p from lane p
+// of each row (a DPP move, no LDS), every lane finds the pivot in it, exchanges
+// its own rows p and q and subtracts; the column loop is unrolled at compile
+// time.  Bound by VALU issue: 65536 matrices of 14 in 92 us, where a wavefront
+// per matrix, exchanging pivot rows and columns through LDS, took 228 (1024 of
+// 3: 4.2 us, 18.5).
+// ---------------------------------------------------------------------------
+template <int P, int NP>
+__device__ __forceinline__ void fwd_col_steps(double (&m)[NP], LogAbsProduct& logdet, int& neg) {
+  if constexpr (P < NP) {
+    double c[NP];
+#pragma unroll
+    for (int i = P; i < NP; ++i) c[i] = dpp_d<0x150 + P>(m[i]);  // row_newbcast:P
+    double best = fabs(c[P]), pv = c[P];
+    int q = P;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) {  // the first of the largest
+      const bool more = fabs(c[i]) > best;
+      best = more ? fabs(c[i]) : best;
+      pv = more ? c[i] : pv;
+      q = more ? i : q;
+    }
+    logdet.mul(pv);
+    neg ^= (pv < 0.0) != (q != P) ? 1 : 0;
+    const double mp = m[P], cp = c[P];
+    double r = mp;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) {
+      const bool sel = i == q;
+      r = sel ? m[i] : r;
+      m[i] = sel ? mp : m[i];
+      c[i] = sel ? cp : c[i];
+    }
+    r /= pv;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) m[i] = fma(-c[i], r, m[i]);
+    fwd_col_steps<P + 1, NP>(m, logdet, neg);
+  }
+}
+
+template <int NP>
+__global__ __launch_bounds__(256) void det_fwd_col_kernel(FermiDims d, const float* __restrict__ Phi, long ldphi,
+                                                          const float* __restrict__ env, double* __restrict__ out) {
+  const int j = threadIdx.x & 15;
+  const long total = (long)d.Bc * d.K;
+  const long det = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const long dc = det < total ? det : total - 1;  // every lane takes part in the moves
+  const int w = (int)(dc / d.K), k = (int)(dc % d.K), N = d.N;
+  double m[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    m[i] = i == j ? 1.0 : 0.0;
+    if (i < N && j < N)
+      m[i] = (double)Phi[(long)unit_idx(d, w, i) * d.Rp * ldphi + (long)k * N + j] *
+             (double)env_ptr(d, env, w, i, k, j)[0];
+  }
+  LogAbsProduct logdet;
+  int neg = 0;
+  fwd_col_steps<0, NP>(m, logdet, neg);
+  if (j == 0 && det < total) {
+    out[det * 3] = logdet.log_abs();
+    out[det * 3 + 1] = neg ? -1.0 : 1.0;
+    out[det * 3 + 2] = 0.0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Small systems (N <= 16), Laplacian mode: one wavefront per determinant, four
+// per workgroup, no workgroup barriers.  The augmented [A | I] (16 x 32 FP64) is
+// reduced by Gauss-Jordan with partial pivoting in registers; then, for each
 // coordinate c, B_c = A^-1 J_c is one 16x16 FP64 MFMA tile (four K steps,
 // A^-1 fragments in registers, J_c from HBM one coordinate pair ahead), with
 // tr(B_c) from the diagonal lanes and tr(B_c^2) from a transposed read of the
@@ -372,17 +442,9 @@ struct SmallDetSmem {
   double M[SM_NP * 2 * SM_NP];  // augmented matrix, later Inv in columns 16..31
   double Tt[2 * SM_NP * 17];    // transpose tiles of B_c, B_c+1 (odd row stride)
 };
-struct SmallFwdSmem {           // forward mode: the matrix and the pivot exchange area
-  double M[SM_NP * 2 * SM_NP];
-  double Tt[48];
-};
-
-template <bool LAPMODE>
 __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const float* __restrict__ Phi, long ldphi,
                                                         const float* __restrict__ env, double* __restrict__ out) {
-  constexpr bool lapmode = LAPMODE;
-  using Smem = typename std::conditional<LAPMODE, SmallDetSmem, SmallFwdSmem>::type;
-  __shared__ Smem smem[4];
+  __shared__ SmallDetSmem smem[4];
   const int N = d.N, T = 3 * N;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // determinants 4cb .. 4cb + 3 of walker w; a walker's blocks share an XCD
@@ -391,7 +453,7 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
   const int k = 4 * cb + wave;
   if (w >= d.Bc || k >= d.K) return;  // whole wave exits together
   const long det_id = (long)w * d.K + k;
-  Smem& S = smem[wave];
+  SmallDetSmem& S = smem[wave];
   const int Rp = d.Rp;
 
   // per-lane elements e = lane + 64 t, t = 0..3: (i, o) = (e / 16, e % 16)
@@ -412,11 +474,9 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
       const float* ep = env_ptr(d, env, w, i, k, o);
       phi0[t] = Phi[base[t]];
       e0[t] = ep[0];
-      if (lapmode) {
-        ej[t][0] = ep[2];
-        ej[t][1] = ep[3];
-        ej[t][2] = ep[4];
-      }
+      ej[t][0] = ep[2];
+      ej[t][1] = ep[3];
+      ej[t][2] = ep[4];
       a = (double)phi0[t] * (double)e0[t];
     }
     S.M[i * 32 + o] = a;
@@ -426,63 +486,6 @@ __global__ __launch_bounds__(256, 4) void det_small_kernel(FermiDims d, const fl
 
   LogAbsProduct logdet;
   int sgn = 1;
-  if constexpr (!lapmode) {
-    // forward mode needs only log|det| and the sign: LU without row
-    // exchanges with the 16x16 block in registers.  Lane (ti, tj) =
-    // (lane % 16, lane / 16) owns row ti, columns tj + 4b (b = 0..3); the
-    // pivot of column p is the unused row with the largest |entry| (DPP
-    // inside the 16-lane row that holds column p); the pivot row and column go
-    // through LDS and the rows not yet used are updated right of column p.
-    // The parity of the row order enters the sign.
-    const int ti = lane & 15, tj = lane >> 4;
-    double x[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) x[b] = S.M[ti * 32 + tj + 4 * b];
-    bool used = false;
-    double* prow = S.Tt;       // 16 doubles
-    double* pcol = S.Tt + 16;  // 16 doubles
-    int* perm = (int*)(S.Tt + 32);
-    for (int p = 0; p < SM_NP; ++p) {
-      const int pb = p >> 2, pr = p & 3;
-      double xp = 0.0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if (b == pb) xp = x[b];
-      double v = used ? -1.0 : fabs(xp);
-      int bi = used ? SM_NP : ti;
-      gj_pick16(v, bi);
-      int q = __builtin_amdgcn_readlane(bi, 16 * pr);
-      if (q >= SM_NP) q = 0;  // unreachable: an unused row always remains
-      const double piv = readlane_d(xp, 16 * pr + q);
-      logdet.mul(piv);
-      if (piv < 0) sgn = -sgn;
-      if (lane == 0) perm[p] = q;
-      if (ti == q) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) prow[tj + 4 * b] = x[b];
-      }
-      if (tj == pr) pcol[ti] = xp;
-      wave_sync();
-      const double rp = 1.0 / piv;
-      if (ti == q) {
-        used = true;
-      } else if (!used) {
-        const double f = pcol[ti] * rp;
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          if (tj + 4 * b > p) x[b] -= f * prow[tj + 4 * b];
-      }
-      wave_sync();
-    }
-    if (lane == 0) {
-      sgn *= perm_sign(perm, SM_NP);
-      double* o_ = out + det_id * 3;
-      o_[0] = logdet.log_abs();
-      o_[1] = (double)sgn;
-      o_[2] = 0.0;
-    }
-    return;
-  }
   // Gauss-Jordan on [A | I] with the matrix in registers (gauss_jordan.h)
   {
     const int ti = lane & 15, tj = lane >> 4;
@@ -781,11 +784,20 @@ int launch_orbital_export(const FermiDims& d, const float* Phi, long ldphi, cons
 
 int launch_det(const FermiDims& d, const float* Phi, long ldphi, const float* env, double* out, hipStream_t s) {
   if (d.N <= SM_NP) {
-    const dim3 grid((unsigned)xcd_grid(d.Bc, (d.K + 3) / 4));
-    if (d.Rp > 1)
-      hipLaunchKernelGGL(det_small_kernel<true>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
+    if (d.Rp > 1) {
+      const dim3 grid((unsigned)xcd_grid(d.Bc, (d.K + 3) / 4));
+      hipLaunchKernelGGL(det_small_kernel, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
+      return 0;
+    }
+    const dim3 grid((unsigned)ceil_div((long)d.Bc * d.K, 16));
+    if (d.N <= 4)
+      hipLaunchKernelGGL(det_fwd_col_kernel<4>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
+    else if (d.N <= 8)
+      hipLaunchKernelGGL(det_fwd_col_kernel<8>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
+    else if (d.N <= 12)
+      hipLaunchKernelGGL(det_fwd_col_kernel<12>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
     else
-      hipLaunchKernelGGL(det_small_kernel<false>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
+      hipLaunchKernelGGL(det_fwd_col_kernel<16>, grid, dim3(256), 0, s, d, Phi, ldphi, env, out);
     return 0;
   }
   if (d.Rp > 1 && d.N <= 64) {

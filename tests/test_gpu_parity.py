@@ -487,3 +487,31 @@ def test_value_batches_are_bit_identical(cuda, prec):
             a, b = dm.logpsi(x[at:at + n].contiguous())
             assert torch.equal(a, lp[at:at + n]) and torch.equal(b, sign[at:at + n]), (n, at)
     dm.close()
+
+
+# the padded sizes 4, 8, 12 and 16 of the column-per-lane kernel, full and not
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 8, 9, 12, 13, 16])
+def test_forward_logdet_small_sizes(cuda, n):
+    """As test_forward_logdet_every_padded_size, for up to 16 electrons (seven
+    matrices: the last group of sixteen is not full)."""
+    import torch
+
+    sysm = S.h_chain(n)
+    _, spec, *_ = S.workload("li")
+    spec.nspins = sysm.nspins
+    spec.n_atoms = n
+    spec.hidden_single, spec.hidden_double, spec.ndets = [32, 32], [8, 8], 1
+    p = P.init_params(spec, seed=5, bias_scale=0.1, env_jitter=0.2)
+    x = S.init_walkers(sysm, 7, seed=6)
+    p64 = P.cast_params(p, np.float64)
+    at = sysm.atoms.astype(np.float64)
+    sg_ref, lp_ref = owf.logpsi(spec.as_oracle(), p64, x.astype(np.float64), at, with_laplacian=False)
+    A = np.asarray(owf.orbital_matrices(spec.as_oracle(), p64, x.astype(np.float64), at))
+    kappa = np.linalg.cond(A).reshape(x.shape[0], -1).max(axis=1)
+    dm = _model(sysm, spec, p)
+    lp, sg = dm.logpsi(torch.from_numpy(x).to(cuda))
+    torch.cuda.synchronize()
+    d = np.abs(lp.cpu().numpy() - lp_ref.v)
+    assert np.all(d <= logpsi_bound(lp_ref.v, kappa, "fp32")), (d, kappa)
+    np.testing.assert_array_equal(sg.cpu().numpy(), np.asarray(sg_ref).reshape(-1))
+    dm.close()

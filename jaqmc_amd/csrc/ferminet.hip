@@ -72,6 +72,19 @@ __global__ __launch_bounds__(256) void ae_features_kernel(FermiDims d, const flo
   }
 }
 
+// Forward mode (value rows only): a thread per nucleus of a unit.
+__global__ __launch_bounds__(256) void ae_features_fwd_kernel(FermiDims d, const float* __restrict__ elec,
+                                                              const float* __restrict__ atoms, float* __restrict__ X,
+                                                              long ldx) {
+  const long t = blockIdx.x * 256L + threadIdx.x;
+  if (t >= (long)d.Bc * d.N * d.M) return;
+  const int u = (int)(t / d.M), I = (int)(t % d.M);
+  const int w = walker_of_unit(u, d.Bc, d.n_up, d.n_dn), i = elec_of_unit(u, d.Bc, d.n_up, d.n_dn);
+  const float* xi = elec + ((long)w * d.N + i) * 3;
+  const float dx = xi[0] - atoms[3 * I], dy = xi[1] - atoms[3 * I + 1], dz = xi[2] - atoms[3 * I + 2];
+  *(float4*)(X + (long)u * ldx + 4 * I) = float4{sqrtf(dx * dx + dy * dy + dz * dz), dx, dy, dz};
+}
+
 // Pair-stream input, H2[w][a][b][row][4], RP2 = 8 rows (Laplacian) or 1.
 __global__ void ee_features_kernel(FermiDims d, int RP2, const float* __restrict__ elec, float* __restrict__ H2) {
   const long total = (long)d.Bc * d.N * d.N;
@@ -345,11 +358,62 @@ __global__ void pair_layer_generic_kernel(long npairs, const float* __restrict__
 // channel s, m_s[i] = mean_{j in s} h2[j][i].  Expanded to dense rows:
 //   d/dx_i   <- mean_j (d/dx_b rows of pair (j, i))
 //   d/dx_j   <- (d/dx_a rows of pair (j, i)) / n_s,   j in s
-// One workgroup per (walker, electron) stages the column H2[w][:, i] in LDS
-// and writes the unit's whole block X[unit][0:Rp][col0:ldx) row by row;
-// columns past nch*f2 are zero-filled (GEMM K padding).  NTH threads: 1024
-// when the staged column is large enough to leave room for few workgroups
-// per CU (large N), else 256.
+// From the column of one (walker, electron) in LDS, feature f of row RP2 j + t at
+// col[at(RP2 j + t, f)] (part: LDS for the sums), the workgroup of NTH threads writes the unit's whole block
+// X[unit][0:Rp][col0:ldx) row by row; columns past nch*f2 are zero-filled (GEMM
+// K padding).  Called with the column complete (behind a barrier).
+struct ColRows {
+  int f2;
+  __device__ int operator()(int row, int f) const { return row * f2 + f; }
+};
+template <typename T, int NTH, typename At>
+__device__ inline void pair_means_rows(const FermiDims& d, int RP2, int w, int i, const float* col, At at, float* part,
+                                       int f2, T* __restrict__ X, long ldx, int col0) {
+  const int tid = threadIdx.x;
+  const int nrow_sum = RP2 > 1 ? 5 : 1;
+  for (int idx = tid; idx < d.nch * nrow_sum * f2; idx += NTH) {
+    const int s = idx / (nrow_sum * f2), q = (idx / f2) % nrow_sum, f = idx % f2;
+    const int j0 = d.nch == 1 ? 0 : (s == 0 ? 0 : d.n_up);
+    const int ns = d.nch == 1 ? d.N : (s == 0 ? d.n_up : d.n_dn);
+    const int row = q < 2 ? q : 5 + (q - 2);  // value, lap, d/dx_b (rows 5..7)
+    float acc = 0.f;
+    for (int j = j0; j < j0 + ns; ++j) acc += col[at(j * RP2 + row, f)];
+    part[(s * 5 + q) * f2 + f] = acc / ns;
+  }
+  __syncthreads();
+  const int u = unit_of(w, i, d.Bc, d.n_up, d.n_dn);
+  const int ncol = (int)(ldx - col0);
+  T* xu = X + (long)u * d.Rp * ldx + col0;
+  // lanes walk columns (per-column constants hoisted), the waves walk rows
+  for (int cc = tid & 63; cc < ncol; cc += 64) {
+    const bool live = cc < d.nch * f2;
+    const int s = live ? cc / f2 : 0, f = live ? cc - s * f2 : 0;
+    const int j0 = d.nch == 1 ? 0 : (s == 0 ? 0 : d.n_up);
+    const int ns = d.nch == 1 ? d.N : (s == 0 ? d.n_up : d.n_dn);
+    const float inv = 1.f / ns;
+    for (int r = tid >> 6; r < d.Rp; r += NTH / 64) {
+      float out = 0.f;
+      if (live) {
+        if (r == ROW_VAL || r == ROW_LAP) {
+          out = part[(s * 5 + r) * f2 + f];
+        } else if (r - ROW_J0 < 3 * d.N) {
+          const int c = r - ROW_J0;
+          const int e = c / 3, ax = c - 3 * e;
+          if (e == i)
+            out = part[(s * 5 + 2 + ax) * f2 + f];
+          else if (e >= j0 && e < j0 + ns)
+            out = col[at(e * RP2 + 2 + ax, f)] * inv;
+        }
+      }
+      xu[(long)r * ldx + cc] = from_f<T>(out);
+    }
+  }
+}
+
+// The means from a pair stream in HBM: one workgroup per (walker, electron)
+// stages the column H2[w][:, i] in LDS.  NTH threads: 1024 when the staged
+// column is large enough to leave room for few workgroups per CU (large N),
+// else 256.
 template <typename T, int NTH>
 __global__ __launch_bounds__(NTH) void pair_means_kernel(FermiDims d, int RP2, const float* __restrict__ H2, int f2,
                                                          T* __restrict__ X, long ldx, int col0) {
@@ -375,43 +439,207 @@ __global__ __launch_bounds__(NTH) void pair_means_kernel(FermiDims d, int RP2, c
     }
   }
   __syncthreads();
-  const int nrow_sum = RP2 > 1 ? 5 : 1;
-  for (int idx = tid; idx < d.nch * nrow_sum * f2; idx += NTH) {
-    const int s = idx / (nrow_sum * f2), q = (idx / f2) % nrow_sum, f = idx % f2;
-    const int j0 = d.nch == 1 ? 0 : (s == 0 ? 0 : d.n_up);
-    const int ns = d.nch == 1 ? d.N : (s == 0 ? d.n_up : d.n_dn);
-    const int row = q < 2 ? q : 5 + (q - 2);  // value, lap, d/dx_b (rows 5..7)
-    float acc = 0.f;
-    for (int j = j0; j < j0 + ns; ++j) acc += col[(j * RP2 + row) * f2 + f];
-    part[(s * 5 + q) * f2 + f] = acc / ns;
-  }
-  __syncthreads();
-  const int u = unit_of(w, i, d.Bc, d.n_up, d.n_dn);
-  const int ncol = (int)(ldx - col0);
-  T* xu = X + (long)u * d.Rp * ldx + col0;
-  // lanes walk columns (per-column constants hoisted), the waves walk rows
-  for (int cc = tid & 63; cc < ncol; cc += 64) {
-    const bool live = cc < d.nch * f2;
-    const int s = live ? cc / f2 : 0, f = live ? cc - s * f2 : 0;
-    const int j0 = d.nch == 1 ? 0 : (s == 0 ? 0 : d.n_up);
-    const int ns = d.nch == 1 ? d.N : (s == 0 ? d.n_up : d.n_dn);
-    const float inv = 1.f / ns;
-    for (int r = tid >> 6; r < d.Rp; r += NTH / 64) {
-      float out = 0.f;
-      if (live) {
-        if (r == ROW_VAL || r == ROW_LAP) {
-          out = part[(s * 5 + r) * f2 + f];
-        } else if (r - ROW_J0 < 3 * d.N) {
-          const int c = r - ROW_J0;
-          const int e = c / 3, ax = c - 3 * e;
-          if (e == i)
-            out = part[(s * 5 + 2 + ax) * f2 + f];
-          else if (e >= j0 && e < j0 + ns)
-            out = col[(e * RP2 + 2 + ax) * f2 + f] * inv;
-        }
-      }
-      xu[(long)r * ldx + cc] = from_f<T>(out);
+  pair_means_rows<T, NTH>(d, RP2, w, i, col, ColRows{f2}, part, f2, X, ldx, col0);
+}
+
+// ---------------------------------------------------------------------------
+// The 32-wide two-electron stream on chip.  h2[j][i] passes through its layers
+// pair by pair (FermiLayers._update_double_stream, ferminet.py:57-63) and only
+// its means reach the one-electron stream, so a workgroup forms the pairs of its
+// electrons from their positions, runs the layers on them in LDS and writes the
+// means of layers L0 and, with TWO, L0 + 1: the stream never goes to HBM.  The
+// layer inputs X alternate between two buffers, so layers 0, 1 and then 2, 3 are
+// served by one launch each; the second repeats the first's layer (4 -> 32),
+// a third more products than one pass, for three passes over 1 KB per pair less.
+// Laplacian mode: one workgroup per (walker, electron i), rows 8 j + t; forward
+// mode: one per walker and as many electrons as 48 KB hold, rows (i - i0) N + j.
+// A wavefront takes 16 rows at a time through the layers on
+// v_mfma_f32_16x16x4f32 (operand layouts of pair_layer32_mfma_kernel, whose
+// products, rule and residual it repeats bit for bit); between layers the rows
+// turn through their own place in LDS (ps_at).  Bound by the tanh of the values
+// and the write of the dense mean rows.  N2, 4096 walkers: features, layers and
+// means 2.2 -> 1.3 ms per Laplacian pass, 258 -> 169 us per value pass; 60
+// electrons, 384 walkers: 3.6 -> 2.4 ms.
+// ---------------------------------------------------------------------------
+constexpr int PS_LAYERS = 3;  // layers of the stream at most
+struct PairStream {
+  const float* W[PS_LAYERS];
+  const float* b[PS_LAYERS];
+  float* X[2];  // where the means of layers L0 and L0 + 1 go: columns col0 .. ldx of X
+  long ldx[2];
+  int col0[2];
+};
+// Entry c of row r of the stream in LDS: the 16-byte groups of a row are
+// permuted by the row, so that 8 rows' equal groups lie on distinct banks.
+__device__ inline int ps_at(int r, int c) { return r * 32 + (((c >> 2) ^ (r & 7)) << 2) + (c & 3); }
+struct ColSwizzled {
+  __device__ int operator()(int row, int f) const { return ps_at(row, f); }
+};
+
+// Feature f of tangent row t of the pair (j, i) at displacement x_j - x_i.
+template <int RP2>
+__device__ inline float pair_feature(int t, int f, float dx, float dy, float dz, bool same) {
+  if (same) return 0.f;
+  const float rr = sqrtf(dx * dx + dy * dy + dz * dz);
+  if (RP2 == 1 || t == 0) return f == 0 ? rr : (f == 1 ? dx : (f == 2 ? dy : dz));
+  if (t == 1) return f == 0 ? 4.f / rr : 0.f;
+  const int ax = t < 5 ? t - 2 : t - 5;
+  const float dv = ax == 0 ? dx : (ax == 1 ? dy : dz);
+  const float v = f == 0 ? dv / rr : (f - 1 == ax ? 1.f : 0.f);
+  return t < 5 ? v : -v;
+}
+
+// tanh rule of 16 rows x 16 columns in the MFMA layout (pair_layer32_mfma_kernel)
+template <int RP2>
+__device__ inline void pair_tanh(f32x4 acc, float bv, int lane, float (&o)[4]) {
+  const int g = lane >> 4;
+  if constexpr (RP2 == 8) {
+    const bool lo = (g & 1) == 0;  // rows 0..3 of the pair (value, Laplacian, first Jacobian rows)
+    if (lo) acc[0] += bv;
+    float sq = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (!lo || v >= 2) sq += acc[v] * acc[v];
+    sq += __shfl_xor(sq, 16);
+    const float y0 = __shfl(acc[0], lane & ~16);
+    const float t = tanhf(y0);
+    const float d1 = 1.f - t * t;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = d1 * acc[v];
+    if (lo) {
+      o[0] = t;
+      o[1] = d1 * acc[1] - 2.f * t * d1 * sq;
     }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = tanhf(acc[v] + bv);
+  }
+}
+
+// Layers LB .. LE - 1 of rows row0 .. row0 + 15 of the workgroup's pairs, in
+// place in col (rows past nrows up to the 16th hold nothing); the input is
+// feature(row, f) for LB = 0, else the rows in col.
+template <int RP2, int LB, int LE, typename F>
+__device__ inline void pair_stream_block(const PairStream& a, const F& feature, int row0, int nrows, float* col) {
+  float* const tile = col + row0 * 32;  // row0 is a multiple of 8: ps_at takes the row in the tile
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  float prev[2][4];  // the layer's input, in the layout of its output
+#pragma unroll
+  for (int l = LB; l < LE; ++l) {
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    if (l == 0) {
+      const float xa = feature(row0 + r < nrows ? row0 + r : nrows - 1, g);
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, a.W[0][g * 32 + 16 * nb + r], acc[nb], 0, 0, 0);
+    } else {
+      const f32x4 x0 = *(const f32x4*)&tile[ps_at(r, 8 * g)], x1 = *(const f32x4*)&tile[ps_at(r, 8 * g + 4)];
+      if (l == LB) {
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) prev[nb][v] = tile[ps_at(4 * g + v, 16 * nb + r)];
+      }
+      wave_sync();  // the rows are read; the layer overwrites them
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk < 4 ? x0[kk & 3] : x1[kk & 3],
+                                                         a.W[l][(8 * g + kk) * 32 + 16 * nb + r], acc[nb], 0, 0, 0);
+    }
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const int c = 16 * nb + r;
+      float o[4];
+      pair_tanh<RP2>(acc[nb], a.b[l][c], lane, o);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (l > 0) o[v] = (o[v] + prev[nb][v]) * 0.70710678118654752f;  // 32 -> 32: residual
+        prev[nb][v] = o[v];
+        tile[ps_at(4 * g + v, c)] = o[v];
+      }
+    }
+    wave_sync();
+  }
+}
+
+template <int L0, bool TWO, int NTH>
+__global__ __launch_bounds__(NTH) void pair_stream_lap_kernel(FermiDims d, PairStream a, const float* __restrict__ elec) {
+  extern __shared__ __attribute__((aligned(16))) float psm[];
+  float* col = psm;                   // rows 8 j + t
+  float* part = col + d.N * 8 * 32;   // [s][5][32], also the last block's rows past 8 N
+  const int w = blockIdx.x / d.N, i = blockIdx.x % d.N;
+  const float* xw = elec + (long)w * d.N * 3;
+  const float xi = xw[3 * i], yi = xw[3 * i + 1], zi = xw[3 * i + 2];
+  const int nrows = 8 * d.N, first = 16 * (threadIdx.x >> 6);
+  auto feature = [&](int row, int f) __attribute__((always_inline)) {
+    const int j = row >> 3;
+    return pair_feature<8>(row & 7, f, xw[3 * j] - xi, xw[3 * j + 1] - yi, xw[3 * j + 2] - zi, j == i);
+  };
+  if constexpr (L0 == 0) {
+    for (int e = threadIdx.x; e < nrows * 4; e += NTH) col[e] = feature(e >> 2, e & 3);
+    __syncthreads();
+    pair_means_rows<float, NTH>(d, 8, w, i, col, ColRows{4}, part, 4, a.X[0], a.ldx[0], a.col0[0]);
+  } else {
+    for (int row0 = first; row0 < nrows; row0 += 16 * (NTH / 64))
+      pair_stream_block<8, 0, L0>(a, feature, row0, nrows, col);
+    __syncthreads();
+    pair_means_rows<float, NTH>(d, 8, w, i, col, ColSwizzled(), part, 32, a.X[0], a.ldx[0], a.col0[0]);
+  }
+  if constexpr (TWO) {
+    __syncthreads();
+    for (int row0 = first; row0 < nrows; row0 += 16 * (NTH / 64))
+      pair_stream_block<8, L0, L0 + 1>(a, feature, row0, nrows, col);
+    __syncthreads();
+    pair_means_rows<float, NTH>(d, 8, w, i, col, ColSwizzled(), part, 32, a.X[1], a.ldx[1], a.col0[1]);
+  }
+}
+
+template <int L0, bool TWO>
+__global__ __launch_bounds__(256) void pair_stream_fwd_kernel(FermiDims d, PairStream a, int ni,
+                                                              const float* __restrict__ elec) {
+  extern __shared__ __attribute__((aligned(16))) float psm[];
+  float* col = psm;  // rows (i - i0) N + j, and the last block's rows past n N
+  const int w = blockIdx.x, i0 = blockIdx.y * ni, N = d.N;
+  const int n = N - i0 < ni ? N - i0 : ni, nrows = n * N, first = 16 * (threadIdx.x >> 6);
+  const float* xw = elec + (long)w * N * 3;
+  auto feature = [&](int row, int f) __attribute__((always_inline)) {
+    const int j = row % N, i = i0 + row / N;
+    return pair_feature<1>(0, f, xw[3 * j] - xw[3 * i], xw[3 * j + 1] - xw[3 * i + 1], xw[3 * j + 2] - xw[3 * i + 2],
+                           j == i);
+  };
+  // thread per output column of a unit, summed in j order (pair_means_fwd_kernel)
+  auto means = [&](auto at, int f2, int q) __attribute__((always_inline)) {
+    const int ncol = (int)(a.ldx[q] - a.col0[q]);
+    for (int e = threadIdx.x; e < n * ncol; e += 256) {
+      const int ii = e / ncol, cc = e % ncol;
+      float out = 0.f;
+      if (cc < d.nch * f2) {
+        const int s = cc / f2, f = cc % f2;
+        const int j0 = d.nch == 1 ? 0 : (s == 0 ? 0 : d.n_up);
+        const int ns = d.nch == 1 ? N : (s == 0 ? d.n_up : d.n_dn);
+        float acc = 0.f;
+        for (int j = j0; j < j0 + ns; ++j) acc += col[at(ii * N + j, f)];
+        out = acc / ns;
+      }
+      a.X[q][(long)unit_of(w, i0 + ii, d.Bc, d.n_up, d.n_dn) * a.ldx[q] + a.col0[q] + cc] = out;
+    }
+  };
+  if constexpr (L0 == 0) {
+    for (int e = threadIdx.x; e < nrows * 4; e += 256) col[e] = feature(e >> 2, e & 3);
+    __syncthreads();
+    means(ColRows{4}, 4, 0);
+  } else {
+    for (int row0 = first; row0 < nrows; row0 += 64) pair_stream_block<1, 0, L0>(a, feature, row0, nrows, col);
+    __syncthreads();
+    means(ColSwizzled(), 32, 0);
+  }
+  if constexpr (TWO) {
+    __syncthreads();
+    for (int row0 = first; row0 < nrows; row0 += 64) pair_stream_block<1, L0, L0 + 1>(a, feature, row0, nrows, col);
+    __syncthreads();
+    means(ColSwizzled(), 32, 1);
   }
 }
 
@@ -609,15 +837,74 @@ int launch_ferminet_features(const FermiDims& d, const float* elec, const float*
                              bool x_bf16, float* H2, hipStream_t s) {
   const unsigned units = (unsigned)(d.Bc * d.N);
   const size_t smem = (size_t)4 * d.M * sizeof(float);
-  if (units > 0 && smem <= 64 * 1024) {
+  if (units > 0 && d.Rp <= 1 && !x_bf16 && ldx % 4 == 0) {
+    hipLaunchKernelGGL(ae_features_fwd_kernel, dim3(ceil_div((long)units * d.M, 256)), dim3(256), 0, s, d, elec, atoms,
+                       (float*)X, ldx);
+  } else if (units > 0 && smem <= 64 * 1024) {
     if (x_bf16)
       hipLaunchKernelGGL(ae_features_kernel<bf16>, dim3(units), 256, smem, s, d, elec, atoms, (bf16*)X, ldx);
     else
       hipLaunchKernelGGL(ae_features_kernel<float>, dim3(units), 256, smem, s, d, elec, atoms, (float*)X, ldx);
   }
+  if (!H2) return 0;
   const long t2 = (long)d.Bc * d.N * d.N;
   hipLaunchKernelGGL(ee_features_kernel, grid_for(t2), 256, 0, s, d, d.Rp > 1 ? 8 : 1, elec, H2);
   return 0;
+}
+
+bool pair_stream_supported(int layers, const int* width) {
+  if (layers > PS_LAYERS) return false;
+  for (int l = 0; l < layers; ++l)
+    if (width[l] != 32) return false;
+  return true;  // N <= 63: 63 x 1 KB of pairs fit 65 KB
+}
+
+template <int L0, bool TWO>
+static int pair_stream_launch(const FermiDims& d, const PairStream& a, const float* elec, hipStream_t s) {
+  if (d.Rp <= 1) {
+    int ni = 48 * 1024 / (d.N * 32 * 4);
+    ni = ni < 1 ? 1 : (ni > d.N ? d.N : ni);
+    const size_t smem = (size_t)(ni * d.N + 15) * 32 * 4;
+    if (smem > 64 * 1024) return -1;
+    hipLaunchKernelGGL((pair_stream_fwd_kernel<L0, TWO>), dim3(d.Bc, (d.N + ni - 1) / ni), dim3(256), smem, s, d, a,
+                       ni, elec);
+    return 0;
+  }
+  const size_t smem = ((size_t)d.N * 8 * 32 + 2 * 5 * 32) * 4;
+  static_assert(2 * 5 * 32 >= 8 * 32, "rows past 8 N lie in the sums' place");
+  const dim3 grid((unsigned)((long)d.Bc * d.N));
+  // four waves while four workgroups fit a CU, eight beyond
+  if (smem <= 40 * 1024) {
+    hipLaunchKernelGGL((pair_stream_lap_kernel<L0, TWO, 256>), grid, dim3(256), smem, s, d, a, elec);
+  } else {
+    static const hipError_t attr = hipFuncSetAttribute((const void*)pair_stream_lap_kernel<L0, TWO, 512>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    if (attr != hipSuccess || smem > 80 * 1024) return -1;
+    hipLaunchKernelGGL((pair_stream_lap_kernel<L0, TWO, 512>), grid, dim3(512), smem, s, d, a, elec);
+  }
+  return 0;
+}
+
+int launch_pair_stream(const FermiDims& d, int l0, bool two, const float* const* W, const float* const* b,
+                       const float* elec, float* const* X, const long* ldx, const int* col0, hipStream_t s) {
+  if ((long)d.Bc * d.N <= 0) return 0;
+  PairStream a{};
+  for (int l = 0; l < l0 + (two ? 1 : 0) && l < PS_LAYERS; ++l) {
+    a.W[l] = W[l];
+    a.b[l] = b[l];
+  }
+  for (int q = 0; q < (two ? 2 : 1); ++q) {
+    a.X[q] = X[q];
+    a.ldx[q] = ldx[q];
+    a.col0[q] = col0[q];
+  }
+  switch (2 * l0 + (two ? 1 : 0)) {
+    case 0: return pair_stream_launch<0, false>(d, a, elec, s);
+    case 1: return pair_stream_launch<0, true>(d, a, elec, s);
+    case 4: return pair_stream_launch<2, false>(d, a, elec, s);
+    case 5: return pair_stream_launch<2, true>(d, a, elec, s);
+  }
+  return -1;
 }
 
 template <int RP2>

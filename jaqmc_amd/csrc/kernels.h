@@ -97,8 +97,9 @@ __host__ __device__ inline int unit_idx(const FermiDims& d, int w, int i) {
 // Laplacian and gradient in Laplacian mode (Rp > 1), the value alone in
 // forward mode.
 __host__ __device__ inline int env_stride(const FermiDims& d) { return d.Rp > 1 ? 5 : 1; }
-// Layer-0 one-electron input (ae features) into X[:, :, 0:4M] and the pair
-// stream input H2 (RP2 rows per pair: 8 in Laplacian mode, 1 in forward mode).
+// Layer-0 one-electron input (ae features) into X[:, :, 0:4M] and, unless H2 is
+// null, the pair stream input H2 (RP2 rows per pair: 8 in Laplacian mode, 1 in
+// forward mode).
 int launch_ferminet_features(const FermiDims& d, const float* elec, const float* atoms,
                              void* X, long ldx, bool x_bf16, float* H2, hipStream_t s);
 // One pair-stream layer: H2out = tanh(H2in W + b) (+ residual).
@@ -108,6 +109,13 @@ int launch_pair_layer(const FermiDims& d, const float* H2in, int fin, float* H2o
 // tangent rows, written into X[:, :, col0 : col0 + nch*f2].
 int launch_pair_means(const FermiDims& d, const float* H2, int f2, void* X, long ldx, int col0,
                       bool x_bf16, hipStream_t s);
+// The same means of the pair stream after l0 layers (l0 = 0 or 2), and with
+// `two` also after l0 + 1, formed on chip from the positions: into columns
+// col0[q] .. ldx[q] of X[q], nch*4 columns for no layers, else nch*32 (weights
+// W[l], biases b[l] of the layers; every width 32, see pair_stream_supported).
+bool pair_stream_supported(int layers, const int* width);
+int launch_pair_stream(const FermiDims& d, int l0, bool two, const float* const* W, const float* const* b,
+                       const float* elec, float* const* X, const long* ldx, const int* col0, hipStream_t s);
 // Spin-channel means of X[:, :, 0:f1] -> g[walker, r, ch*f1 + f]  (ldg row stride).
 int launch_spin_means(const FermiDims& d, const void* X, long ldx, int f1, void* g, long ldg,
                       bool bf16io, hipStream_t s);

@@ -94,6 +94,7 @@ struct jq_model {
 
   // FermiNet
   std::vector<FermiLayer> fl;
+  bool pairs_on_chip = false;  // launch_pair_stream instead of a pair stream in H2
   // Psiformer
   std::vector<PsiLayer> pl;
   int D = 0, H = 0, dh = 0, kin = 0;  // model dim, heads, head dim, padded input K

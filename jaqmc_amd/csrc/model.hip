@@ -222,9 +222,15 @@ int jq_model::init_ferminet(const float* packed, size_t n_floats) {
   }
   kx = std::max(kx, (size_t)korb);
   ldphi = round_up(K * N, 4);
+  {
+    int widths[JQ_MAX_LAYERS];
+    for (int l = 0; l + 1 < L; ++l) widths[l] = fl[l].d2;
+    pairs_on_chip = !xbf && pair_stream_supported(L - 1, widths);
+  }
+  const size_t pair_streams = pairs_on_chip ? 0 : 2;
   auto per_walker = [&](int R, int RP2) {
     return 2 * (size_t)N * R * kx * es() + (size_t)R * kgm * es() + (size_t)R * d1m * 4 +
-           2 * (size_t)N * N * RP2 * f2m * 4 + (size_t)N * R * ldphi * 4 + (size_t)N * K * N * 5 * 4 +
+           pair_streams * (size_t)N * N * RP2 * f2m * 4 + (size_t)N * R * ldphi * 4 + (size_t)N * K * N * 5 * 4 +
            (size_t)K * (3 + T) * 8 + 64;
   };
   const size_t pw_lap = per_walker(Rp, 8), pw_fwd = per_walker(1, 1);
@@ -242,12 +248,11 @@ int jq_model::init_ferminet(const float* packed, size_t n_floats) {
   X[1] = alloc(nX * es());
   g = alloc(ng * es());
   G = (float*)alloc(nG * 4);
-  H2[0] = (float*)alloc(nH * 4);
-  H2[1] = (float*)alloc(nH * 4);
+  for (size_t i = 0; i < pair_streams; ++i) H2[i] = (float*)alloc(nH * 4);
   Phi = (float*)alloc(nP * 4);
   env = (float*)alloc(nE * 4);
   det = (double*)alloc(nD * 8);
-  if (!X[0] || !X[1] || !g || !G || !H2[0] || !H2[1] || !Phi || !env || !det)
+  if (!X[0] || !X[1] || !g || !G || (pair_streams && (!H2[0] || !H2[1])) || !Phi || !env || !det)
     return jq_fail(JQ_ENOMEM, "workspace allocation failed");
   rc = alloc_mh_scratch();
   if (!rc && grads) rc = alloc_grad_workspace(4ull << 30);
@@ -270,9 +275,25 @@ int jq_model::forward_ferminet(const float* elec, int Bc, bool lap, hipStream_t 
   void* Xn = X[1];
   int rc = launch_ferminet_features(fd, elec, atoms, Xc, fl[0].kmain, xbf, H2[0], s);
   int hc = 0;
+  const float *W2[JQ_MAX_LAYERS] = {}, *b2[JQ_MAX_LAYERS] = {};
+  for (int l = 0; l < L; ++l) {
+    W2[l] = fl[l].W2;
+    b2[l] = fl[l].b2;
+  }
   for (int l = 0; l < L && !rc; ++l) {
     const FermiLayer& ly = fl[l];
-    rc = launch_pair_means(fd, H2[hc], ly.f2, Xc, ly.kmain, ly.f1, xbf, s);
+    if (pairs_on_chip) {
+      if (l % 2 == 0) {  // this layer's means and the next one's, whose input is Xn
+        const bool two = l + 1 < L;
+        float* const px[2] = {(float*)Xc, (float*)Xn};
+        const long pld[2] = {ly.kmain, two ? fl[l + 1].kmain : 0};
+        const int pc[2] = {ly.f1, two ? fl[l + 1].f1 : 0};
+        ProfScope ps(lap ? PROF_PAIR_LAP : -1, s);
+        rc = launch_pair_stream(fd, l, two, W2, b2, elec, px, pld, pc, s);
+      }
+    } else {
+      rc = launch_pair_means(fd, H2[hc], ly.f2, Xc, ly.kmain, ly.f1, xbf, s);
+    }
     if (!rc) rc = launch_spin_means(fd, Xc, ly.kmain, ly.f1, g, ly.kg, xbf, s);
     if (rc) break;
     GemmArgs ga{};
@@ -321,7 +342,7 @@ int jq_model::forward_ferminet(const float* elec, int Bc, bool lap, hipStream_t 
       rc = launch_gemm(gm, prec, xbf, s);
     }
     if (rc) return jq_fail(JQ_EINVAL, "layer GEMM launch rejected");
-    if (ly.has_pair) {
+    if (ly.has_pair && !pairs_on_chip) {
       ProfScope ps(lap ? PROF_PAIR_LAP : -1, s);
       rc = launch_pair_layer(fd, H2[hc], ly.f2, H2[hc ^ 1], ly.d2, ly.W2, ly.b2, ly.res2, s);
       hc ^= 1;

@@ -515,3 +515,43 @@ def test_forward_logdet_small_sizes(cuda, n):
     assert np.all(d <= logpsi_bound(lp_ref.v, kappa, "fp32")), (d, kappa)
     np.testing.assert_array_equal(sg.cpu().numpy(), np.asarray(sg_ref).reshape(-1))
     dm.close()
+
+
+# the on-chip pair stream (every pair width 32): no, one, two and three layers,
+# one electron, one spin channel, ragged 16-row blocks, eight-wave workgroups
+PAIR_CASES = {
+    "h5_1": (lambda: S.h_chain(5), 1),
+    "h_2": (_hydrogen, 2),
+    "h17_3": (_h17, 3),
+    "li_polarized_4": (_polarized_li, 4),
+    "h39_4": (lambda: S.h_chain(39), 4),
+}
+
+
+@pytest.mark.parametrize("case", list(PAIR_CASES))
+def test_pair_stream_layers(cuda, case):
+    """log|psi| and E_L against the FP64 oracle, to this file's bounds."""
+    import torch
+
+    mk, layers = PAIR_CASES[case]
+    sysm = mk()
+    _, spec, *_ = S.workload("li")
+    spec.nspins, spec.n_atoms = sysm.nspins, sysm.atoms.shape[0]
+    spec.hidden_single, spec.hidden_double, spec.ndets = [32] * layers, [32] * layers, 2
+    p = P.init_params(spec, seed=81, bias_scale=0.1, env_jitter=0.5)
+    x = S.init_walkers(sysm, 5, seed=82)
+    p64, x64, at = P.cast_params(p, np.float64), x.astype(np.float64), sysm.atoms.astype(np.float64)
+    ref = ham.local_energy(spec.as_oracle(), p64, x64, at, sysm.charges.astype(np.float64))
+    A = np.asarray(owf.orbital_matrices(spec.as_oracle(), p64, x64, at))
+    kappa, cancel = np.linalg.cond(A).reshape(5, -1).max(axis=1), cancellation(A)
+    dm = _model(sysm, spec, p)
+    xe = torch.from_numpy(x).to(cuda)
+    lp, sg = dm.logpsi(xe)
+    out = dm.local_energy(xe)
+    bound = logpsi_bound(ref["logpsi"], kappa, "fp32", cancel)
+    assert np.all(np.abs(lp.cpu().numpy() - ref["logpsi"]) <= bound)
+    assert np.all(np.abs(out["logpsi"].cpu().numpy() - ref["logpsi"]) <= bound)
+    np.testing.assert_array_equal(sg.cpu().numpy(), ref["sign"])
+    rel, bnd = el_report(case, out["e_loc"].cpu().numpy(), ref["e_loc"], kappa, "fp32", cancel)
+    assert np.all(rel <= bnd), (rel, bnd)
+    dm.close()

@@ -190,7 +190,10 @@ int jq_logpsi(jq_model* m, const float* elec, int B, float* logpsi, float* sign,
   if (!m || B < 0 || (B > 0 && (!elec || !logpsi))) return jq_fail(JQ_EINVAL, "jq_logpsi: bad argument");
   if (B == 0) return JQ_OK;
   hipStream_t s = (hipStream_t)stream;
-  for (int b0 = 0; b0 < B; b0 += m->chunk_fwd) {
+  const bool small = m->use_small(B);
+  if (small && launch_small_logpsi(m->small, elec, B, logpsi, sign, s))
+    return jq_fail(JQ_EHIP, "jq_logpsi: small-network launch rejected");
+  for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {
     const int Bc = std::min(m->chunk_fwd, B - b0);
     int rc = m->forward(elec, b0, Bc, false, logpsi, sign, nullptr, nullptr, nullptr, nullptr, s);
     if (rc) return rc;
@@ -248,7 +251,12 @@ int jq_mh_steps(jq_model* m, float* elec, float* logp, int B, int n_steps, float
   // walker chunks outermost: each chunk makes all its moves through the
   // model's one-chunk proposal scratch (walkers are independent and the
   // Philox streams are keyed by the global walker index)
-  for (int b0 = 0; b0 < B; b0 += m->chunk_fwd) {
+  const bool small = m->use_small(B);
+  if (small) {
+    const SmallMoves mv{elec, logp, B, n_steps, width, nullptr, normals, uniforms, seed, ctr, n_accept, 0};
+    if (launch_small_moves(m->small, mv, s)) return jq_fail(JQ_EHIP, "jq_mh_steps: small-network launch rejected");
+  }
+  for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {
     const int Bc = std::min(m->chunk_fwd, B - b0);
     float* ec = elec + (long)b0 * n3;
     for (int st = 0; st < n_steps; ++st) {
@@ -274,8 +282,14 @@ int jq_sample(jq_model* m, float* elec, float* logp, int B, int n_outer, int ste
   if (B == 0 || n_outer == 0 || steps == 0) return JQ_OK;  // MCMCSampler.step with steps == 0 is a no-op
   hipStream_t s = (hipStream_t)stream;
   const long n3 = 3L * m->N;
+  const bool small = m->use_small(B);
   for (int o = 0; o < n_outer; ++o) {
-    for (int b0 = 0; b0 < B; b0 += m->chunk_fwd) {
+    if (small) {
+      const SmallMoves mv{elec, logp,    B,        steps, 0.f, state, nullptr, nullptr, seed, ctr + (uint64_t)o * steps,
+                          n_accept, 1};
+      if (launch_small_moves(m->small, mv, s)) return jq_fail(JQ_EHIP, "jq_sample: small-network launch rejected");
+    }
+    for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {
       const int Bc = std::min(m->chunk_fwd, B - b0);
       float* ec = elec + (long)b0 * n3;
       // logp = 2 log|psi| at the current walkers, recomputed each sampler step

@@ -357,46 +357,10 @@ __global__ __launch_bounds__(256) void det_fwd_reg_kernel(FermiDims d, const flo
 // ---------------------------------------------------------------------------
 // Forward mode, N <= 16: log|det| and sign, four determinants per wavefront,
 // one in each 16-lane DPP row: lane j holds column j (NP >= N rows in
-// registers, padded with the identity).  Step p broadcasts column p from lane p
-// of each row (a DPP move, no LDS), every lane finds the pivot in it, exchanges
-// its own rows p and q and subtracts; the column loop is unrolled at compile
-// time.  Bound by VALU issue: 65536 matrices of 14 in 92 us, where a wavefront
+// registers, padded with the identity; fwd_col_steps).  Bound by VALU issue: 65536 matrices of 14 in 92 us, where a wavefront
 // per matrix, exchanging pivot rows and columns through LDS, took 228 (1024 of
 // 3: 4.2 us, 18.5).
 // ---------------------------------------------------------------------------
-template <int P, int NP>
-__device__ __forceinline__ void fwd_col_steps(double (&m)[NP], LogAbsProduct& logdet, int& neg) {
-  if constexpr (P < NP) {
-    double c[NP];
-#pragma unroll
-    for (int i = P; i < NP; ++i) c[i] = dpp_d<0x150 + P>(m[i]);  // row_newbcast:P
-    double best = fabs(c[P]), pv = c[P];
-    int q = P;
-#pragma unroll
-    for (int i = P + 1; i < NP; ++i) {  // the first of the largest
-      const bool more = fabs(c[i]) > best;
-      best = more ? fabs(c[i]) : best;
-      pv = more ? c[i] : pv;
-      q = more ? i : q;
-    }
-    logdet.mul(pv);
-    neg ^= (pv < 0.0) != (q != P) ? 1 : 0;
-    const double mp = m[P], cp = c[P];
-    double r = mp;
-#pragma unroll
-    for (int i = P + 1; i < NP; ++i) {
-      const bool sel = i == q;
-      r = sel ? m[i] : r;
-      m[i] = sel ? mp : m[i];
-      c[i] = sel ? cp : c[i];
-    }
-    r /= pv;
-#pragma unroll
-    for (int i = P + 1; i < NP; ++i) m[i] = fma(-c[i], r, m[i]);
-    fwd_col_steps<P + 1, NP>(m, logdet, neg);
-  }
-}
-
 template <int NP>
 __global__ __launch_bounds__(256) void det_fwd_col_kernel(FermiDims d, const float* __restrict__ Phi, long ldphi,
                                                           const float* __restrict__ env, double* __restrict__ out) {

@@ -1,7 +1,8 @@
-// FP64 Gauss-Jordan inversion with the augmented matrix [A | I] in registers,
-// shared by the determinant kernels (det.hip) and their adjoint (grad.hip).
+// FP64 elimination with the matrix in registers: Gauss-Jordan inversion of the
+// augmented matrix [A | I], shared by the determinant kernels (det.hip) and their
+// adjoint (grad.hip), and the LU of small matrices (det.hip, ferminet_small.hip).
 //
-// No rows are exchanged: the pivot of column p is the unused row with the
+// Gauss-Jordan: no rows are exchanged: the pivot of column p is the unused row with the
 // largest |entry| (the smallest row on ties; any unused row is taken, even a
 // non-finite one), and at the end row p of A^-1 is the right half of the pivot
 // row of column p.  The parity of that row permutation is perm_sign's.
@@ -238,5 +239,44 @@ __device__ __forceinline__ void gj_wave16(double (&x)[8], int& pos, double* scra
       pos = p;
     }
     wave_sync();
+  }
+}
+
+// ---- LU of 16-lane rows: log|det| and sign, no inverse ---------------------
+// Lane j of a DPP row holds column j of an NP x NP matrix (NP <= 16).  Step P
+// broadcasts column P from lane P (a DPP move, no LDS), every lane finds the
+// pivot in it (the first row of the largest |entry|), exchanges its own rows P
+// and q and subtracts; the column loop is unrolled at compile time.  Call with
+// P = 0; every lane of the wave takes part.
+template <int P, int NP>
+__device__ __forceinline__ void fwd_col_steps(double (&m)[NP], LogAbsProduct& logdet, int& neg) {
+  if constexpr (P < NP) {
+    double c[NP];
+#pragma unroll
+    for (int i = P; i < NP; ++i) c[i] = dpp_d<0x150 + P>(m[i]);  // row_newbcast:P
+    double best = fabs(c[P]), pv = c[P];
+    int q = P;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) {  // the first of the largest
+      const bool more = fabs(c[i]) > best;
+      best = more ? fabs(c[i]) : best;
+      pv = more ? c[i] : pv;
+      q = more ? i : q;
+    }
+    logdet.mul(pv);
+    neg ^= (pv < 0.0) != (q != P) ? 1 : 0;
+    const double mp = m[P], cp = c[P];
+    double r = mp;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) {
+      const bool sel = i == q;
+      r = sel ? m[i] : r;
+      m[i] = sel ? mp : m[i];
+      c[i] = sel ? cp : c[i];
+    }
+    r /= pv;
+#pragma unroll
+    for (int i = P + 1; i < NP; ++i) m[i] = fma(-c[i], r, m[i]);
+    fwd_col_steps<P + 1, NP>(m, logdet, neg);
   }
 }

@@ -4,45 +4,12 @@
 // coordinate.  Accept (sampler/mcmc.py:127-137): ratio = logp(x') - logp(x),
 // accept iff ratio > log(u) (strict), u ~ U(0, 1).
 //
-// Randomness, when not supplied by the caller, is Philox-4x32-10 (Salmon et al.,
-// "Parallel random numbers: as easy as 1, 2, 3", SC'11) with key = seed and
-// counter = (block index, walker, step low word, step high word ^ stream tag);
-// normals by the Box-Muller transform.  Streams are keyed by (seed, step,
-// walker, element), never by launch geometry, so a walker's trajectory does
-// not depend on the batch it is evaluated in.
+// Randomness, when not supplied by the caller: philox.h.
 
 #include "kernels.h"
+#include "philox.h"
 
 namespace {
-
-struct u32x4 {
-  uint32_t x, y, z, w;
-};
-
-__device__ inline uint32_t mulhilo(uint32_t a, uint32_t b, uint32_t& hi) {
-  const uint64_t p = (uint64_t)a * b;
-  hi = (uint32_t)(p >> 32);
-  return (uint32_t)p;
-}
-
-__device__ inline u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
-#pragma unroll
-  for (int r = 0; r < 10; ++r) {
-    uint32_t hi0, hi1;
-    const uint32_t lo0 = mulhilo(0xD2511F53u, c.x, hi0);
-    const uint32_t lo1 = mulhilo(0xCD9E8D57u, c.z, hi1);
-    c = u32x4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
-  }
-  return c;
-}
-
-// (0, 1], never 0 so log(u) is finite
-__device__ inline float u01(uint32_t v) { return ((v >> 8) + 1u) * (1.0f / 16777216.0f); }
-
-constexpr uint32_t TAG_NORMAL = 0u;
-constexpr uint32_t TAG_UNIFORM = 0x80000000u;
 
 __global__ void propose_kernel(const float* __restrict__ elec, float* __restrict__ prop, int B, int N3, float width,
                                const double* __restrict__ width_dev, const float* __restrict__ normals,
@@ -61,18 +28,7 @@ __global__ void propose_kernel(const float* __restrict__ elec, float* __restrict
         z[e] = c < N3 ? normals[(long)w * N3 + c] : 0.f;
       }
     } else {
-      const u32x4 r = philox4x32_10(
-          u32x4{(uint32_t)gi, (uint32_t)(w0 + w), (uint32_t)step, (uint32_t)(step >> 32) ^ TAG_NORMAL},
-          (uint32_t)seed, (uint32_t)(seed >> 32));
-      const float u1 = u01(r.x), u2 = u01(r.y), u3 = u01(r.z), u4 = u01(r.w);
-      const float m1 = sqrtf(-2.f * logf(u1)), m2 = sqrtf(-2.f * logf(u3));
-      float s1, c1, s2, c2;
-      sincospif(2.f * u2, &s1, &c1);
-      sincospif(2.f * u4, &s2, &c2);
-      z[0] = m1 * c1;
-      z[1] = m1 * s1;
-      z[2] = m2 * c2;
-      z[3] = m2 * s2;
+      philox_normals(seed, step, (uint32_t)(w0 + w), (uint32_t)gi, z);
     }
     for (int e = 0; e < 4; ++e) {
       const int c = 4 * gi + e;
@@ -91,10 +47,7 @@ __global__ void accept_kernel(float* __restrict__ elec, const float* __restrict_
     if (uniforms) {
       u = uniforms[w];
     } else {
-      const u32x4 r = philox4x32_10(
-          u32x4{0u, (uint32_t)(w0 + w), (uint32_t)step, (uint32_t)(step >> 32) ^ TAG_UNIFORM},
-          (uint32_t)seed, (uint32_t)(seed >> 32));
-      u = u01(r.x);
+      u = philox_uniform(seed, step, (uint32_t)(w0 + w));
     }
     const float lp2 = 2.f * logpsi_prop[w];
     const float ratio = lp2 - logp[w];

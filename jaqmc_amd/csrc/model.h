@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "../../include/jaqmc_amd.h"
+#include "ferminet_small.h"
 #include "kernels.h"
 
 int jq_fail(int code, const std::string& msg);
@@ -95,6 +96,14 @@ struct jq_model {
   // FermiNet
   std::vector<FermiLayer> fl;
   bool pairs_on_chip = false;  // launch_pair_stream instead of a pair stream in H2
+  SmallNet small{};
+  bool small_ok = false;       // the value path also runs as one kernel (ferminet_small.hip)
+  // Whether a batch of B walkers takes it: up to five workgroups per CU (what
+  // their LDS lets run at once), where launches bound the general path.  Three
+  // electrons, log|psi| of 1024 walkers: 25 us (general path 71), of 4096: 46 (92);
+  // general 123 of 8192.  Fourteen, 256 walkers: 37 us (80), 1024: 77 (101);
+  // general 130 of 2048.
+  bool use_small(int B) const { return small_ok && B <= 5L * 256 * small.G; }
   // Psiformer
   std::vector<PsiLayer> pl;
   int D = 0, H = 0, dh = 0, kin = 0;  // model dim, heads, head dim, padded input K

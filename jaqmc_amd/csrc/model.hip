@@ -212,6 +212,32 @@ int jq_model::init_ferminet(const float* packed, size_t n_floats) {
     if (norb == 1) Worb_o[1] = Worb_o[0];
   }
 
+  if (prec == JQ_PREC_FP32 && L <= kSmallLayers) {
+    SmallNet& n = small;
+    n.L = L;
+    n.N = N;
+    n.n_up = n_up;
+    n.n_dn = n_dn;
+    n.nch = nch;
+    n.M = M;
+    n.K = K;
+    n.korb = korb;
+    n.env_kind = d.envelope;
+    n.atoms = atoms;
+    for (int l = 0; l < L; ++l) {
+      const FermiLayer& ly = fl[l];
+      n.l[l] = SmallLayer{(const float*)ly.Wm, (const float*)ly.Wg, ly.b,     ly.W2,     ly.b2,
+                          ly.f1,               ly.f2,               ly.d1,    ly.d2,     ly.kmain,
+                          ly.kg,               ly.res1 ? 1 : 0,     ly.res2 ? 1 : 0};
+    }
+    for (int c = 0; c < 2; ++c) {
+      n.Worb[c] = (const float*)Worb[c];
+      n.pi[c] = pi[c];
+      n.sigma[c] = sigma[c];
+    }
+    small_ok = small_net_plan(n);
+  }
+
   // ---- workspace ----
   size_t kx = 0, kgm = 0, d1m = 0, f2m = 4;
   for (auto& ly : fl) {

@@ -555,3 +555,60 @@ def test_pair_stream_layers(cuda, case):
     rel, bnd = el_report(case, out["e_loc"].cpu().numpy(), ref["e_loc"], kappa, "fp32", cancel)
     assert np.all(rel <= bnd), (rel, bnd)
     dm.close()
+
+
+# networks of the one-kernel value path: electrons per 16-row tile and its
+# remainders, one channel, every envelope, shared orbitals, pair widths whose
+# layers add the bias first (16) and last (8, 12), layers of 32 to 96
+SMALL_CASES = {
+    "h1": (_hydrogen, dict(hidden_single=[32, 32], hidden_double=[8, 8], ndets=2)),
+    "li": (S.li_atom, dict(hidden_single=[64, 64], hidden_double=[16, 16], ndets=4, envelope="isotropic")),
+    "li_polarized": (_polarized_li, dict(hidden_single=[32, 64, 64], hidden_double=[8, 12, 12], ndets=3)),
+    "h5_shared": (lambda: S.h_chain(5), dict(hidden_single=[96, 96], hidden_double=[12, 16], ndets=5,
+                                             orbitals_spin_split=False)),
+    "h9_null": (lambda: S.h_chain(9), dict(hidden_single=[64], hidden_double=[16], ndets=1, envelope="null")),
+    "h16": (lambda: S.h_chain(16), dict(hidden_single=[32, 32, 32, 32], hidden_double=[16, 16, 16, 16], ndets=2)),
+}
+
+
+@pytest.mark.parametrize("case", list(SMALL_CASES))
+def test_small_network_kernel_is_bit_identical(cuda, case):
+    """Walkers of a batch too large for the one-kernel path and the same walkers
+    in a batch that takes it: the same log|psi|, signs and trajectories, with
+    Philox and with given random numbers, and through the device sampler."""
+    import torch
+
+    mk, kw = SMALL_CASES[case]
+    sysm = mk()
+    _, spec, *_ = S.workload("li")
+    spec.nspins, spec.n_atoms = sysm.nspins, sysm.atoms.shape[0]
+    for k, v in kw.items():
+        setattr(spec, k, v)
+    p = P.init_params(spec, seed=91, bias_scale=0.1, env_jitter=0.5)
+    N = spec.n_elec
+    B, n = 5 * 256 * (16 // N) + 1, 77
+    x = torch.from_numpy(S.init_walkers(sysm, B, seed=92)).to(cuda)
+    dm = _model(sysm, spec, p)
+
+    def evaluate(x):
+        x = x.clone()
+        lp, sg = dm.logpsi(x)
+        logp = 2 * lp
+        acc = dm.mh_steps(x, logp, 3, 0.3, seed=5, ctr=11)
+        g = torch.Generator(device="cpu").manual_seed(3)
+        normals, uniforms = torch.randn(2, n, N, 3, generator=g), torch.rand(2, n, generator=g)
+        pad = len(x) - n  # the walkers compared have the same numbers in both batches
+        normals = torch.cat([normals, torch.zeros(2, pad, N, 3)], 1).to(cuda)
+        uniforms = torch.cat([uniforms, torch.full((2, pad), 0.5)], 1).to(cuda)
+        dm.mh_steps(x, logp, 2, 0.2, normals=normals, uniforms=uniforms, n_accept=acc)
+        moved = (x.clone(), logp.clone())
+        state = torch.zeros(3 + 4, dtype=torch.float64, device=cuda)
+        state[0] = 0.25
+        logp2, acc2 = dm.sample(x, state, 2, 3, adapt_frequency=4, seed=9)
+        return lp, sg, *moved, acc, x, logp2, acc2
+
+    big, small = evaluate(x), evaluate(x[:n].contiguous())
+    dm.close()
+    for a, b in zip(big, small):
+        assert torch.equal(a[:n], b)
+    assert 0 < int(small[4].sum()) < 5 * n or N == 1

@@ -14,6 +14,8 @@ int gemm_dispatch_bf16(const GemmArgs& a, hipStream_t s);
 int gemm_dispatch_x3(const GemmArgs& a, hipStream_t s);
 int gemm_dispatch_x6(const GemmArgs& a, hipStream_t s);
 int gemm_dispatch_h3(const GemmArgs& a, hipStream_t s);
+bool gemm_panel_ok(const GemmArgs& a);  // gemm_panel.hip
+int gemm_panel(const GemmArgs& a, hipStream_t s);
 void bgemm_dispatch_f32(const BGemmArgs& a, hipStream_t s);
 void bgemm_dispatch_bf16(const BGemmArgs& a, hipStream_t s);
 void bgemm_dispatch_x3(const BGemmArgs& a, hipStream_t s);
@@ -63,7 +65,9 @@ int launch_gemm(const GemmArgs& a, int prec, bool y_bf16, hipStream_t s) {
     case PREC_BF16X3: return gemm_dispatch_x3(a, s);
     case PREC_BF16X6: return gemm_dispatch_x6(a, s);
     // value-only rows keep the BF16X6 arithmetic (no per-unit row scales)
-    case PREC_FP16X3: return (a.R <= 1 && a.lrp <= 0) ? gemm_dispatch_x6(a, s) : gemm_dispatch_h3(a, s);
+    case PREC_FP16X3:
+      if (a.R <= 1 && a.lrp <= 0) return gemm_dispatch_x6(a, s);
+      return g_gemm_variant == 0 && gemm_panel_ok(a) ? gemm_panel(a, s) : gemm_dispatch_h3(a, s);
   }
   return -1;
 }

@@ -612,3 +612,27 @@ def test_small_network_kernel_is_bit_identical(cuda, case):
     for a, b in zip(big, small):
         assert torch.equal(a[:n], b)
     assert 0 < int(small[4].sum()) < 5 * n or N == 1
+
+
+# 48-, 96- and 128-row units: a last tile of one unit of two, column blocks that
+# are not full (24 x 13, 16 x 30, 12 x 42 orbitals), head-split projections
+@pytest.mark.parametrize("n,ndets,B", [(13, 24, 159), (30, 16, 35), (42, 12, 25)])
+def test_wide_projections_are_bit_identical(cuda, n, ndets, B):
+    """In FP16X3 a batch whose projections run on whole row panels gives every
+    walker the results of chunks too small for them."""
+    import torch
+
+    sysm = S.h_chain(n)
+    _, spec, *_ = S.workload("ring42")
+    spec.nspins, spec.n_atoms, spec.ndets, spec.num_layers = sysm.nspins, n, ndets, 2
+    p = P.init_params(spec, seed=101, bias_scale=0.1, env_jitter=0.3)
+    x = torch.from_numpy(S.init_walkers(sysm, B, seed=102)).to(cuda)
+    out = []
+    for chunk in (0, B // 3):
+        dm = _model(sysm, spec, p, prec="fp16x3", chunk=chunk)
+        out.append(dm.local_energy(x, with_grad=True))
+        torch.cuda.synchronize()
+        dm.close()
+    for k, v in out[0].items():
+        assert torch.equal(v, out[1][k]), k
+    assert torch.isfinite(out[0]["e_loc"]).all()

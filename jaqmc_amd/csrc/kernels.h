@@ -83,6 +83,27 @@ int launch_bgemm(const BGemmArgs& a, int prec, hipStream_t s);
 // FP32 in memory (y_bf16 must be false).
 int launch_gemm(const GemmArgs& a, int prec, bool y_bf16, hipStream_t s);
 
+// ---- row-wise part of a Psiformer layer (psi_chain.hip) ----
+constexpr int kChainMlp = 4;  // most dense layers of an MLP in one launch
+struct PsiChainArgs {
+  const float* O; long ldo;        // attention output (units * Rp, ldo), 16-byte rows
+  float* x;                        // (units * Rp, 256) residual stream, updated in place
+  int units, R;                    // R of the Rp rows of a unit are tangent rows
+  int nm;                          // dense layers of the MLP
+  const void* W[1 + kChainMlp];    // output projection, MLP: weight planes (GemmArgs::Wt_lo)
+  const float* bias[1 + kChainMlp];
+  const float *ln2_s, *ln2_b;
+  const void* Wp;                  // next layer's stacked q, k, v, or null: none
+  const float* bp;
+  const float *ln1_s, *ln1_b;
+  float* Y;                        // head-split output (GemmArgs::hs_*)
+  int N, H, dh;
+  float eps;
+};
+// Whether layers of D features with MLP widths width[0 .. n_mlp] run there.
+bool psi_chain_supported(int Rp, int D, int prec, int n_mlp, const int* width);
+int launch_psi_chain(const PsiChainArgs& a, int Rp, hipStream_t s);
+
 // ---- FermiNet feature / stream kernels (ferminet.hip) ----
 struct FermiDims {
   int Bc, N, n_up, n_dn, M, K;  // walkers in chunk, electrons, atoms, dets

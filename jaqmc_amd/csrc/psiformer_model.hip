@@ -305,18 +305,19 @@ int jq_model::forward_psiformer(const float* elec, int Bc, bool lap, hipStream_t
 
   int rc = launch_psi_features(fd, elec, atoms, T2, kin, (options & JQ_OPT_NO_RESCALE) ? 0 : 1, s);
   // ln1_in_t1: T1 already holds LN1(x) of the coming layer (fused above)
-  bool ln1_in_t1 = lnf && L > 0;
+  bool ln1_in_t1 = lnf && L > 0, qkv_done = false;
   rc |= gemm(T2, kin, Win, Win_lo, (long)D * kin, kin, x, D, D, bin, ACT_NONE, nullptr, 0, ln1_in_t1 ? T1 : nullptr,
              L > 0 ? pl[0].ln1_s : nullptr, L > 0 ? pl[0].ln1_b : nullptr);
   for (int l = 0; l < L && !rc; ++l) {
     const PsiLayer& ly = pl[l];
+    const int nm = (int)ly.Wm.size();
     const float* qin = x;  // attention input: LN1(x) pre-LN, x otherwise
-    if (ln_mode == JQ_LN_PRE) {
+    if (ln_mode == JQ_LN_PRE && !qkv_done) {
       if (!ln1_in_t1) rc |= launch_layernorm_lap((int)units, RP, R, D, x, T1, ly.ln1_s, ly.ln1_b, 1e-5f, s);
       qin = T1;
     }
     ln1_in_t1 = false;
-    {
+    if (!qkv_done) {
       GemmArgs g{};
       g.X = qin;
       g.ldx = D;
@@ -436,6 +437,41 @@ int jq_model::forward_psiformer(const float* elec, int Bc, bool lap, hipStream_t
         rc |= launch_bgemm(g6, prec, s);
       }
     }
+    // Everything from the output projection to the next layer's q, k, v is
+    // row-wise: one launch where the kernel takes the widths.
+    if (lap && ln_mode == JQ_LN_PRE && psi_chain_supported(RP, D, prec, nm, ly.mdims.data())) {
+      PsiChainArgs ca{};
+      ca.O = Om;
+      ca.ldo = DO;
+      ca.x = x;
+      ca.units = (int)units;
+      ca.R = R;
+      ca.nm = nm;
+      ca.W[0] = ly.Wo_lo;
+      ca.bias[0] = ly.bo;
+      for (int j = 0; j < nm; ++j) {
+        ca.W[1 + j] = ly.Wm_lo[j];
+        ca.bias[1 + j] = ly.bm[j];
+      }
+      ca.ln2_s = ly.ln2_s;
+      ca.ln2_b = ly.ln2_b;
+      if (l + 1 < L) {
+        ca.Wp = pl[l + 1].Wqkv_lo;
+        ca.bp = pl[l + 1].bqkv;
+        ca.ln1_s = pl[l + 1].ln1_s;
+        ca.ln1_b = pl[l + 1].ln1_b;
+        ca.Y = QKV;
+        ca.N = N;
+        ca.H = H;
+        ca.dh = dh;
+      }
+      ca.eps = 1e-5f;
+      ProfScope ps(PROF_GEMM_LAYER_LAP, s);
+      rc |= launch_psi_chain(ca, RP, s);
+      qkv_done = l + 1 < L;
+      continue;
+    }
+    qkv_done = false;
     // x += Wo O + bo  (and T1 = LN2(x) when fused)
     rc |= gemm(Om, DO, ly.Wo, ly.Wo_lo, (long)D * D, D, x, D, D, ly.bo, ACT_NONE, x, 0, lnf ? T1 : nullptr,
                ly.ln2_s, ly.ln2_b);
@@ -450,7 +486,6 @@ int jq_model::forward_psiformer(const float* elec, int Bc, bool lap, hipStream_t
       cur = T1;
     }
     int curw = D;
-    const int nm = (int)ly.Wm.size();
     for (int j = 0; j < nm && !rc; ++j) {
       const int outw = ly.mdims[j + 1];
       const int ka = round_up(curw, 32);

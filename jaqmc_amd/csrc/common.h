@@ -113,5 +113,15 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Workgroup barrier that orders LDS accesses alone.  __syncthreads also waits
+// for every global load and store of the wavefront: a kernel that keeps loads
+// in flight or lets its stores drain across a barrier, and shares no global
+// data between its threads, takes this one.
+__device__ inline void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 static inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 static inline int ceil_div(long x, long m) { return (int)((x + m - 1) / m); }

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kThreads, 3) void panel_kernel(const GemmArgs a, in
     int t = t0 + slot;
     if (t < t1) load(t);
     for (; t < t1; t += step) {
-      __syncthreads();  // the panel is free
+      lds_barrier();  // the panel is free
       float sk = kJScale, ik = 1.f / kJScale;  // lane j keeps the scales of row p + 4 j
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kThreads, 3) void panel_kernel(const GemmArgs a, in
         rsc[p + 4 * lane] = sk;
         rsi[p + 4 * lane] = ik;
       }
-      __syncthreads();  // the panel is ready
+      lds_barrier();  // the panel is ready
       if (t + step < t1) load(t + step);
     }
     return;
@@ -158,8 +158,8 @@ __global__ __launch_bounds__(kThreads, 3) void panel_kernel(const GemmArgs a, in
   };
   bload(S0{}, 0, 0);
   for (int t = t0 + slot; t < t1; t += step) {
-    __syncthreads();  // every consumer is done with the panel
-    __syncthreads();  // the producers have filled it
+    lds_barrier();  // every consumer is done with the panel
+    lds_barrier();  // the producers have filled it
     const int z = t / tiles_per_batch;
     const long row0 = (long)(t - z * tiles_per_batch) * BM;
     for (int cb = 0; cb < ncb; ++cb) {

@@ -102,7 +102,7 @@ struct PsiChainArgs {
 };
 // Whether layers of D features with MLP widths width[0 .. n_mlp] run there.
 bool psi_chain_supported(int Rp, int D, int prec, int n_mlp, const int* width);
-int launch_psi_chain(const PsiChainArgs& a, int Rp, hipStream_t s);
+int launch_psi_chain(const PsiChainArgs& a, hipStream_t s);
 
 // ---- FermiNet feature / stream kernels (ferminet.hip) ----
 struct FermiDims {

@@ -1,8 +1,9 @@
 // The row-wise part of a pre-LN Psiformer layer in one kernel (Laplacian mode,
-// FP16X3, 256 features): for every tile of whole units
+// FP16X3, 256 features, 128-row units): for every unit
 //   x1 = x + O Wo + bo;  t = LN2(x1);  t = tanh(t Wm + bm), ...;  x = x1 + t;
 //   QKV = LN1'(x) Wqkv' + bqkv'   (the next layer's, head-split; none after the last)
-// by the forward-Laplacian rules of gemm_kernel and layernorm_lap_kernel.
+// by the forward-Laplacian rules of gemm_kernel, in its order: the results are the same
+// bit for bit as those of a GEMM a stage with the LayerNorms in their epilogues.
 //
 // Bound by the FP16 matrix rate, the LayerNorms and the memory together: as one
 // GEMM a stage, with the LayerNorms in their epilogues, a layer read and wrote
@@ -13,42 +14,63 @@
 // owns 32 columns of every row, so accumulators (64 registers), the residual
 // stream x1 (64) and two chunks of weight fragments fit the 256 registers of two
 // waves per SIMD.  The columns of a lane are adjacent: x, q, k, v move as 128-byte
-// row segments straight from registers.  Loads hide behind products: weights two
-// chunks ahead (the next stage's before this one's stores), x row block by row
-// block during the first stage, the next tile's O during the first q, k, v block.
+// row segments straight from registers, past the L2's weights (nontemporal).
+// Vector-memory results return in order, so a load from HBM issued between the
+// weights' delays them: O of the next tile is requested before the second
+// LayerNorm and x as soon as the panel is written, the weights two chunks ahead
+// (the next stage's before this one's stores), and no barrier waits for any of
+// them.
 // Measured, the four layers of 768 walkers of 42 electrons (4.1M rows of 128-row
-// units, two-layer MLP): 61.1 ms in separate launches, 44.2 ms here (0.77 PFLOP/s
-// issued); their energies 111.0 -> 92.9 ms.
+// units, two-layer MLP): 61.1 ms in separate launches, 45.6 ms here (0.75 PFLOP/s
+// issued).  A tile takes about 200k cycles: 74k are the products' at the matrix
+// rate (what they take where no store is draining), the rest the LayerNorms' sums
+// and the waits for the stores of x, q, k and v.  Taken back: loads of x and O
+// spread over the chunks of a stage (+20k cycles), workgroups started at
+// staggered times (no change), LayerNorm sums by halving steps over a lane row
+// (10k cycles less, another rounding).
 #include "kernels.h"
 
 namespace {
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kD = 256;          // features of every stage
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
 constexpr int kLS = kD + 8;      // f16 per panel row
+constexpr int kFS = kD + 4;      // floats per row of the LayerNorm
 constexpr int kNK = kD / 32;     // k chunks of a stage
 constexpr int kCus = 256;
 constexpr float kJScale = 64.f;  // fixed scale of Jacobian rows (gemm_impl.h)
+constexpr int kMB = 8;           // 16-row blocks of a unit
 constexpr int kProj = 3;         // column blocks of the projection
 
-template <int MB>
-constexpr int chain_lds() {
-  return 2 * 16 * MB * kLS * 2 + 4 * (kWaves * 16 * MB + 16 * MB + 16 * kWaves + 2 * 16 + 2 * 16) +
-         4 * kD * (2 * (1 + kChainMlp + kProj) + 4);
-}
+constexpr int kLds = 2 * 16 * kMB * kLS * 2 + 4 * (256 + 2 * 16 * kMB + 2 * kWaves + 4) +
+                     4 * kD * (2 * (1 + kChainMlp + kProj) + 4);
 
-// Sum and maximum over the 16 lanes of a DPP row.
-__device__ inline float sum16(float t) {
-  t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0xB1, 0xF, 0xF, false));
-  t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x4E, 0xF, 0xF, false));
-  t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x141, 0xF, 0xF, false));
-  return t + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x140, 0xF, 0xF, false));
-}
+// Maximum over the 16 lanes of a DPP row.
 __device__ inline float max16(float t) {
   t = fmaxf(t, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0xB1, 0xF, 0xF, false)));
   t = fmaxf(t, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x4E, 0xF, 0xF, false)));
   t = fmaxf(t, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x141, 0xF, 0xF, false)));
   return fmaxf(t, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x140, 0xF, 0xF, false)));
+}
+// x * sc (sc a power of two) as the sum of two FP16; each one mixed-precision
+// multiply-add, which rounds once.
+__device__ inline void split(float x, float sc, f16* h, f16* l) {
+  *h = (f16)__builtin_fmaf(x, sc, 0.f);
+  *l = (f16)__builtin_fmaf(x, sc, -(float)*h);
+}
+template <int CTRL>
+__device__ inline float dpp_f(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+// Sum over the wavefront's 64 lanes: 16-lane rows first, then (0 + 1) + (2 + 3).
+__device__ inline float row_sum(float t) {
+  t += dpp_f<0xB1>(t);
+  t += dpp_f<0x4E>(t);
+  t += dpp_f<0x141>(t);
+  t += dpp_f<0x140>(t);
+  t += __shfl_xor(t, 16);
+  return t + __shfl_xor(t, 32);
 }
 // Power of two that brings mx into [2^13, 2^14), and its inverse.
 __device__ inline void pow2_scale(float mx, float* sc, float* si) {
@@ -63,21 +85,23 @@ __device__ inline void pow2_scale(float mx, float* sc, float* si) {
   }
 }
 
-// MB: 16-row blocks of a tile; MBU: of a unit
-template <int MB, int MBU>
+// PROJ: with the projection
+template <bool PROJ>
 __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainArgs a, int tiles) {
-  constexpr int BM = 16 * MB, RU = 16 * MBU, UPT = MB / MBU, NJ = BM / kWaves;
-  static_assert(MB % MBU == 0 && MB <= kNK && UPT <= 4, "whole units; one row block a chunk");
+  constexpr int MB = kMB, BM = 16 * MB, NJ = BM / kWaves;
+  constexpr int MP = 6;  // row blocks from here on can hold padding rows (R > 96)
+  static_assert(BM * kFS * 4 <= 2 * BM * kLS * 2, "the rows fit the panel");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   f16* const P0 = (f16*)smem;  // high plane, then the low plane
   f16* const P1 = P0 + BM * kLS;
-  float* const part = (float*)(P1 + BM * kLS);  // [waves][BM] row partials
-  float* const rowv = part + kWaves * BM;       // [BM] row means, then J_v,r
-  float* const mx8 = rowv + BM;                 // [2 UPT][waves] maxima of value and Laplacian rows
-  float* const mx1 = mx8 + 16 * kWaves;         // [2 UPT] the same of a loaded panel
-  float* const scal = mx1 + 32;                 // [waves][4] sums of squares per unit
-  float* const pv = scal + 32;                  // per stage: inverse column scales, then biases
-  const int nst = 1 + a.nm + (a.Wp ? kProj : 0);
+  float* const sqp = (float*)(P1 + BM * kLS);   // [4][64] sums of squares
+  float* const rowm = sqp + 256;                // [BM] row means
+  float* const rowv = rowm + BM;                // [BM] J_v,r
+  float* const mx8 = rowv + BM;                 // [2][waves] maxima of value and Laplacian rows
+  float* const mx1 = mx8 + 2 * kWaves;          // [2] the same of a loaded panel
+  float* const scal = mx1 + 2;                 // <d_r, d_0> of the value and Laplacian rows
+  float* const pv = scal + 2;                  // per stage: inverse column scales, then biases
+  const int nst = 1 + a.nm + (PROJ ? kProj : 0);
   float* const pbias = pv + nst * kD;
   float* const pln = pbias + nst * kD;          // scale and bias of LN2, then of the next LN1
 
@@ -108,15 +132,15 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
   for (int i = tid; i < kD; i += kThreads) {
     pln[i] = a.ln2_s[i];
     pln[kD + i] = a.ln2_b[i];
-    pln[2 * kD + i] = a.Wp ? a.ln1_s[i] : 0.f;
-    pln[3 * kD + i] = a.Wp ? a.ln1_b[i] : 0.f;
+    pln[2 * kD + i] = PROJ ? a.ln1_s[i] : 0.f;
+    pln[3 * kD + i] = PROJ ? a.ln1_b[i] : 0.f;
   }
 
   // XCD x = b % 8 takes a contiguous range of tiles, its workgroups neighbours
   const int tpx = (tiles + kXcds - 1) / kXcds;
   const int t0 = (int)(blockIdx.x % kXcds) * tpx, t1 = t0 + tpx < tiles ? t0 + tpx : tiles;
   const int slot = (int)blockIdx.x / kXcds, step = (int)gridDim.x / kXcds;
-  const int rows = a.units * RU;
+  const int rows = a.units * BM;
 
   f32x4 acc[MB][2], aux[2 * MB];  // aux: x, x1 (two rows of two columns each), or the next panel
   uint4 b[2][2][2];               // [set][plane][column of the pair]
@@ -130,13 +154,12 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
   auto load_row = [&](int t, int j, int lane) __attribute__((always_inline)) {
     int r = t * BM + wave + kWaves * j;
     r = r < rows ? r : rows - 1;
-    aux[j] = *(const f32x4*)(a.O + (long)r * a.ldo + 4 * lane);
+    aux[j] = __builtin_nontemporal_load((const f32x4*)(a.O + (long)r * a.ldo + 4 * lane));
   };
   // One stage: acc = panel . W^T over this wave's 32 columns, every row.  Its
   // first two chunks' fragments are there; those of the next stage's (Wn) are
   // requested after their sets' last products, before the epilogue's stores.
-  // extra(c) issues other loads after chunk c.
-  auto products = [&](const f16* W, long wp, const f16* Wn, long wpn, auto extra) __attribute__((always_inline)) {
+  auto products = [&](const f16* W, long wp, const f16* Wn, long wpn) __attribute__((always_inline)) {
     LANE
     const int boff = col * kD + 8 * lg;
 #pragma unroll
@@ -165,12 +188,11 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
         bload(c & 1, W, wp, c + 2, boff);
       else
         bload(c & 1, Wn, wpn, c + 2 - kNK, boff);
-      extra(c, lane);
       __builtin_amdgcn_sched_barrier(0);  // no other chunk's operands in registers
     }
   };
   // inverse scales of the panel's value and Laplacian rows
-  float ival[UPT], ilap[UPT];
+  float ival = 1.f, ilap = 1.f;
   // acc without the power-of-two scales, the bias on the value rows
   auto unscale = [&](int st) __attribute__((always_inline)) {
     LANE
@@ -181,206 +203,202 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float ir = 1.f / kJScale;
-        if (mb % MBU == 0 && v < ROW_J0) ir = lg == 0 ? (v == ROW_VAL ? ival[mb / MBU] : ilap[mb / MBU]) : ir;
+        if (mb == 0 && v < ROW_J0) ir = lg == 0 ? (v == ROW_VAL ? ival : ilap) : ir;
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
           acc[mb][nb][v] *= ir * csi[nb];
-          if (mb % MBU == 0 && v == ROW_VAL) acc[mb][nb][v] += lg == 0 ? bb[nb] : 0.f;
+          if (mb == 0 && v == ROW_VAL) acc[mb][nb][v] += lg == 0 ? bb[nb] : 0.f;
         }
       }
   };
-  // (the fused multiply-adds of this rule and of the LayerNorm are written out,
-  // so that a unit's result does not depend on its place in the tile)
+  // (the fused multiply-adds of this rule and of the LayerNorm are written out as
+  // gemm_kernel's are compiled)
   auto tanh_rule = [&]() __attribute__((always_inline)) {
 #pragma clang fp contract(off)
     LANE
 #pragma unroll
-    for (int u = 0; u < UPT; ++u)
+    for (int nb = 0; nb < 2; ++nb) {
+      float sq = 0.f;
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        float sq = 0.f;
+      for (int m = 0; m < MB; ++m)
 #pragma unroll
-        for (int m = 0; m < MBU; ++m)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float j = acc[u * MBU + m][nb][v];
-            const bool jrow = !(m == 0 && lg == 0 && v < ROW_J0);
-            sq = fmaf(jrow ? j : 0.f, j, sq);
-          }
-        sq += __shfl_xor(sq, 16);
-        sq += __shfl_xor(sq, 32);
-        const float y0 = __shfl(acc[u * MBU][nb][ROW_VAL], lr);
-        const float y1 = __shfl(acc[u * MBU][nb][ROW_LAP], lr);
-        const float th = tanhf(y0);
-        const float d1 = fmaf(-th, th, 1.f);
-        const float lap = fmaf(d1, y1, -2.f * th * d1 * sq);
-#pragma unroll
-        for (int m = 0; m < MBU; ++m)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[u * MBU + m][nb][v] *= d1;
-        if (lg == 0) {
-          acc[u * MBU][nb][ROW_VAL] = th;
-          acc[u * MBU][nb][ROW_LAP] = lap;
+        for (int v = 0; v < 4; ++v) {
+          const float j = acc[m][nb][v];
+          if (m == 0 && v == 0)
+            sq = lg == 0 ? 0.f : fmaf(j, j, acc[0][nb][1] * acc[0][nb][1]);
+          else if (m > 0 || v > 1)
+            sq = fmaf(j, j, sq);
         }
+      sq += __shfl_xor(sq, 16);
+      sq += __shfl_xor(sq, 32);
+      const float y0 = __shfl(acc[0][nb][ROW_VAL], lr);
+      const float y1 = __shfl(acc[0][nb][ROW_LAP], lr);
+      const float th = tanhf(y0);
+      const float d1 = fmaf(-th, th, 1.f);
+      const float lap = fmaf(d1, y1, -2.f * th * d1 * sq);
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[m][nb][v] *= d1;
+      if (lg == 0) {
+        acc[0][nb][ROW_VAL] = th;
+        acc[0][nb][ROW_LAP] = lap;
       }
+    }
   };
-  // acc = LN(acc).  A row statistic is a sum over the 16 lanes of a lane group,
-  // combined over the waves in LDS.
+  // acc = LN(acc).  The rows go through LDS (the panel is free), where a
+  // wave sums sixteen of them whole, a row's 256 columns over its lanes:
+  // position 4 l + q of a row holds column 64 (l / 16) + 16 q + l % 16.
+  // Sums are taken in gemm_kernel's order.
   auto layernorm = [&](const float* ln) __attribute__((always_inline)) {
 #pragma clang fp contract(off)
     LANE
     constexpr float invD = 1.f / kD;
+    float* const F = (float*)smem;
+    lds_barrier();  // every wave is done with the panel
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int nb = 0; nb < 2; ++nb) {
+      float* const fp = F + 4 * lg * kFS + (wave >> 1) * 64 + ((2 * lr + nb) & 15) * 4 + (wave & 1) * 2 + (lr >> 3);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float t = sum16(acc[mb][0][v] + acc[mb][1][v]);
-        if (lr == 0) part[wave * BM + mb * 16 + 4 * lg + v] = t;
-      }
-    __syncthreads();
-    auto total = [&](int r) __attribute__((always_inline)) {
-      float t[kWaves];
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) t[w] = part[w * BM + r];
-      return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
-    };
-    if (tid < BM) rowv[tid] = total(tid) * invD;
-    __syncthreads();
-    float d0[UPT][2];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const f32x4 m = *(const f32x4*)&rowv[mb * 16 + 4 * lg];
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb) acc[mb][nb] -= m;
-      if (mb % MBU == 0)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) d0[mb / MBU][nb] = __shfl(acc[mb][nb][ROW_VAL], lr);
+        for (int v = 0; v < 4; ++v) fp[(mb * 16 + v) * kFS] = acc[mb][nb][v];
     }
-    // <d_r, d_0> per row; sum of |d_r|^2 over the Jacobian rows of a unit
+    lds_barrier();
+    {
+      auto sum4 = [](const f32x4& x) __attribute__((always_inline)) {
+        return row_sum(((x.x + x.y) + x.z) + x.w);
+      };
+      f32x4 z = *(const f32x4*)&F[4 * lane];
+      z -= sum4(z) * invD;  // centred value row
+      float mean = 0.f, dot = 0.f;  // of row 16 wave + lane % 16
 #pragma unroll
-    for (int u = 0; u < UPT; ++u) {
+      for (int k = 0; k < 16; ++k) {
+        const int r = 16 * wave + k;
+        f32x4 x = *(const f32x4*)&F[r * kFS + 4 * lane];
+        const float m = sum4(x) * invD;
+        x -= m;
+        const float t = row_sum(fmaf(x.w, z.w, fmaf(x.z, z.z, fmaf(x.y, z.y, x.x * z.x))));
+        mean = lr == k ? m : mean;
+        dot = lr == k ? t : dot;
+        if (r > 0) F[r * kFS + 4 * lane] = fmaf(x.w, x.w, fmaf(x.z, x.z, fmaf(x.x, x.x, x.y * x.y)));
+      }
+      if (lane < 16) {
+        const int r = 16 * wave + lane;
+        rowm[r] = mean;
+        rowv[r] = r >= ROW_J0 && r < a.R ? 2.f * invD * dot : 0.f;  // J_v,r = 2/D <d_r, d_0>
+        if (r < ROW_J0) scal[r] = dot;
+      }
+    }
+    lds_barrier();
+    // sums of |d_r|^2 over the Jacobian rows, a lane group's rows in turn
+    if (wave < 4) {
       float sq = 0.f;
 #pragma unroll
-      for (int m = 0; m < MBU; ++m)
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int mb = u * MBU + m, r = m * 16 + 4 * lg + v;
-          const float x0 = acc[mb][0][v], x1 = acc[mb][1][v];
-          sq += (r >= ROW_J0 && r < a.R) ? fmaf(x1, x1, x0 * x0) : 0.f;
-          const float t = sum16(fmaf(x1, d0[u][1], x0 * d0[u][0]));
-          if (lr == 0) part[wave * BM + u * RU + r] = t;
+          const int r = mb * 16 + 4 * wave + v;
+          if (r >= ROW_J0 && r < a.R) sq += F[r * kFS + 4 * lane];
         }
-      sq = wave_sum(sq);
-      if (lane == 0) scal[wave * 4 + u] = sq;
+      sqp[wave * 64 + lane] = sq;
     }
-    __syncthreads();
-    // J_v,r = 2/D <d_r, d_0> of the Jacobian rows; per unit the variance, its
-    // Laplacian, s = (v + eps)^-1/2 and its derivatives
-    float sv[UPT], s1[UPT], s2[UPT], lapv[UPT];
+    float d0[2];
 #pragma unroll
-    for (int u = 0; u < UPT; ++u) {
-      float q[kWaves];
+    for (int mb = 0; mb < MB; ++mb) {
+      const f32x4 m = *(const f32x4*)&rowm[mb * 16 + 4 * lg];
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) q[w] = scal[w * 4 + u];
-      const float sqt = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
-      lapv[u] = 2.f * invD * (total(u * RU + ROW_LAP) + sqt);
-      const float ve = fmaf(total(u * RU + ROW_VAL), invD, a.eps);
-      sv[u] = rsqrtf(ve);
-      s1[u] = -0.5f * sv[u] / ve;
-      s2[u] = 0.75f * sv[u] / (ve * ve);
+      for (int nb = 0; nb < 2; ++nb) acc[mb][nb] -= m;
     }
-    if (tid < BM) {
-      const int r = tid % RU;
-      rowv[tid] = (r >= ROW_J0 && r < a.R) ? 2.f * invD * total(tid) : 0.f;
-    }
-    __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) d0[nb] = __shfl(acc[0][nb][ROW_VAL], lr);
+    const float j0 = rowv[lane], j1 = rowv[64 + lane];
+    const float jv2 = wave_sum(j0 * j0) + wave_sum(j1 * j1);
+    lds_barrier();
+    float sqt = (sqp[lane] + sqp[128 + lane]) + (sqp[64 + lane] + sqp[192 + lane]);
+    sqt += __shfl_xor(sqt, 8);
+    sqt += __shfl_xor(sqt, 4);
+    sqt += __shfl_xor(sqt, 2);
+    sqt += __shfl_xor(sqt, 1);
+    sqt += __shfl_xor(sqt, 16);
+    sqt += __shfl_xor(sqt, 32);
+    // the variance, its Laplacian, s = (v + eps)^-1/2 and its derivatives
+    const float lapv = 2.f * invD * (scal[ROW_LAP] + sqt);
+    const float ve = fmaf(scal[ROW_VAL], invD, a.eps);
+    const float sv = rsqrtf(ve);
+    const float s1 = -0.5f * sv / ve;
+    const float s2 = 0.75f * sv / (ve * ve);
+    const float laps = fmaf(s1, lapv, s2 * jv2);
     const float2 g2 = *(const float2*)&ln[col], b2 = *(const float2*)&ln[kD + col];
     const float g[2] = {g2.x, g2.y}, bb[2] = {b2.x, b2.y};
+    float cross[2] = {0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < UPT; ++u) {
-      float cross[2] = {0.f, 0.f}, jv2 = 0.f;
+    for (int mb = 0; mb < MB; ++mb) {
+      const f32x4 jv = *(const f32x4*)&rowv[mb * 16 + 4 * lg];
 #pragma unroll
-      for (int m = 0; m < MBU; ++m) {
-        const int mb = u * MBU + m;
-        const f32x4 jv = *(const f32x4*)&rowv[mb * 16 + 4 * lg];
+      for (int v = 0; v < 4; ++v) {
+        const float js = s1 * jv[v];  // 0 outside the Jacobian rows
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = m * 16 + 4 * lg + v;
-          const float js = s1[u] * jv[v];  // 0 outside the Jacobian rows
-          jv2 = fmaf(jv[v], jv[v], jv2);
-          const bool jr = r >= ROW_J0 && r < a.R;
-#pragma unroll
-          for (int nb = 0; nb < 2; ++nb) {
-            const float d = acc[mb][nb][v];
-            cross[nb] = fmaf(d, js, cross[nb]);
-            const float y = jr ? g[nb] * fmaf(d, sv[u], d0[u][nb] * js) : 0.f;
-            if (m == 0 && v == ROW_VAL)
-              acc[mb][nb][v] = lg == 0 ? fmaf(g[nb], d * sv[u], bb[nb]) : y;
-            else if (m == 0 && v == ROW_LAP)
-              acc[mb][nb][v] = lg == 0 ? d : y;
-            else
-              acc[mb][nb][v] = y;
+        for (int nb = 0; nb < 2; ++nb) {
+          const float d = acc[mb][nb][v];
+          cross[nb] = fmaf(d, js, cross[nb]);
+          float y = g[nb] * fmaf(sv, d, js * d0[nb]);
+          if (mb >= MP) y = mb * 16 + 4 * lg + v < a.R ? y : 0.f;
+          if (mb == 0 && v == ROW_VAL) {
+            // (gemm_kernel's rounding of this row block: from the second 16
+            // columns of a 64-column group on, sv d is the rounded product)
+            const float p = sv * d;
+            if ((wave & 1) != 0 || lr >= 8) y = g[nb] * fmaf(js, d0[nb], p);
+            y = lg == 0 ? fmaf(p, g[nb], bb[nb]) : y;
           }
+          if (mb == 0 && v == ROW_LAP) y = lg == 0 ? d : y;
+          acc[mb][nb][v] = y;
         }
       }
-      jv2 += __shfl_xor(jv2, 16);
-      jv2 += __shfl_xor(jv2, 32);
-      const float laps = fmaf(s1[u], lapv[u], s2[u] * jv2);
+    }
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        float t = cross[nb] + __shfl_xor(cross[nb], 16);
-        t += __shfl_xor(t, 32);
-        if (lg == 0)
-          acc[u * MBU][nb][ROW_LAP] = g[nb] * fmaf(2.f, t, fmaf(acc[u * MBU][nb][ROW_LAP], sv[u], d0[u][nb] * laps));
-      }
+    for (int nb = 0; nb < 2; ++nb) {
+      float t = cross[nb] + __shfl_xor(cross[nb], 16);
+      t += __shfl_xor(t, 32);
+      if (lg == 0) acc[0][nb][ROW_LAP] = g[nb] * fmaf(2.f, t, fmaf(acc[0][nb][ROW_LAP], sv, d0[nb] * laps));
     }
   };
   // acc into the panel: value and Laplacian rows scaled to [2^13, 2^14)
   auto put_panel = [&]() __attribute__((always_inline)) {
     LANE
 #pragma unroll
-    for (int u = 0; u < UPT; ++u)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const float m = max16(fmaxf(fabsf(acc[u * MBU][0][p]), fabsf(acc[u * MBU][1][p])));
-        if (lane == 0) mx8[(2 * u + p) * kWaves + wave] = m;
-      }
-    __syncthreads();  // every wave is done with the panel
-    float sval[UPT], slap[UPT];
-#pragma unroll
-    for (int u = 0; u < UPT; ++u) {
-      float m[2];
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const f32x4 q0 = *(const f32x4*)&mx8[(2 * u + p) * kWaves], q1 = *(const f32x4*)&mx8[(2 * u + p) * kWaves + 4];
-        m[p] = fmaxf(fmaxf(fmaxf(q0.x, q0.y), fmaxf(q0.z, q0.w)), fmaxf(fmaxf(q1.x, q1.y), fmaxf(q1.z, q1.w)));
-      }
-      pow2_scale(m[0], &sval[u], &ival[u]);
-      pow2_scale(m[1], &slap[u], &ilap[u]);
+    for (int p = 0; p < 2; ++p) {
+      const float m = max16(fmaxf(fabsf(acc[0][0][p]), fabsf(acc[0][1][p])));
+      if (lane == 0) mx8[p * kWaves + wave] = m;
     }
+    lds_barrier();  // every wave is done with the panel
+    float m[2], sval, slap;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const f32x4 q0 = *(const f32x4*)&mx8[p * kWaves], q1 = *(const f32x4*)&mx8[p * kWaves + 4];
+      m[p] = fmaxf(fmaxf(fmaxf(q0.x, q0.y), fmaxf(q0.z, q0.w)), fmaxf(fmaxf(q1.x, q1.y), fmaxf(q1.z, q1.w)));
+    }
+    pow2_scale(m[0], &sval, &ival);
+    pow2_scale(m[1], &slap, &ilap);
     f16 *p0 = P0 + 4 * lg * kLS + col, *p1 = P1 + 4 * lg * kLS + col;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float sc = kJScale;
-        if (mb % MBU == 0 && v < ROW_J0) sc = lg == 0 ? (v == ROW_VAL ? sval[mb / MBU] : slap[mb / MBU]) : sc;
+        if (mb == 0 && v < ROW_J0) sc = lg == 0 ? (v == ROW_VAL ? sval : slap) : sc;
         f16 h[2], l[2];
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          const float y = acc[mb][nb][v] * sc;
-          h[nb] = (f16)y;
-          l[nb] = (f16)(y - (float)h[nb]);
-        }
+        for (int nb = 0; nb < 2; ++nb) split(acc[mb][nb][v], sc, &h[nb], &l[nb]);
         *(unsigned*)(p0 + (mb * 16 + v) * kLS) = *(const unsigned*)h;
         *(unsigned*)(p1 + (mb * 16 + v) * kLS) = *(const unsigned*)l;
       }
-    __syncthreads();  // the panel is ready
+    lds_barrier();  // the panel is ready
   };
 
   const long wpD = (long)kD * kD, wpP = (long)kProj * kD * kD;
   const f16* const W0 = planes(a.W[0], wpD);
-  const f16* const Wp = a.Wp ? planes(a.Wp, wpP) : W0;
+  const f16* const Wp = PROJ ? planes(a.Wp, wpP) : W0;
   int t = t0 + slot;
   if (t >= t1) return;
   {
@@ -390,50 +408,48 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
 #pragma unroll
     for (int j = 0; j < NJ; ++j) load_row(t, j, lane);
   }
+  // none outstanding from before the loop (vmcnt 0), so that its waits cover
+  // the loads of the tile before and not the stores behind them
+  __builtin_amdgcn_s_waitcnt(0x0F70);
   for (; t < t1; t += step) {
     // ---- the panel of O; wave w holds rows w, w + 8, ... ----
-    __syncthreads();  // every wave is done with the previous tile
+    lds_barrier();  // every wave is done with the previous tile
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       LANE
       float sc = kJScale;
-      if (j % (2 * MBU) == 0 && wave < ROW_J0) {
+      if (j == 0 && wave < ROW_J0) {
         const f32x4 v = aux[j];
         const float mx = wave_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
         float si;
         pow2_scale(mx, &sc, &si);
-        if (lane == 0) mx1[j / (2 * MBU) * 2 + wave] = si;
+        if (lane == 0) mx1[wave] = si;
       }
       f16 h[4], l[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float y = aux[j][e] * sc;
-        h[e] = (f16)y;
-        l[e] = (f16)(y - (float)h[e]);
-      }
+      for (int e = 0; e < 4; ++e) split(aux[j][e], sc, &h[e], &l[e]);
       const int at = (wave + kWaves * j) * kLS + 4 * lane;
       *(uint2*)(P0 + at) = *(const uint2*)h;
       *(uint2*)(P1 + at) = *(const uint2*)l;
     }
-    __syncthreads();
+    float* const xt = a.x + (long)t * BM * kD;
+    {
+      LANE
+      const int xoff = 4 * lg * kD + col;
 #pragma unroll
-    for (int u = 0; u < UPT; ++u) {
-      ival[u] = mx1[2 * u];
-      ilap[u] = mx1[2 * u + 1];
-    }
-    // ---- x1 = x + O Wo + bo, LN2 ----
-    const long row0 = (long)t * BM;
-    float* const xt = a.x + row0 * kD;
-    products(W0, wpD, planes(a.W[1], wpD), wpD, [&](int c, int lane) __attribute__((always_inline)) {
-      const int xoff = (lane >> 4) * 4 * kD + wave * 32 + 2 * (lane & 15);
-      if (c < MB && (UPT == 1 || row0 + (c / MBU + 1) * RU <= rows))
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float2 q = *(const float2*)(xt + (c * 16 + v) * kD + xoff);
-          aux[2 * c + v / 2][2 * (v & 1)] = q.x;
-          aux[2 * c + v / 2][2 * (v & 1) + 1] = q.y;
+          const f32x2 q = __builtin_nontemporal_load((const f32x2*)(xt + (mb * 16 + v) * kD + xoff));
+          aux[2 * mb + v / 2][2 * (v & 1)] = q.x;
+          aux[2 * mb + v / 2][2 * (v & 1) + 1] = q.y;
         }
-    });
+    }
+    lds_barrier();
+    ival = mx1[ROW_VAL];
+    ilap = mx1[ROW_LAP];
+    // ---- x1 = x + O Wo + bo, LN2 ----
+    products(W0, wpD, planes(a.W[1], wpD), wpD);
     unscale(0);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -451,7 +467,7 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
     for (int st = 1; st <= a.nm; ++st) {
       const bool last = st == a.nm;
       const f16* const Wn = last ? Wp : planes(a.W[st + 1], wpD);
-      products(planes(a.W[st], wpD), wpD, Wn, last && a.Wp ? wpP : wpD, [](int, int) {});
+      products(planes(a.W[st], wpD), wpD, Wn, last && PROJ ? wpP : wpD);
       unscale(st);
       tanh_rule();
       if (!last) put_panel();
@@ -461,21 +477,20 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
       const int xoff = 4 * lg * kD + col;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
-        if (UPT == 1 || row0 + (mb / MBU + 1) * RU <= rows)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
+        for (int v = 0; v < 4; ++v) {
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) acc[mb][nb][v] += aux[2 * mb + v / 2][2 * (v & 1) + nb];
-            *(float2*)(xt + (mb * 16 + v) * kD + xoff) = float2{acc[mb][0][v], acc[mb][1][v]};
-          }
+          for (int nb = 0; nb < 2; ++nb) acc[mb][nb][v] += aux[2 * mb + v / 2][2 * (v & 1) + nb];
+          __builtin_nontemporal_store(f32x2{acc[mb][0][v], acc[mb][1][v]}, (f32x2*)(xt + (mb * 16 + v) * kD + xoff));
+        }
     }
-    const int tn = t + step < t1 ? t + step : t;
-    if (!a.Wp) {
+    {  // the next tile's O
       LANE
+      const int tn = t + step < t1 ? t + step : t;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) load_row(tn, j, lane);
-      continue;
     }
+    if constexpr (!PROJ) continue;
     // ---- LN1 and the projection of the next layer ----
     layernorm(pln + 2 * kD);
     put_panel();
@@ -484,31 +499,20 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
       LANE
       const int n0 = cb * kD + wave * 32;  // 32 columns of one head
       const int prt = n0 / kD, hh = (n0 % kD) / a.dh, dd = n0 % a.dh;
+      const int w = t / a.N, i = t % a.N;
+      float* const y = a.Y + ((((long)w * kProj + prt) * a.H + hh) * a.N + i) * ((long)BM * a.dh) + dd;
+      const int yoff = 4 * lg * a.dh + 2 * lr;
 #pragma unroll
-      for (int u = 0; u < UPT; ++u) {
-        const int unit = t * UPT + u;
-        if (UPT > 1 && unit >= a.units) break;
-        const int w = unit / a.N, i = unit % a.N;
-        float* const yu = a.Y + ((((long)w * kProj + prt) * a.H + hh) * a.N + i) * ((long)RU * a.dh) + dd;
-        const int yoff = 4 * lg * a.dh + 2 * lr;
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int m = 0; m < MBU; ++m)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            *(float2*)(yu + (long)(m * 16 + v) * a.dh + yoff) = float2{acc[u * MBU + m][0][v], acc[u * MBU + m][1][v]};
-      }
+        for (int v = 0; v < 4; ++v)
+          __builtin_nontemporal_store(f32x2{acc[mb][0][v], acc[mb][1][v]},
+                                      (f32x2*)(y + (long)(mb * 16 + v) * a.dh + yoff));
     };
-    products(Wp, wpP, Wp + wpD, wpP, [&](int c, int lane) __attribute__((always_inline)) {
-      if (c < MB) {
-        load_row(tn, 2 * c, lane);
-        load_row(tn, 2 * c + 1, lane);
-      }
-    });
-    store(0);
 #pragma unroll 1
-    for (int cb = 1; cb < kProj; ++cb) {
+    for (int cb = 0; cb < kProj; ++cb) {
       const bool last = cb == kProj - 1;
-      products(Wp + cb * wpD, wpP, last ? W0 : Wp + (cb + 1) * wpD, last ? wpD : wpP, [](int, int) {});
+      products(Wp + cb * wpD, wpP, last ? W0 : Wp + (cb + 1) * wpD, last ? wpD : wpP);
       store(cb);
     }
   }
@@ -516,41 +520,27 @@ __global__ __launch_bounds__(kThreads, 2) void psi_chain_kernel(const PsiChainAr
 
 #undef LANE
 
-template <int MB, int MBU>
+template <bool PROJ>
 int launch_chain(const PsiChainArgs& a, hipStream_t s) {
-  constexpr int lds = chain_lds<MB>();
+  constexpr int lds = kLds;
   static_assert(lds <= 160 * 1024, "one workgroup per CU");
-  static const hipError_t attr = hipFuncSetAttribute((const void*)psi_chain_kernel<MB, MBU>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)psi_chain_kernel<PROJ>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return -1;
-  const int tiles = ceil_div(a.units, MB / MBU);
-  hipLaunchKernelGGL((psi_chain_kernel<MB, MBU>), dim3(kCus), dim3(kThreads), lds, s, a, tiles);
+  hipLaunchKernelGGL((psi_chain_kernel<PROJ>), dim3(kCus), dim3(kThreads), lds, s, a, a.units);
   return 0;
 }
-
 }  // namespace
 
+// 128-row units (32 to 42 electrons) alone: there the stages in a GEMM each round
+// alike, whatever the batch.  Both sides measured, energies of 42 electrons: 1 walker
+// 2785 us in separate launches, 2652 us here; 16 walkers 4147 and 3916 us; 64 walkers
+// 10180 and 8551 us.
 bool psi_chain_supported(int Rp, int D, int prec, int n_mlp, const int* width) {
-  if (prec != PREC_FP16X3 || D != kD || n_mlp < 1 || n_mlp > kChainMlp) return false;
+  if (prec != PREC_FP16X3 || Rp != 128 || D != kD || n_mlp < 1 || n_mlp > kChainMlp) return false;
   for (int j = 0; j <= n_mlp; ++j)
     if (width[j] != kD) return false;
-  return Rp == 128 || Rp == 96 || Rp == 64 || Rp == 48 || Rp == 32;
+  return true;
 }
 
-int launch_psi_chain(const PsiChainArgs& a, int Rp, hipStream_t s) {
-  // One unit a tile while every unit has a CU of its own; beyond that 96- and
-  // 128-row tiles, whose weights are read once for several units.  Both sides
-  // measured, energies: 10 electrons (32-row
-  // units) x 16 walkers 682 us in 128-row tiles, 547 us in 32-row tiles; 14 electrons
-  // x 16 walkers 751 and 696 us.  At any size below the separate launches' times
-  // (7 to 42 electrons, 1 to 768 walkers).
-  const bool few = a.units <= kCus;
-  switch (Rp) {
-    case 128: return launch_chain<8, 8>(a, s);
-    case 96: return launch_chain<6, 6>(a, s);
-    case 64: return few ? launch_chain<4, 4>(a, s) : launch_chain<8, 4>(a, s);
-    case 48: return few ? launch_chain<3, 3>(a, s) : launch_chain<6, 3>(a, s);
-    case 32: return few ? launch_chain<2, 2>(a, s) : launch_chain<8, 2>(a, s);
-  }
-  return -1;
-}
+int launch_psi_chain(const PsiChainArgs& a, hipStream_t s) { return a.Wp ? launch_chain<true>(a, s) : launch_chain<false>(a, s); }

@@ -467,7 +467,7 @@ int jq_model::forward_psiformer(const float* elec, int Bc, bool lap, hipStream_t
       }
       ca.eps = 1e-5f;
       ProfScope ps(PROF_GEMM_LAYER_LAP, s);
-      rc |= launch_psi_chain(ca, RP, s);
+      rc |= launch_psi_chain(ca, s);
       qkv_done = l + 1 < L;
       continue;
     }

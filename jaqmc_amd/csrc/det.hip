@@ -305,7 +305,7 @@ __device__ __forceinline__ void fwd_lu_steps(double (&m)[NP], int N, int lane, F
       const double pv = readlane_f64(x, piv);
       st.logdet.mul(pv);
       st.neg ^= pv < 0.0 ? 1 : 0;
-      const double l = (open && lane != piv) ? x / pv : 0.0;
+      const double l = (open && lane != piv) ? x / pivot_divisor(pv) : 0.0;
       // pivot-row entries read four at a time ahead of their multiply-adds, so
       // the scalar reads do not wait on each other
 #pragma unroll

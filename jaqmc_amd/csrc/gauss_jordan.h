@@ -13,8 +13,10 @@
 // log|prod_p v_p| over the pivots without one log per factor: the running
 // product is kept as a mantissa in [0.5, 1) and a binary exponent (both
 // factors split with frexp, so it neither overflows nor underflows), and one
-// log is taken at the end.  A zero pivot gives -inf, a NaN or inf pivot
-// propagates, as the sum of logs would.
+// log is taken at the end.  A zero factor gives -inf, a NaN or inf factor
+// propagates, as the sum of logs would.  The value-only eliminations go on past
+// a zero pivot (pivot_divisor), so a singular matrix gives -inf there; the ones
+// that form an inverse divide by it, and give NaN.
 struct LogAbsProduct {
   double m = 1.0;
   int e = 0;
@@ -26,6 +28,12 @@ struct LogAbsProduct {
   }
   __device__ double log_abs() const { return log(m) + (double)e * 0.69314718055994530942; }
 };
+
+// What a value-only elimination divides by.  Beside a zero pivot its column holds
+// nothing to eliminate: dividing by infinity gives zero, and the step leaves the
+// other columns as they are (0 / 0 would turn them, and the identity that pads
+// the matrix, into NaN); non-finite entries become NaN and stay in the result.
+__device__ inline double pivot_divisor(double pv) { return pv == 0.0 ? INFINITY : pv; }
 
 // Sign of the permutation perm[0 .. n-1] (n <= 64), from its cycles.
 __device__ inline int perm_sign(const int* perm, int n) {
@@ -274,7 +282,7 @@ __device__ __forceinline__ void fwd_col_steps(double (&m)[NP], LogAbsProduct& lo
       m[i] = sel ? mp : m[i];
       c[i] = sel ? cp : c[i];
     }
-    r /= pv;
+    r /= pivot_divisor(pv);
 #pragma unroll
     for (int i = P + 1; i < NP; ++i) m[i] = fma(-c[i], r, m[i]);
     fwd_col_steps<P + 1, NP>(m, logdet, neg);

@@ -670,3 +670,60 @@ def test_psiformer_row_wise_chain(cuda, n, B, kw):
     rel, bnd = el_report(f"chain {n}", out["e_loc"].cpu().numpy(), ref["e_loc"], kappa, "fp16x3", cancel)
     assert np.all(rel <= bnd), (rel, bnd)
     dm.close()
+
+
+# one determinant of three exactly singular: zero at once, from its first column,
+# at its last; full and not full sizes of the column-per-lane kernel, the
+# row-per-lane kernel; fp32 at up to 16 electrons: the one-kernel network
+@pytest.mark.parametrize("prec", ["fp32", "fp16x3"])
+@pytest.mark.parametrize("n", [2, 3, 4, 9, 13, 16, 17, 33])
+def test_singular_determinant_among_several(cuda, n, prec):
+    """log|psi| and its sign are those of the other determinants (slogdet of a
+    singular matrix is -inf), against the FP64 oracle to this file's bounds."""
+    import torch
+
+    sysm = S.h_chain(n)
+    _, spec, *_ = S.workload("li")
+    spec.nspins, spec.n_atoms = sysm.nspins, n
+    spec.hidden_single, spec.hidden_double, spec.ndets = [32, 32], [8, 8], 3
+    x = S.init_walkers(sysm, 7, seed=6)
+    at = sysm.atoms.astype(np.float64)
+    for orbitals in (slice(None), slice(0, 1), slice(n - 1, n)):
+        p = P.init_params(spec, seed=5, bias_scale=0.1, env_jitter=0.2)
+        for pi, _ in p["envelope"]:
+            pi[orbitals, :, 1] = 0.0  # these columns of determinant 1 vanish
+        p64 = P.cast_params(p, np.float64)
+        A = np.asarray(owf.orbital_matrices(spec.as_oracle(), p64, x.astype(np.float64), at))
+        assert np.all(np.linalg.slogdet(A[:, 1])[1] == -np.inf)
+        others = A[:, [0, 2]]
+        kappa, cancel = np.linalg.cond(others).max(axis=1), cancellation(others)
+        s, l = np.linalg.slogdet(others)
+        m = l.max(axis=1, keepdims=True)
+        total = (s * np.exp(l - m)).sum(axis=1)
+        ref = np.log(np.abs(total)) + m[:, 0]
+        dm = _model(sysm, spec, p, prec=prec, chunk=7)
+        lp, sg = dm.logpsi(torch.from_numpy(x).to(cuda))
+        d = np.abs(lp.cpu().numpy() - ref)
+        assert np.all(d <= logpsi_bound(ref, kappa, prec, cancel)), (orbitals, d)
+        np.testing.assert_array_equal(sg.cpu().numpy(), np.sign(total))
+        dm.close()
+
+
+def test_singular_walker_with_a_nan_stays_nan(cuda):
+    """A zero column does not hide a NaN in the matrix."""
+    import torch
+
+    for n in (3, 17):
+        sysm = S.h_chain(n)
+        _, spec, *_ = S.workload("li")
+        spec.nspins, spec.n_atoms = sysm.nspins, n
+        spec.hidden_single, spec.hidden_double, spec.ndets = [32, 32], [8, 8], 1
+        p = P.init_params(spec, seed=5, bias_scale=0.1, env_jitter=0.2)
+        for pi, _ in p["envelope"]:
+            pi[0] = 0.0
+            pi[1] = np.nan
+        for prec in ("fp32", "fp16x3"):
+            dm = _model(sysm, spec, p, prec=prec, chunk=7)
+            lp, _ = dm.logpsi(torch.from_numpy(S.init_walkers(sysm, 7, seed=6)).to(cuda))
+            assert torch.isnan(lp).all(), (n, prec)
+            dm.close()

@@ -12,11 +12,14 @@
 extern "C" {
 #endif
 
-#define JQ_PROF_GEMM_LAYER_LAP 0 /* one-electron layer GEMMs, Laplacian mode */
+#define JQ_PROF_GEMM_LAYER_LAP 0 /* one-electron layer GEMMs, Laplacian mode; a Psiformer layer's
+                                    whole row-wise part where one kernel runs it */
 #define JQ_PROF_DET_LAP 1        /* determinant + Laplacian kernel          */
 #define JQ_PROF_GEMM_ORB_LAP 2   /* orbital projection GEMMs, Laplacian mode */
-#define JQ_PROF_PAIR_LAP 3       /* two-electron stream, Laplacian mode      */
-#define JQ_PROF_FORWARD 4        /* whole log|psi| chunk                     */
+#define JQ_PROF_PAIR_LAP 3       /* two-electron stream, Laplacian mode; with its means where it
+                                    stays on chip                            */
+#define JQ_PROF_FORWARD 4        /* whole log|psi| chunk; a small network's Metropolis moves of one
+                                    call (jq_sample: of one outer step) are one launch */
 #define JQ_PROF_LOCAL_ENERGY 5   /* whole local-energy chunk                 */
 #define JQ_PROF_ATTN_LAP 6       /* Psiformer attention, Laplacian mode      */
 

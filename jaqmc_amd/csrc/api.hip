@@ -12,6 +12,7 @@
 #include "../../include/jaqmc_amd.h"
 #include "kernels.h"
 #include "model.h"
+#include "prof.h"
 
 thread_local std::string g_jq_err;
 
@@ -191,8 +192,11 @@ int jq_logpsi(jq_model* m, const float* elec, int B, float* logpsi, float* sign,
   if (B == 0) return JQ_OK;
   hipStream_t s = (hipStream_t)stream;
   const bool small = m->use_small(B);
-  if (small && launch_small_logpsi(m->small, elec, B, logpsi, sign, s))
-    return jq_fail(JQ_EHIP, "jq_logpsi: small-network launch rejected");
+  if (small) {
+    ProfScope ps(PROF_FORWARD, s);
+    if (launch_small_logpsi(m->small, elec, B, logpsi, sign, s))
+      return jq_fail(JQ_EHIP, "jq_logpsi: small-network launch rejected");
+  }
   for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {
     const int Bc = std::min(m->chunk_fwd, B - b0);
     int rc = m->forward(elec, b0, Bc, false, logpsi, sign, nullptr, nullptr, nullptr, nullptr, s);
@@ -254,6 +258,7 @@ int jq_mh_steps(jq_model* m, float* elec, float* logp, int B, int n_steps, float
   const bool small = m->use_small(B);
   if (small) {
     const SmallMoves mv{elec, logp, B, n_steps, width, nullptr, normals, uniforms, seed, ctr, n_accept, 0};
+    ProfScope ps(PROF_FORWARD, s);
     if (launch_small_moves(m->small, mv, s)) return jq_fail(JQ_EHIP, "jq_mh_steps: small-network launch rejected");
   }
   for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {
@@ -287,6 +292,7 @@ int jq_sample(jq_model* m, float* elec, float* logp, int B, int n_outer, int ste
     if (small) {
       const SmallMoves mv{elec, logp,    B,        steps, 0.f, state, nullptr, nullptr, seed, ctr + (uint64_t)o * steps,
                           n_accept, 1};
+      ProfScope ps(PROF_FORWARD, s);
       if (launch_small_moves(m->small, mv, s)) return jq_fail(JQ_EHIP, "jq_sample: small-network launch rejected");
     }
     for (int b0 = 0; b0 < B && !small; b0 += m->chunk_fwd) {

@@ -3,11 +3,11 @@
 #include <hip/hip_runtime.h>
 
 enum ProfClass {
-  PROF_GEMM_LAYER_LAP = 0,  // one-electron layer GEMMs, Laplacian mode
+  PROF_GEMM_LAYER_LAP = 0,  // one-electron layer GEMMs or layer kernels, Laplacian mode
   PROF_DET_LAP = 1,         // determinant + Laplacian kernel
   PROF_GEMM_ORB_LAP = 2,    // orbital projection GEMMs, Laplacian mode
-  PROF_PAIR_LAP = 3,        // two-electron stream layers, Laplacian mode
-  PROF_FORWARD = 4,         // one whole forward (log|psi|) chunk
+  PROF_PAIR_LAP = 3,        // two-electron stream layers (on chip: with its means), Laplacian mode
+  PROF_FORWARD = 4,         // one whole forward (log|psi|) chunk, or the moves of a small network
   PROF_LOCAL_ENERGY = 5,    // one whole local-energy chunk
   PROF_ATTN_LAP = 6,        // Psiformer attention kernels, Laplacian mode
   PROF_NCLASS = 8

@@ -727,3 +727,29 @@ def test_singular_walker_with_a_nan_stays_nan(cuda):
             lp, _ = dm.logpsi(torch.from_numpy(S.init_walkers(sysm, 7, seed=6)).to(cuda))
             assert torch.isnan(lp).all(), (n, prec)
             dm.close()
+
+
+def test_small_network_launches_are_profiled(cuda):
+    """JQ_PROF_FORWARD records the value path of a small network: one launch of
+    log|psi|, one for the moves of a call, one per outer step of the sampler."""
+    import torch
+
+    from jaqmc_amd import _lib
+
+    sysm, spec, *_ = S.workload("li")
+    dm = _model(sysm, spec, P.init_params(spec, seed=0, bias_scale=0.1))
+    x = torch.from_numpy(S.init_walkers(sysm, 64, seed=1)).to(cuda)
+    logp = 2 * dm.logpsi(x)[0]
+    state = torch.zeros(3 + 4, dtype=torch.float64, device=cuda)
+    state[0] = 0.2
+    counts = []
+    for call in (lambda: dm.logpsi(x), lambda: dm.mh_steps(x, logp, 5, 0.1, seed=2),
+                 lambda: dm.sample(x, state, 2, 3, adapt_frequency=4, seed=9)):
+        _lib.profile_enable(True)
+        call()
+        _lib.profile_enable(False)
+        ms, n = _lib.profile_read("forward")
+        assert ms > 0
+        counts.append(n)
+    assert counts == [1, 1, 2]
+    dm.close()

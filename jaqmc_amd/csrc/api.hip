@@ -191,7 +191,7 @@ int jq_logpsi(jq_model* m, const float* elec, int B, float* logpsi, float* sign,
   if (!m || B < 0 || (B > 0 && (!elec || !logpsi))) return jq_fail(JQ_EINVAL, "jq_logpsi: bad argument");
   if (B == 0) return JQ_OK;
   hipStream_t s = (hipStream_t)stream;
-  const bool small = m->use_small(B);
+  const bool small = m->use_small(B, false);
   if (small) {
     ProfScope ps(PROF_FORWARD, s);
     if (launch_small_logpsi(m->small, elec, B, logpsi, sign, s))
@@ -255,7 +255,7 @@ int jq_mh_steps(jq_model* m, float* elec, float* logp, int B, int n_steps, float
   // walker chunks outermost: each chunk makes all its moves through the
   // model's one-chunk proposal scratch (walkers are independent and the
   // Philox streams are keyed by the global walker index)
-  const bool small = m->use_small(B);
+  const bool small = m->use_small(B, true);
   if (small) {
     const SmallMoves mv{elec, logp, B, n_steps, width, nullptr, normals, uniforms, seed, ctr, n_accept, 0};
     ProfScope ps(PROF_FORWARD, s);
@@ -287,7 +287,7 @@ int jq_sample(jq_model* m, float* elec, float* logp, int B, int n_outer, int ste
   if (B == 0 || n_outer == 0 || steps == 0) return JQ_OK;  // MCMCSampler.step with steps == 0 is a no-op
   hipStream_t s = (hipStream_t)stream;
   const long n3 = 3L * m->N;
-  const bool small = m->use_small(B);
+  const bool small = m->use_small(B, true);
   for (int o = 0; o < n_outer; ++o) {
     if (small) {
       const SmallMoves mv{elec, logp,    B,        steps, 0.f, state, nullptr, nullptr, seed, ctr + (uint64_t)o * steps,

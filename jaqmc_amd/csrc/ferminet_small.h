@@ -18,11 +18,12 @@ struct SmallNet {
   const float* Worb[2];  // per channel: (K N, korb) transposed
   const float *pi[2], *sigma[2];
   const float* atoms;
-  int G;  // walkers per workgroup
+  int G;                      // walkers per workgroup
+  int max_groups, max_moves;  // workgroups up to which log|psi|, and the moves, are the faster path
   // LDS layout, in floats
   int ldx, ldg, ldG, ldh, ldo, o_X[2], o_g, o_G, o_h2[2], o_phi, o_env, o_geo, o_det, o_misc, lds_floats;
 };
-// Fills G and the LDS layout; false where the network does not fit the kernel.
+// Fills G, the lines and the LDS layout; false where the network does not fit the kernel.
 bool small_net_plan(SmallNet& n);
 
 // log|psi| and sign (sign may be null) of B walkers.

@@ -324,6 +324,39 @@ __global__ __launch_bounds__(kThreads) void small_moves_kernel(SmallNet n, Small
   }
 }
 
+// Workgroups up to which this path is the faster one.  A CU runs a round of as many
+// as its LDS holds at once, two at most in the moves (their registers); every round
+// takes the same time, while the general path's launches cost `layer_us` a layer and
+// once more for the features and determinants, and little more for more walkers.  One
+// round is always taken, further ones while they fit that.  The time of a round is an
+// estimate, within 4 % (mean) of the moves of 152 networks of 1 to 16 electrons: steps
+// between barriers, a wave's 32 x 64 chunks of weights, pair products, envelope terms,
+// elimination.  Where three workgroups fit a CU every launch measured, up to five per
+// CU, was faster.
+int faster_groups(const SmallNet& n, double layer_us) {
+  constexpr int kCus = 256, kCuLds = 160 * 1024;
+  const int fit = kCuLds / (n.lds_floats * 4);
+  if (fit >= 3) return 5 * kCus;
+  const int rows = n.G * n.N, KN = n.K * n.N, np = round_up(n.N, 4);
+  long chunks = (long)n.nch * ceil_div(KN, 64) * (n.korb / 32), pair = 0;
+  for (int l = 0; l < n.L; ++l) {
+    const SmallLayer& y = n.l[l];
+    chunks += (long)ceil_div(y.d1, 64) * ((y.kmain + y.kg) / 32);
+    if (y.W2) pair += (long)ceil_div((long)rows * n.N * y.d2, kThreads) * y.f2;
+  }
+  const long env = (long)ceil_div((long)rows * KN, kThreads) * n.M;
+  const long det = (long)ceil_div((long)n.G * n.K, kThreads / 16) * np * np;
+  const double round_us = 3.2 + 4.8 * n.L + 0.31 * chunks + 0.08 * pair + 0.11 * env + 0.036 * det;
+  const int rounds = std::max(1, (int)(layer_us * (1 + n.L) / round_us));
+  return std::min(5, std::min(fit, 2) * rounds) * kCus;
+}
+// Measured, here and in the general path (us), four determinants: layers 2 x 64, three
+// electrons, log|psi| of 1280 walkers 24 and 67, 6400 48 and 111; fourteen, 512 43 and
+// 93, 1024 80 and 106, general from there (1280: 108 and 118).  Ten moves: 4 x 128,
+// fourteen electrons, 512 walkers 1181 and 1748, general from there (640: 2103 and
+// 1839); sixteen, one workgroup per CU, 256 1104 and 1625, 384 2194 and 1732.
+constexpr double kLayerUs = 28.0, kMoveLayerUs = 36.0;
+
 }  // namespace
 
 bool small_net_plan(SmallNet& n) {
@@ -362,7 +395,10 @@ bool small_net_plan(SmallNet& n) {
   n.o_det = take(4L * n.G * n.K);
   n.o_misc = take(2L * kRows * 3 + 4 * kRows);  // positions, proposals; log|psi|, sign, logp, decisions
   n.lds_floats = at;
-  return (size_t)at * 4 <= kMaxLds;
+  if ((size_t)at * 4 > kMaxLds) return false;
+  n.max_groups = faster_groups(n, kLayerUs);
+  n.max_moves = faster_groups(n, kMoveLayerUs);
+  return true;
 }
 
 template <typename K>

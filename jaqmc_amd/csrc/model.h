@@ -98,12 +98,10 @@ struct jq_model {
   bool pairs_on_chip = false;  // launch_pair_stream instead of a pair stream in H2
   SmallNet small{};
   bool small_ok = false;       // the value path also runs as one kernel (ferminet_small.hip)
-  // Whether a batch of B walkers takes it: up to five workgroups per CU (what
-  // their LDS lets run at once), where launches bound the general path.  Three
-  // electrons, log|psi| of 1024 walkers: 25 us (general path 71), of 4096: 46 (92);
-  // general 123 of 8192.  Fourteen, 256 walkers: 37 us (80), 1024: 77 (101);
-  // general 130 of 2048.
-  bool use_small(int B) const { return small_ok && B <= 5L * 256 * small.G; }
+  // Whether log|psi|, or the moves, of B walkers take it (small_net_plan)
+  bool use_small(int B, bool moves) const {
+    return small_ok && B <= (long)(moves ? small.max_moves : small.max_groups) * small.G;
+  }
   // Psiformer
   std::vector<PsiLayer> pl;
   int D = 0, H = 0, dh = 0, kin = 0;  // model dim, heads, head dim, padded input K

@@ -753,3 +753,35 @@ def test_small_network_launches_are_profiled(cuda):
         counts.append(n)
     assert counts == [1, 1, 2]
     dm.close()
+
+
+# workgroups (16 // electrons walkers each) on both sides of the lines between the
+# one-kernel path and the general one: log|psi|, moves
+@pytest.mark.parametrize("n,width,layers,most,most_moves", [
+    (3, 64, 2, 1280, 1280), (14, 64, 2, 1024, 1024), (14, 96, 2, 512, 1024), (14, 128, 4, 512, 512),
+    (16, 128, 4, 256, 256), (10, 192, 2, 256, 512), (3, 256, 2, 256, 512)])
+def test_small_network_kernel_ends_where_it_loses(cuda, n, width, layers, most, most_moves):
+    """A batch takes one launch up to the workgroups that a CU works off faster
+    than the general path's launches, and that path's chunks beyond."""
+    import torch
+
+    from jaqmc_amd import _lib
+
+    sysm = S.h_chain(n)
+    _, spec, *_ = S.workload("li")
+    spec.nspins, spec.n_atoms, spec.ndets = sysm.nspins, n, 4
+    spec.hidden_single, spec.hidden_double = [width] * layers, [16] * layers
+    dm = _model(sysm, spec, P.init_params(spec, seed=0, bias_scale=0.1), chunk=1)
+
+    def launches(walkers, moves):
+        x = torch.from_numpy(S.init_walkers(sysm, walkers, seed=1)).to(cuda)
+        logp = torch.zeros(walkers, device=cuda)
+        _lib.profile_enable(True)
+        dm.mh_steps(x, logp, 1, 0.1, seed=2) if moves else dm.logpsi(x)
+        _lib.profile_enable(False)
+        return _lib.profile_read("forward")[1]
+
+    G = 16 // n
+    got = [launches(w, moves) for moves, line in ((False, most), (True, most_moves)) for w in (line * G, line * G + 1)]
+    dm.close()
+    assert got[0] == got[2] == 1 and got[1] > 1 and got[3] > 1, got

@@ -32,7 +32,10 @@ int jq_profile_read(int cls, double* total_ms, int* count);
 /* Time `reps` launches of the tangent GEMM kernel on synthetic zero buffers:
  * Y (rows x ncols) = X (rows x K) W^T, R tangent rows per unit (1: plain rows),
  * act 0/1 (none/tanh rule), prec JQ_PREC_*, variant 0 (default tiling) or
- * 10*units_per_tile + col_blocks_per_wave.  Average milliseconds -> *ms. */
+ * 10*units_per_tile + col_blocks_per_wave (-1 where there is no such tile).  Plain
+ * rows: 10*row_blocks + col_blocks, tiles of 16*row_blocks x 64*col_blocks, of which
+ * there are 11, 21, 41 and, but for FP32, 82; any other variant times the default
+ * tiling.  Average milliseconds -> *ms. */
 int jq_bench_gemm(int prec, int R, int rows, int K, int ncols, int act, int variant, int reps, float* ms);
 
 #ifdef __cplusplus

@@ -45,7 +45,7 @@
 
 #include "kernels.h"
 
-// 0: default tile table; else UPT*10 + NBW, plain rows MB*10 + NBW (benchmark override)
+// 0: default tile table; else UPT*10 + NBW, plain rows MB*10 + NBW where there is such a tile (benchmark override)
 extern int g_gemm_variant;
 // 4: no eight-wave tiles (benchmark override); 0: default
 extern int g_gemm_nw;
@@ -976,7 +976,8 @@ void default_cfg(int R, int prec, bool wide, int* upt, int* nbw) {
 }
 
 // Tile of a plain (value-row) launch: 16 mb rows x 64 nbw columns, from sweeps
-// on MI355X (jq_bench_gemm; every tile gives the same bits).  A CU works its
+// on MI355X (jq_bench_gemm; every tile gives the same bits; 64 x 128 tiles, and
+// 128 x 128 in FP32, are the ones that this table replaced).  A CU works its
 // tiles off at the matrix rate, so the time follows the most tiles a CU gets:
 // the largest tile only where it leaves every CU enough of them.
 //   FP32: 64 x 64 from two tiles per CU on (10752 rows, K = N = 256: 20.4 us,
@@ -1010,21 +1011,19 @@ int dispatch(const GemmArgs& a, hipStream_t s) {
   const bool wide = a.ncols > 128;
   if (a.R <= 1) {
     if (a.Yln) return -1;
-    int mb, nbw;
-    plain_cfg<PREC>(a, &mb, &nbw);
-    if (g_gemm_variant > 0) {
-      mb = g_gemm_variant / 10;
-      nbw = g_gemm_variant % 10;
+    int tile = g_gemm_variant;
+    if (!(tile == 11 || tile == 21 || tile == 41 || (tile == 82 && PREC != PREC_F32))) {  // none of its own
+      int mb, nbw;
+      plain_cfg<PREC>(a, &mb, &nbw);
+      tile = 10 * mb + nbw;
     }
-    switch (10 * mb + nbw) {
+    switch (tile) {
       case 82:
-        if constexpr (PREC == PREC_F32) return -1;
-        else launch_one<8, 1, 2, PREC, false>(a, s);
+        if constexpr (PREC != PREC_F32) launch_one<8, 1, 2, PREC, false>(a, s);
         break;
       case 41: launch_one<4, 1, 1, PREC, false>(a, s); break;
       case 21: launch_one<2, 1, 1, PREC, false>(a, s); break;
-      case 11: launch_one<1, 1, 1, PREC, false>(a, s); break;
-      default: return -1;
+      default: launch_one<1, 1, 1, PREC, false>(a, s); break;
     }
     return 0;
   }

@@ -785,3 +785,25 @@ def test_small_network_kernel_ends_where_it_loses(cuda, n, width, layers, most, 
     got = [launches(w, moves) for moves, line in ((False, most), (True, most_moves)) for w in (line * G, line * G + 1)]
     dm.close()
     assert got[0] == got[2] == 1 and got[1] > 1 and got[3] > 1, got
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16", "bf16x3", "bf16x6", "fp16x3"])
+def test_bench_gemm_takes_every_plain_variant(cuda, prec):
+    """jq_bench_gemm times plain rows with any variant: the tile it names, or the
+    default where there is none of that name; Laplacian rows only with a tile."""
+    import ctypes
+
+    from jaqmc_amd import _lib
+
+    lib = _lib.load()
+    ms = ctypes.c_float()
+
+    def bench(R, variant):
+        ms.value = -1.0
+        rc = lib.jq_bench_gemm(_lib.PRECISION[prec], R, 960, 64, 96, 0, variant, 2, ctypes.byref(ms))
+        return rc, ms.value
+
+    for variant in (0, 11, 21, 41, 82, 12, 42, 14, 24, 84, 142):
+        rc, t = bench(1, variant)
+        assert rc == 0 and t > 0, variant
+    assert bench(48, 22)[0] == 0 and bench(48, 91)[0] == -1

@@ -61,6 +61,10 @@ extern "C" {
  * workspace at create, for jq_logpsi_vjp (FermiNet with hidden widths
  * multiples of 32; Psiformer with N <= 64 and heads_dim 32 or 64). */
 #define JQ_OPT_WITH_GRADIENTS (1 << 16)
+/* Library option: every stage of the network in a launch of its own, without the
+ * kernels that run several (the row-wise part of a Psiformer layer, the value path
+ * of a small FermiNet).  The results are the same bit for bit; for comparisons. */
+#define JQ_OPT_SEPARATE_LAUNCHES (1 << 17)
 
 /* Arithmetic of the layer / tangent GEMMs.  Determinants (LU, inverse,
  * Laplacian traces) and walker reductions are FP64 in every mode. */

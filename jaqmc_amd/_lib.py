@@ -25,6 +25,7 @@ OPT_NO_RESCALE = 1 << 3
 OPT_SHARED_ORBITALS = 1 << 4
 OPT_USE_LAST_LAYER = 1 << 5
 OPT_WITH_GRADIENTS = 1 << 16
+OPT_SEPARATE_LAUNCHES = 1 << 17
 
 EXPORTS = (
     "jq_model_create", "jq_model_destroy", "jq_model_workspace_bytes", "jq_logpsi", "jq_mh_steps",

@@ -46,7 +46,7 @@ int jq_model::init(const jq_model_desc& desc, const float* packed, size_t n_floa
   options = desc.options;
   ln_mode = desc.layer_norm_mode;
   const int known = JQ_OPT_NO_ATTN_BIAS | JQ_OPT_NO_INPUT_BIAS | JQ_OPT_ORBITAL_BIAS | JQ_OPT_NO_RESCALE |
-                    JQ_OPT_SHARED_ORBITALS | JQ_OPT_USE_LAST_LAYER | JQ_OPT_WITH_GRADIENTS;
+                    JQ_OPT_SHARED_ORBITALS | JQ_OPT_USE_LAST_LAYER | JQ_OPT_WITH_GRADIENTS | JQ_OPT_SEPARATE_LAUNCHES;
   if (options & ~known) return jq_fail(JQ_EINVAL, "unknown option bits");
   if (options & JQ_OPT_USE_LAST_LAYER)
     return jq_fail(JQ_EINVAL, "FermiNet use_last_layer=True (aggregated orbital input) is not supported");
@@ -212,7 +212,7 @@ int jq_model::init_ferminet(const float* packed, size_t n_floats) {
     if (norb == 1) Worb_o[1] = Worb_o[0];
   }
 
-  if (prec == JQ_PREC_FP32 && L <= kSmallLayers) {
+  if (prec == JQ_PREC_FP32 && L <= kSmallLayers && !(options & JQ_OPT_SEPARATE_LAUNCHES)) {
     SmallNet& n = small;
     n.L = L;
     n.N = N;

@@ -3,7 +3,8 @@
 //   x1 = x + O Wo + bo;  t = LN2(x1);  t = tanh(t Wm + bm), ...;  x = x1 + t;
 //   QKV = LN1'(x) Wqkv' + bqkv'   (the next layer's, head-split; none after the last)
 // by the forward-Laplacian rules of gemm_kernel, in its order: the results are the same
-// bit for bit as those of a GEMM a stage with the LayerNorms in their epilogues.
+// bit for bit as those of a GEMM a stage with the LayerNorms in their epilogues
+// (JQ_OPT_SEPARATE_LAUNCHES; test_psiformer_chain_is_bit_identical holds both to it).
 //
 // Bound by the FP16 matrix rate, the LayerNorms and the memory together: as one
 // GEMM a stage, with the LayerNorms in their epilogues, a layer read and wrote

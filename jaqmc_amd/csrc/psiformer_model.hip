@@ -439,7 +439,8 @@ int jq_model::forward_psiformer(const float* elec, int Bc, bool lap, hipStream_t
     }
     // Everything from the output projection to the next layer's q, k, v is
     // row-wise: one launch where the kernel takes the widths.
-    if (lap && ln_mode == JQ_LN_PRE && psi_chain_supported(RP, D, prec, nm, ly.mdims.data())) {
+    if (lap && ln_mode == JQ_LN_PRE && !(options & JQ_OPT_SEPARATE_LAUNCHES) &&
+        psi_chain_supported(RP, D, prec, nm, ly.mdims.data())) {
       PsiChainArgs ca{};
       ca.O = Om;
       ca.ldo = DO;

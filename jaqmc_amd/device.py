@@ -34,10 +34,13 @@ class DeviceModel:
     column scaling for FP16's range; value-only launches use bf16x6).  Every
     mode accumulates in FP32 and keeps activations FP32 in HBM; determinants,
     E_L assembly and reductions are FP64 in every mode.
+
+    separate_launches: every stage of the network in a launch of its own, also
+    where one kernel runs several (the same results bit for bit).
     """
 
     def __init__(self, spec: ModelSpec, atoms, charges, params, precision="fp32", chunk_walkers=0,
-                 with_gradients=False):
+                 with_gradients=False, separate_launches=False):
         lib = _lib.load()
         if not torch.cuda.is_available():
             raise _lib.JqError("DeviceModel needs a ROCm GPU (torch.cuda.is_available() is False)")
@@ -68,6 +71,7 @@ class DeviceModel:
         d.precision = _lib.PRECISION[precision]
         d.layer_norm_mode = _lib.LAYER_NORM[spec.layer_norm_mode] if spec.kind == "psiformer" else 0
         d.options = spec.options() | (_lib.OPT_WITH_GRADIENTS if with_gradients else 0)
+        d.options |= _lib.OPT_SEPARATE_LAUNCHES if separate_launches else 0
         d.chunk_walkers = int(chunk_walkers)
         d.atoms = self.atoms.ctypes.data_as(ctypes.POINTER(ctypes.c_float))
         d.charges = self.charges.ctypes.data_as(ctypes.POINTER(ctypes.c_float))

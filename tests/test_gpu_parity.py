@@ -807,3 +807,74 @@ def test_bench_gemm_takes_every_plain_variant(cuda, prec):
         rc, t = bench(1, variant)
         assert rc == 0 and t > 0, variant
     assert bench(48, 22)[0] == 0 and bench(48, 91)[0] == -1
+
+
+# as test_psiformer_row_wise_chain, and heads of 128, several units a workgroup,
+# every remainder of an MLP's depth
+@pytest.mark.parametrize("n,B,kw", [
+    (32, 2, dict(num_layers=2, mlp_hidden=[])),
+    (33, 9, dict(num_layers=2, mlp_hidden=[256, 256])),
+    (35, 1, dict(num_layers=2, num_heads=2, heads_dim=128)),
+    (37, 3, dict(num_layers=3, num_heads=8, heads_dim=32)),
+    (39, 20, dict(num_layers=1)),
+    (42, 13, dict(num_layers=4)),
+    (42, 2, dict(num_layers=2, mlp_hidden=[256, 256, 256])),
+])
+def test_psiformer_chain_is_bit_identical(cuda, n, B, kw):
+    """Layers whose row-wise part runs in one kernel and the same layers in a
+    launch a stage: the same log|psi|, energies and gradients."""
+    import torch
+
+    from jaqmc_amd.device import DeviceModel
+
+    sysm = S.h_chain(n)
+    _, spec, *_ = S.workload("ring42")
+    spec.nspins, spec.n_atoms, spec.ndets = sysm.nspins, n, 2
+    for k, v in kw.items():
+        setattr(spec, k, v)
+    p = P.init_params(spec, seed=121, bias_scale=0.1, env_jitter=0.3)
+    x = torch.from_numpy(S.init_walkers(sysm, B, seed=122)).to(cuda)
+    out = []
+    for separate in (False, True):
+        dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, precision="fp16x3", chunk_walkers=B,
+                         separate_launches=separate)
+        out.append(dm.local_energy(x, with_grad=True))
+        torch.cuda.synchronize()
+        dm.close()
+    for k, v in out[0].items():
+        assert torch.equal(v, out[1][k]), k
+    assert torch.isfinite(out[0]["e_loc"]).all()
+
+
+def test_separate_launches_run_the_stages_apart(cuda):
+    """JQ_OPT_SEPARATE_LAUNCHES: more layer launches for the Psiformer, chunks in
+    place of the one-kernel value path for a small FermiNet."""
+    import torch
+
+    from jaqmc_amd import _lib
+    from jaqmc_amd.device import DeviceModel
+
+    sysm, spec, *_ = S.workload("ring42")
+    p = P.init_params(spec, seed=0)
+    counts = []
+    for separate in (False, True):
+        dm = DeviceModel(spec, sysm.atoms, sysm.charges, p, precision="fp16x3", chunk_walkers=2,
+                         separate_launches=separate)
+        x = torch.from_numpy(S.init_walkers(sysm, 2, seed=1)).to(cuda)
+        dm.local_energy(x)
+        _lib.profile_enable(True)
+        dm.local_energy(x)
+        _lib.profile_enable(False)
+        counts.append(_lib.profile_read("gemm_layer_lap")[1])
+        dm.close()
+    L, stages = spec.num_layers, 2 + len(spec.mlp_hidden) + 1  # q k v, output projection, MLP
+    assert counts == [1 + 1 + L, 1 + L * stages]  # the input projection; its first q k v; the layers
+    sysm, spec, *_ = S.workload("li")
+    dm = DeviceModel(spec, sysm.atoms, sysm.charges, P.init_params(spec, seed=0), chunk_walkers=1,
+                     separate_launches=True)
+    x = torch.from_numpy(S.init_walkers(sysm, 400, seed=1)).to(cuda)
+    _lib.profile_enable(True)
+    dm.logpsi(x)
+    _lib.profile_enable(False)
+    assert _lib.profile_read("forward")[1] > 1
+    dm.close()

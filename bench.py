@@ -35,10 +35,11 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 
 
-def measured_traffic(workload: str, mixed: str):
-    """HBM bytes per dispatch of the mixed-precision layer GEMM of this workload,
+def measured_traffic(workload: str, mixed: str, kernel: str):
+    """HBM bytes per dispatch of this workload's mixed-precision layer launches,
     from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary (copy-calibrated;
-    see jaqmc_amd/profiling.py), or None when no summary is committed."""
+    see jaqmc_amd/profiling.py), or None when no summary of launches of `kernel`
+    is committed."""
     for name in (f"gemm_layer_lap_{workload}_{mixed}_traffic.txt", f"gemm_layer_lap_{workload}_traffic.txt"):
         path = os.path.join(ROOT, "profiles", name)
         if not os.path.exists(path):
@@ -47,6 +48,8 @@ def measured_traffic(workload: str, mixed: str):
             txt = f.read()
         if mixed not in txt and name.endswith(f"{workload}_traffic.txt") and mixed != "bf16x6":
             continue  # the generic summary is the bf16x6 kernel's
+        if not any(line.startswith("Kernel:") and kernel in line for line in txt.splitlines()):
+            continue  # of another kernel than the one that runs
         for line in txt.splitlines():
             if line.startswith("traffic_bytes_per_dispatch:"):
                 return float(line.split(":", 1)[1]), "profiles/" + name
@@ -300,8 +303,8 @@ def main():
         acc_info = fixture_accuracy(spec, system, params, args.workload, ("fp32", args.mixed), width)
         log("accuracy:", json.dumps(acc_info))
 
-    # --- roofline of the dominant kernel class (layer GEMMs in Laplacian mode) ---
-    # achieved = algorithmic FLOPs of all layer-GEMM launches in the timed region
+    # --- roofline of the dominant kernel class (dense layers in Laplacian mode) ---
+    # achieved = algorithmic FLOPs of all layer launches in the timed region
     # / their summed device time (HIP events on the launching stream)
     fl = RF.flops(spec, system.atoms.shape[0])
     mixed = res[args.mixed]
@@ -310,7 +313,8 @@ def main():
     peak = RF.PEAKS[RF.MODE_PEAK[args.mixed]]
     mult = RF.MFMA_PER_PRODUCT[args.mixed]
     alg_bytes = RF.layer_bytes(spec, system.atoms.shape[0], args.mixed) * B * args.steps
-    traffic, traffic_src = measured_traffic(args.workload, args.mixed)
+    layer_kernel = RF.layer_kernel(spec, args.mixed)
+    traffic, traffic_src = measured_traffic(args.workload, args.mixed, layer_kernel)
     avg_s = tot_ms * 1e-3 / max(n, 1)
     # the binding roof: the larger of the minimum MFMA time (algorithmic
     # FLOPs x MFMAs per product at the mode's dense peak) and the minimum HBM
@@ -331,7 +335,7 @@ def main():
             "alg_bytes_per_launch": alg_bytes / max(n, 1),
             "hbm_frac_alg_bytes": (alg_bytes / (tot_ms * 1e-3) / RF.PEAKS["hbm"]) if n else 0.0,
             "hbm_frac_measured_traffic": (traffic / avg_s / RF.PEAKS["hbm"]) if (n and traffic) else None,
-            "kernel": f"gemm_kernel ({spec.kind} dense layers, Laplacian mode, {args.mixed})",
+            "kernel": f"{layer_kernel} ({spec.kind} dense layers, Laplacian mode, {args.mixed})",
             "avg_launch_ms": tot_ms / max(n, 1), "launches": n,
             "per_class_ms_per_step": {k: v[0] / args.steps for k, v in mixed["prof"].items()},
             "fp32_per_class_ms_per_step": {k: v[0] / args.steps for k, v in res["fp32"]["prof"].items()}}

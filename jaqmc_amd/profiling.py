@@ -10,7 +10,8 @@ calibrated against a plain device copy of known size recorded in the same runs
     python -m jaqmc_amd.profiling stats  <run_results.db> "<command>" "<title>"
     python -m jaqmc_amd.profiling traffic <fetch.db> <write.db> <kernel-substring> <copy-bytes> "<commands>" "<title>" [<exclusions>]
 
-Exclusions (comma-separated) name dispatches of another launch class of the
+The kernel substring may be several, joined by `|`.  Exclusions
+(comma-separated) name dispatches of another launch class of the
 same kernel instantiation, such as the orbital projection beside the layer
 GEMMs: `g<grid size>` or `d<ordinal>` (0-based among the matching
 dispatches).  They are listed but not averaged.
@@ -49,7 +50,7 @@ def _dispatches(db: str, counter: str, kernel: str):
     con = sqlite3.connect(db)
     rows = con.execute("select kernel_name, grid_size, value from counters_collection where counter_name = ? "
                        "order by dispatch_id", (counter,))
-    return [(int(g), float(v)) for n, g, v in rows if kernel in _short(n)]
+    return [(int(g), float(v)) for n, g, v in rows if any(k in _short(n) for k in kernel.split("|"))]
 
 
 def _excluded(i: int, grid: int, exclude) -> bool:
@@ -57,7 +58,8 @@ def _excluded(i: int, grid: int, exclude) -> bool:
 
 
 def traffic(fetch_db: str, write_db: str, kernel: str, copy_bytes: int, exclude=()):
-    """HBM bytes per dispatch of the kernels whose name contains ``kernel``.
+    """HBM bytes per dispatch of the kernels whose name contains ``kernel`` (or
+    one of several names joined by ``|``: a launch class of several kernels).
 
     The calibration dispatch is the largest ``__amd_rocclr_copyBuffer`` in each
     run (a device-to-device copy of ``copy_bytes`` that reads and writes

@@ -122,16 +122,32 @@ def ln_fused(spec: ModelSpec, precision: str) -> bool:
     return rp == 128 and spec.num_heads * spec.heads_dim == 256
 
 
-def psiformer_layer_bytes(spec: ModelSpec, n_atoms: int, fused_ln: bool = False):
+def layer_kernel(spec: ModelSpec, precision: str) -> str:
+    """The kernel of the Laplacian-mode dense layers: psi_chain_kernel where a
+    Psiformer layer's row-wise part is one launch (the library's
+    psi_chain_supported: the fused LayerNorm's shapes and one to four MLP layers
+    as wide as the model), gemm_kernel otherwise."""
+    if ln_fused(spec, precision) and len(spec.mlp_hidden) < 4:
+        if all(w == spec.num_heads * spec.heads_dim for w in spec.mlp_hidden):
+            return "psi_chain_kernel"
+    return "gemm_kernel"
+
+
+def psiformer_layer_bytes(spec: ModelSpec, n_atoms: int, fused_ln: bool = False, chain: bool = False):
     """Per-walker minimum HBM bytes of the Psiformer Laplacian-mode projections:
     Q/K/V (input, 3D output), output projection and last MLP layer (input,
     residual stream read, residual stream written), hidden MLP layers; with
     fused_ln also the LayerNorm outputs those GEMMs write (LN1 of every layer,
-    LN2 of every layer)."""
+    LN2 of every layer).  chain (one launch from the attention output to the next
+    layer's Q/K/V): attention output and residual stream read, residual stream
+    and 3D written, the last layer without the 3D; before the first layer the
+    input projection, its LayerNorm and Q/K/V as above."""
     N = spec.n_elec
     C = 3 * N + 2
     D = spec.num_heads * spec.heads_dim
     tot = 4.0 * N * (5 * (4 * n_atoms + 1) + C * D)
+    if chain:
+        return tot + 4.0 * N * C * D * (1 + 4 + 6 * (spec.num_layers - 1) + 3)
     for _ in range(spec.num_layers):
         tot += 4.0 * N * C * (D + 3 * D)
         tot += 4.0 * N * C * 3 * D
@@ -145,7 +161,8 @@ def psiformer_layer_bytes(spec: ModelSpec, n_atoms: int, fused_ln: bool = False)
 
 def layer_bytes(spec: ModelSpec, n_atoms: int, precision: str = "fp32"):
     return (ferminet_layer_bytes(spec, n_atoms) if spec.kind == "ferminet"
-            else psiformer_layer_bytes(spec, n_atoms, ln_fused(spec, precision)))
+            else psiformer_layer_bytes(spec, n_atoms, ln_fused(spec, precision),
+                                       layer_kernel(spec, precision) == "psi_chain_kernel"))
 
 
 MFMA_PER_PRODUCT = {"fp32": 1, "bf16": 1, "bf16x3": 3, "bf16x6": 6, "fp16x3": 3}

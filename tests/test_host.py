@@ -1,6 +1,7 @@
 """Host logic and the C-ABI library's exports (CPU only)."""
 
 import ctypes
+import dataclasses
 import re
 
 import numpy as np
@@ -194,3 +195,44 @@ def test_traffic_summary_calibration_and_exclusions(tmp_path):
     assert len(t["FETCH_SIZE"]["each"]) == 3  # the excluded dispatch is still listed
     t2 = traffic(str(tmp_path / "f.db"), str(tmp_path / "w.db"), "gemm_kernel<8, 1, 4, 4, true", copy, ("d0", "d2"))
     assert t2["FETCH_SIZE"]["bytes_per_dispatch"] == 3000.0 * 1024 * 2
+
+
+def test_layer_bytes_follow_the_kernels_that_run():
+    """Dense-layer bytes of the 42-electron Psiformer: six streams of the
+    (rows, 256) array per layer where one kernel runs from the attention output
+    to the next q, k, v, fourteen in a launch a stage."""
+    from jaqmc_amd import roofline as RF
+
+    _, spec, *_ = S.workload("ring42")
+    M, L = 12, spec.num_layers
+    stream = 4.0 * 42 * 128 * 256
+    inputs = 4.0 * 42 * 5 * (4 * M + 1)
+    assert RF.layer_kernel(spec, "fp16x3") == "psi_chain_kernel"
+    assert RF.layer_bytes(spec, M, "fp16x3") == inputs + stream * (1 + 1 + 4 + 6 * (L - 1) + 3)
+    for change, precision, streams in ((dict(mlp_hidden=[128]), "fp16x3", 1 + L * 13),
+                                       (dict(mlp_hidden=[256] * 4), "fp16x3", 1 + L * 20),
+                                       ({}, "fp32", 1 + L * 12)):
+        s = dataclasses.replace(spec, **change)
+        assert RF.layer_kernel(s, precision) == "gemm_kernel"
+        assert RF.layer_bytes(s, M, precision) == inputs + stream * streams, change
+    _, n2, *_ = S.workload("n2")
+    assert RF.layer_kernel(n2, "fp16x3") == "gemm_kernel"
+
+
+def test_measured_traffic_is_of_the_kernel_that_runs(tmp_path, monkeypatch):
+    """bench.py takes a committed traffic summary for the kernel that it names
+    only, and the committed ones are of the kernels that their workloads run."""
+    import bench
+    from jaqmc_amd import roofline as RF
+
+    for w in ("n2", "ring42", "h60"):
+        _, spec, *_ = S.workload(w)
+        bytes_, src = bench.measured_traffic(w, "fp16x3", RF.layer_kernel(spec, "fp16x3"))
+        assert bytes_ > 0 and w in src
+    (tmp_path / "profiles").mkdir()
+    (tmp_path / "profiles" / "gemm_layer_lap_ring42_fp16x3_traffic.txt").write_text(
+        "fp16x3\nKernel: dispatches whose name contains `gemm_kernel<8, 1, 4, 4, true`.\n"
+        "traffic_bytes_per_dispatch: 2.0e10\n")
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    assert bench.measured_traffic("ring42", "fp16x3", "psi_chain_kernel") == (None, None)
+    assert bench.measured_traffic("ring42", "fp16x3", "gemm_kernel")[0] == 2.0e10

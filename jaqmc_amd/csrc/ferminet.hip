@@ -359,9 +359,10 @@ __global__ void pair_layer_generic_kernel(long npairs, const float* __restrict__
 //   d/dx_i   <- mean_j (d/dx_b rows of pair (j, i))
 //   d/dx_j   <- (d/dx_a rows of pair (j, i)) / n_s,   j in s
 // From the column of one (walker, electron) in LDS, feature f of row RP2 j + t at
-// col[at(RP2 j + t, f)] (part: LDS for the sums), the workgroup of NTH threads writes the unit's whole block
-// X[unit][0:Rp][col0:ldx) row by row; columns past nch*f2 are zero-filled (GEMM
-// K padding).  Called with the column complete (behind a barrier).
+// col[at(RP2 j + t, f)] (part: LDS for the sums), the workgroup of NTH threads
+// writes the unit's whole block X[unit][0:Rp][col0:ldx) row by row; columns past
+// nch*f2 are zero-filled (GEMM K padding).  Called with the column complete
+// (behind a barrier).
 struct ColRows {
   int f2;
   __device__ int operator()(int row, int f) const { return row * f2 + f; }

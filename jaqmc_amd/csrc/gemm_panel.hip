@@ -268,8 +268,9 @@ int launch_panel(const GemmArgs& a, hipStream_t s) {
 }  // namespace
 
 // Takes a projection (no activation, broadcast term or residual) of 256 k onto
-// more columns than one block, with 16-byte rows and stores, where the panel of a
-// tile fits LDS.  Both sides measured: the panel is split once for all column
+// more columns than one block, with 16-byte rows and stores, of 48-, 96- and
+// 128-row units (the panel of 192 rows does not fit LDS; 16-, 32- and 64-row units
+// stay with gemm_kernel, not measured here).  Both sides measured: the panel is split once for all column
 // blocks, which wins from the second on (1.23M rows of 128-row units: 1239 -> 1019 us
 // at 320 columns) and loses with only one (733 -> 854 us at 256, 657 -> 791 at 224);
 // and the last round of tiles idles the fewer CUs the more tiles each has (768

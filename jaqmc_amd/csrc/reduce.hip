@@ -24,11 +24,12 @@
 //     us (70 launches of two kernels per 8-bit pass and statistic ran before,
 //     the digit picked by a single thread); on 16384: 555 -> 57 us.
 //   larger: a histogram pass per 11-bit digit over up to 256 workgroups; the
-//     last workgroup to finish a pass picks the digits (17 launches at most).
+//     last workgroup to finish a pass picks the digits (mad: two selections of a range
+//     and six digit passes, 17 launches with the set-up, the means and the weights).
 //     200000 values: 1906 -> 401 us, 2^20: 2819 -> 524 us.
 // The line between them is the register budget of one workgroup of 1024
 // threads: 16 values each (the second form takes 223 us just past it).
-
+//
 // The scratch buffer (histograms + selection state, used by the second form)
 // is a caller workspace of jq_loss_clip_workspace_bytes() bytes, or, for
 // jq_loss_clip_noalloc, a static device array of the same size.

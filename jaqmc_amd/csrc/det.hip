@@ -305,7 +305,10 @@ __device__ __forceinline__ void fwd_lu_steps(double (&m)[NP], int N, int lane, F
       const double pv = readlane_f64(x, piv);
       st.logdet.mul(pv);
       st.neg ^= pv < 0.0 ? 1 : 0;
-      const double l = (open && lane != piv) ? x / pivot_divisor(pv) : 0.0;
+      // the divisor of pivot_divisor, formed in scalar registers (2 % of the
+      // kernel; with vector compares, on x or on the pivot, 8 %)
+      const double dv = (__double_as_longlong(pv) << 1) == 0 ? INFINITY : pv;
+      const double l = (open && lane != piv) ? x / dv : 0.0;
       // pivot-row entries read four at a time ahead of their multiply-adds, so
       // the scalar reads do not wait on each other
 #pragma unroll

@@ -14,9 +14,9 @@
 // product is kept as a mantissa in [0.5, 1) and a binary exponent (both
 // factors split with frexp, so it neither overflows nor underflows), and one
 // log is taken at the end.  A zero factor gives -inf, a NaN or inf factor
-// propagates, as the sum of logs would.  The value-only eliminations go on past
-// a zero pivot (pivot_divisor), so a singular matrix gives -inf there; the ones
-// that form an inverse divide by it, and give NaN.
+// propagates, as the sum of logs would.  The value-only eliminations (fwd_col_steps,
+// fwd_lu_steps) go on past a zero pivot, so a singular matrix gives -inf there; the
+// ones that form an inverse divide by it, and give NaN.
 struct LogAbsProduct {
   double m = 1.0;
   int e = 0;
@@ -29,7 +29,7 @@ struct LogAbsProduct {
   __device__ double log_abs() const { return log(m) + (double)e * 0.69314718055994530942; }
 };
 
-// What a value-only elimination divides by.  Beside a zero pivot its column holds
+// What the value-only eliminations divide by.  Beside a zero pivot its column holds
 // nothing to eliminate: dividing by infinity gives zero, and the step leaves the
 // other columns as they are (0 / 0 would turn them, and the identity that pads
 // the matrix, into NaN); non-finite entries become NaN and stay in the result.

@@ -270,11 +270,11 @@ int launch_panel(const GemmArgs& a, hipStream_t s) {
 // Takes a projection (no activation, broadcast term or residual) of 256 k onto
 // more columns than one block, with 16-byte rows and stores, of 48-, 96- and
 // 128-row units (the panel of 192 rows does not fit LDS; 16-, 32- and 64-row units
-// stay with gemm_kernel, not measured here).  Both sides measured: the panel is split once for all column
-// blocks, which wins from the second on (1.23M rows of 128-row units: 1239 -> 1019 us
-// at 320 columns) and loses with only one (733 -> 854 us at 256, 657 -> 791 at 224);
-// and the last round of tiles idles the fewer CUs the more tiles each has (768
-// columns: 264 -> 225 us at 4.5 tiles per CU).
+// stay with gemm_kernel, not measured here).  Both sides measured: the panel is
+// split once for all column blocks, which wins from the second on (1.23M rows of
+// 128-row units: 1239 -> 1019 us at 320 columns) and loses with only one (733 -> 854
+// us at 256, 657 -> 791 at 224); and the last round of tiles idles the fewer CUs the
+// more tiles each has (768 columns: 264 -> 225 us at 4.5 tiles per CU).
 bool gemm_panel_ok(const GemmArgs& a) {
   const int bm = a.R == 128 ? 128 : (a.R == 48 || a.R == 96 ? 96 : 0);
   if (bm == 0 || a.K != kK || a.ncols <= 256 || a.act != ACT_NONE || a.G || a.Res || a.Yln || a.rgrp > 0 || a.linear_tiles)

@@ -305,8 +305,9 @@ __device__ __forceinline__ void fwd_lu_steps(double (&m)[NP], int N, int lane, F
       const double pv = readlane_f64(x, piv);
       st.logdet.mul(pv);
       st.neg ^= pv < 0.0 ? 1 : 0;
-      // the divisor of pivot_divisor, formed in scalar registers (2 % of the
-      // kernel; with vector compares, on x or on the pivot, 8 %)
+      // past a zero pivot as in fwd_col_steps: dividing by infinity gives zeros, and
+      // NaN for what is not finite; chosen in scalar registers (2 % of the kernel,
+      // with vector compares, on x or on the pivot, 8 %)
       const double dv = (__double_as_longlong(pv) << 1) == 0 ? INFINITY : pv;
       const double l = (open && lane != piv) ? x / dv : 0.0;
       // pivot-row entries read four at a time ahead of their multiply-adds, so

@@ -29,12 +29,6 @@ struct LogAbsProduct {
   __device__ double log_abs() const { return log(m) + (double)e * 0.69314718055994530942; }
 };
 
-// What the value-only eliminations divide by.  Beside a zero pivot its column holds
-// nothing to eliminate: dividing by infinity gives zero, and the step leaves the
-// other columns as they are (0 / 0 would turn them, and the identity that pads
-// the matrix, into NaN); non-finite entries become NaN and stay in the result.
-__device__ inline double pivot_divisor(double pv) { return pv == 0.0 ? INFINITY : pv; }
-
 // Sign of the permutation perm[0 .. n-1] (n <= 64), from its cycles.
 __device__ inline int perm_sign(const int* perm, int n) {
   unsigned long long seen = 0ull;
@@ -282,7 +276,10 @@ __device__ __forceinline__ void fwd_col_steps(double (&m)[NP], LogAbsProduct& lo
       m[i] = sel ? mp : m[i];
       c[i] = sel ? cp : c[i];
     }
-    r /= pivot_divisor(pv);
+    // A zero pivot has nothing beside it to eliminate, and the step leaves the other
+    // columns as they are (0 / 0 would turn them, and the identity that pads the
+    // matrix, into NaN); a non-finite r stays in the result as NaN.
+    r = pv == 0.0 ? r * 0.0 : r / pv;
 #pragma unroll
     for (int i = P + 1; i < NP; ++i) m[i] = fma(-c[i], r, m[i]);
     fwd_col_steps<P + 1, NP>(m, logdet, neg);

@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256) void det_fwd_reg_kernel(FermiDims d, const flo
 // Forward mode, N <= 16: log|det| and sign, four determinants per wavefront,
 // one in each 16-lane DPP row: lane j holds column j (NP >= N rows in
 // registers, padded with the identity; fwd_col_steps).  Bound by VALU issue:
-// 65536 matrices of 14 in 92 us, where a wavefront per matrix, exchanging pivot
+// 65536 matrices of 14 in 82 us, where a wavefront per matrix, exchanging pivot
 // rows and columns through LDS, took 228 (1024 of 3: 4.2 us, 18.5).
 // ---------------------------------------------------------------------------
 template <int NP>
